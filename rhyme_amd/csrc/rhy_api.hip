@@ -141,28 +141,6 @@ int check_params(const rhy_params_t* p, int nd) {
   return RHY_OK;
 }
 
-Consts make_consts(const rhy_params_t* p) {
-  Consts k{};
-  const double g = p->gamma;
-  k.g = g;
-  k.gm1 = g - 1.0;
-  k.gp1 = g + 1.0;
-  k.gm1_gp1 = k.gm1 / k.gp1;
-  k.gm1_2g = k.gm1 / (2.0 * g);
-  k.gp1_2g = k.gp1 / (2.0 * g);
-  k.g_inv = 1.0 / g;
-  k.kb_amu = p->kb_amu;
-  k.omega = p->omega;
-  k.tol = p->tolerance;
-  k.w_rho = p->w_vacuum_rho;
-  k.w_p = p->w_vacuum_p;
-  k.e_rho = std::nextafter(p->w_vacuum_rho, INFINITY);
-  k.limiter = p->limiter;
-  k.n_iter = p->n_iteration;
-  k.defer_every = defer_every_setting();
-  return k;
-}
-
 BcTypes make_bc(const rhy_params_t* p) {
   BcTypes b{};
   for (int f = 0; f < 6; ++f) b.t[f] = p->bc_types[f];
@@ -525,7 +503,7 @@ int launch_acc_step(rhy_box* b, const Consts& k, const double* dx,
 template <int ND>
 int run_steps(rhy_box* b, const rhy_params_t* p, const double* dx, int32_t nsteps) {
   b->coarse_walked = false;
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   const BcTypes bc = make_bc(p);
   int rc;
   if ((rc = ensure_dt_log(b, nsteps > 0 ? nsteps : 1))) return rc;
@@ -1144,7 +1122,7 @@ int rhy_cfl_time_step(rhy_box_t* b, const rhy_params_t* p, const double dx[3], d
   if ((rc = check_box(b))) return rc;
   if ((rc = check_params(p, b->ndim))) return rc;
   if (!dx || !dt) return fail(RHY_ERR_ARG, "dx/dt is NULL");
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   if (b->ndim == 1) rc = launch_cfl<1>(b, k);
   else if (b->ndim == 2) rc = launch_cfl<2>(b, k);
   else rc = launch_cfl<3>(b, k);
@@ -1171,7 +1149,7 @@ int mh_solve_enqueue(rhy_box* b, const rhy_params_t* p, const double* dx, double
   if (!dx) return fail(RHY_ERR_ARG, "dx is NULL");
   if (p->solver_type != RHY_CPU_INTENSIVE && p->solver_type != RHY_MEMORY_INTENSIVE)
     return fail(RHY_ERR_SOLVER, "Unknown solver type");
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(64), 0, b->stream, b->dt, dt);
   const BcTypes bc = make_bc(p);
   if (b->ndim == 1) {
@@ -1212,7 +1190,7 @@ int rhy_amr_coarse_step(rhy_box_t* b, const rhy_params_t* p, const double dx[3],
   if (!dx) return fail(RHY_ERR_ARG, "dx is NULL");
   if (p->solver_type != RHY_CPU_INTENSIVE && p->solver_type != RHY_MEMORY_INTENSIVE)
     return fail(RHY_ERR_SOLVER, "Unknown solver type");
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   if ((rc = b->ndim == 2 ? launch_bc<2>(b, p, -1) : launch_bc<3>(b, p, -1))) return rc;
   hipLaunchKernelGGL(set_step_kernel, dim3(1), dim3(64), 0, b->stream, b->dt, step_consts(b),
                      dt, dx[0], b->ndim > 1 ? dx[1] : 1.0, b->ndim > 2 ? dx[2] : 1.0,
@@ -1416,7 +1394,7 @@ static int riemann_solve_common(const rhy_params_t* p, int64_t n, const double* 
   if (dx && ((rc = to_dev(ddx, dx, sizeof(double) * (size_t)n)) ||
              (rc = to_dev(ddt, dt, sizeof(double) * (size_t)n))))
     return rc;
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   const unsigned g = grid_for(n);
   const double* L = (const double*)dl.p;
   const double* R = (const double*)dr.p;
@@ -1460,7 +1438,7 @@ int rhy_riemann_star_batch(const rhy_params_t* p, int64_t n, rhy_rp_solution_t* 
   DevBuf ds, da;
   if ((rc = to_dev(ds, sol, sb)) || (rc = to_dev(da, axis, sizeof(int32_t) * (size_t)n)))
     return rc;
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   const unsigned g = grid_for(n);
   rhy_rp_solution_t* S = (rhy_rp_solution_t*)ds.p;
   const int32_t* A = (const int32_t*)da.p;
@@ -1497,7 +1475,7 @@ static int rp_sample_common(const rhy_params_t* p, int64_t n, const rhy_rp_solut
   } else if ((rc = to_dev(d1, dx, nb)) || (rc = to_dev(d2, dt, nb))) {
     return rc;
   }
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   const unsigned g = grid_for(n);
   const rhy_rp_solution_t* S = (const rhy_rp_solution_t*)ds.p;
   const int32_t* A = (const int32_t*)da.p;
@@ -1553,7 +1531,7 @@ static int irs_common(const rhy_params_t* p, int64_t n, const double* l, const d
              (rc = to_dev(drf, nullptr, nb))) {
     return rc;
   }
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   hipLaunchKernelGGL(irs_batch_kernel, dim3(grid_for(n)), dim3(kThreads), 0, 0, k, n,
                      (const double*)dl.p, (const double*)dr.p, (double*)dp.p, (double*)dlf.p,
                      (double*)drf.p, (double*)dg.p);
@@ -1610,7 +1588,7 @@ int rhy_limiter_batch(const rhy_params_t* p, int64_t n, const double* ul, const 
   if ((rc = to_dev(a, ul, vb)) || (rc = to_dev(b, u, vb)) || (rc = to_dev(c, ur, vb)) ||
       (rc = to_dev(d, nullptr, vb)))
     return rc;
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   const unsigned g = grid_for(n);
   if (p->ndim == 1)
     hipLaunchKernelGGL(limiter_batch_kernel<1>, dim3(g), dim3(kThreads), 0, 0, k, n,
@@ -1639,7 +1617,7 @@ int rhy_half_step_batch(const rhy_params_t* p, int64_t n, const double* u, const
       (rc = to_dev(da, axis, sizeof(int32_t) * (size_t)n)) || (rc = to_dev(dl, nullptr, vb)) ||
       (rc = to_dev(dr, nullptr, vb)))
     return rc;
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   const unsigned g = grid_for(n);
   if (p->ndim == 1)
     hipLaunchKernelGGL(half_step_batch_kernel<1>, dim3(g), dim3(kThreads), 0, 0, k, n,
@@ -1671,7 +1649,7 @@ int rhy_flux_batch(const rhy_params_t* p, int64_t n, const double* u, const int3
   if ((rc = to_dev(du, u, vb)) || (rc = to_dev(da, axis, sizeof(int32_t) * (size_t)n)) ||
       (rc = to_dev(df, nullptr, vb)))
     return rc;
-  const Consts k = make_consts(p);
+  const Consts k = consts_of(p);
   const unsigned g = grid_for(n);
   if (p->ndim == 1)
     hipLaunchKernelGGL(flux_batch_kernel<1>, dim3(g), dim3(kThreads), 0, 0, k, n,

@@ -690,28 +690,6 @@ struct rhy_batch {
 
 namespace {
 
-Consts consts_of(const rhy_params_t* p) {
-  Consts k{};
-  const double g = p->gamma;
-  k.g = g;
-  k.gm1 = g - 1.0;
-  k.gp1 = g + 1.0;
-  k.gm1_gp1 = k.gm1 / k.gp1;
-  k.gm1_2g = k.gm1 / (2.0 * g);
-  k.gp1_2g = k.gp1 / (2.0 * g);
-  k.g_inv = 1.0 / g;
-  k.kb_amu = p->kb_amu;
-  k.omega = p->omega;
-  k.tol = p->tolerance;
-  k.w_rho = p->w_vacuum_rho;
-  k.w_p = p->w_vacuum_p;
-  k.e_rho = std::nextafter(p->w_vacuum_rho, INFINITY);
-  k.limiter = p->limiter;
-  k.n_iter = p->n_iteration;
-  k.defer_every = defer_every_setting();
-  return k;
-}
-
 // Geometry and arena footprint (elements) of a box.
 int box_geom(int ndim, const int32_t* dims, Geom& G) {
   int64_t st = 1;

@@ -113,6 +113,38 @@ struct BcTypes {
 int32_t defer_every_setting();
 int64_t defer_cap_setting();
 
+// The kernels' constants from the caller's parameters.
+inline Consts consts_of(const rhy_params_t* p) {
+  Consts k{};
+  const double g = p->gamma;
+  k.g = g;
+  k.gm1 = g - 1.0;
+  k.gp1 = g + 1.0;
+  k.gm1_gp1 = k.gm1 / k.gp1;
+  k.gm1_2g = k.gm1 / (2.0 * g);
+  k.gp1_2g = k.gp1 / (2.0 * g);
+  k.g_inv = 1.0 / g;
+  k.c2g = 2.0 / k.gm1;
+  k.hgm1 = .5 * k.gm1;
+  k.g_gm1 = g / k.gm1;
+  k.two_gp1 = 2.0 / k.gp1;
+  k.qgp1 = .25 * k.gp1;
+  k.inv_z = 1.0 / k.gm1_2g;
+  k.nroot = 0;
+  for (int n : {5, 7, 8})
+    if (std::fabs(k.inv_z - n) < 1e-13 * n) k.nroot = n;
+  k.kb_amu = p->kb_amu;
+  k.omega = p->omega;
+  k.tol = p->tolerance;
+  k.w_rho = p->w_vacuum_rho;
+  k.w_p = p->w_vacuum_p;
+  k.e_rho = std::nextafter(p->w_vacuum_rho, INFINITY);
+  k.limiter = p->limiter;
+  k.n_iter = p->n_iteration;
+  k.defer_every = defer_every_setting();
+  return k;
+}
+
 // A box's device state as the hierarchy kernels see it (box_view waits for
 // the box's stream).
 struct BoxView {
@@ -798,8 +830,10 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void acc_walk_kernel(
 // One face's flux from scratch: the half steps of its two cells (the
 // stencil of four cells along A) and the Riemann solve with policy PW, the
 // computation the flux walks make for it.  of: offset of the low cell.
+// (Out of line: its callers are the fixup and reflux kernels, which hold
+// several of these calls and run on few faces.)
 template <int ND, int A, typename R, class PW>
-__device__ __forceinline__ void face_flux(const Consts& k, const Geom& G,
+__device__ __noinline__ void face_flux(const Consts& k, const Geom& G,
                                           const R* __restrict__ cells, double dt, double dx,
                                           int64_t of, R* Fr) {
   constexpr int NV = ND + 2;

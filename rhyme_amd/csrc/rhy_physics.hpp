@@ -30,6 +30,14 @@ struct Consts {
   double tol;            // irs%tolerance
   double w_rho, w_p;     // rp%w_vacuum(rho), rp%w_vacuum(p)
   double e_rho;          // nearest(w_rho, +1), computed on the host
+  // products the walks' Riemann solve needs, formed on the host
+  double c2g;            // 2 / (gamma - 1)
+  double hgm1;           // (gamma - 1) / 2
+  double g_gm1;          // gamma / (gamma - 1)
+  double two_gp1;        // 2 / (gamma + 1)
+  double qgp1;           // (gamma + 1) / 4
+  double inv_z;          // 2 gamma / (gamma - 1)
+  int32_t nroot;         // inv_z where it is 5, 7 or 8 (gamma 5/3, 7/5, 4/3), else 0
   int32_t limiter;       // slid
   int32_t n_iter;        // irs%n_iteration
   int32_t defer_every;   // > 0: test hook, defer every such face (by offset)
@@ -237,22 +245,137 @@ __device__ __forceinline__ R limit_one(int type, R w, R ul, R u, R ur) {
   }
 }
 
+// ----------------------------------- FP64 arithmetic of the walks ----
+//
+// The unit-level kernels evaluate the reference's expressions operation for
+// operation (above).  The FP64 walks, which form a half step and a Riemann
+// solve per cell and face, evaluate the same formulas with the terms
+// arranged so that one reciprocal serves all quotients of a state:
+//   v = m / rho, p = (E - m.v / 2) (gamma - 1), F = (m_A, m v_A + p, v_A (E + p)),
+// every reciprocal and root to an ulp.  A gas at rest with uniform E then has
+// bitwise uniform p whatever its density, so that all its faces are exact
+// contacts (below): with the reference's rho (E / rho - kin) one wave in
+// seven held a face that missed by an ulp and iterated.  (The mixed form has
+// formed p this way from the start, and keeps the reference's forms
+// otherwise: its FP32 roundings are part of its results.)
+
+// 1 / b to within an ulp: the hardware reciprocal (2^-22) and one
+// third-order step.
+__device__ __forceinline__ double recip(double b) {
+  const double r = __builtin_amdgcn_rcp(b);
+  const double e = __builtin_fma(-b, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+
+// 1 / sqrt(x), x > 0 normal: hardware estimate and one third-order step.
+__device__ __forceinline__ double rsqrt_of(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * y, y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+}
+// sqrt(x), x > 0 normal, with a residual step on x / sqrt(x).
+__device__ __forceinline__ double sqrt_of(double x) {
+  const double y = rsqrt_of(x);
+  const double s = x * y;
+  return __builtin_fma(0.5 * __builtin_fma(-s, s, x), y, s);
+}
+
+// |x| where the reciprocals, products and roots of the walks neither
+// overflow nor lose bits to denormals; other states take the reference's
+// forms.
+__device__ __forceinline__ bool plain_range(double x) {
+  return fabs(x) >= 0x1p-200 && fabs(x) <= 0x1p200;
+}
+
+// flux_of with the shared reciprocal of rho.
+template <int ND, int A>
+__device__ __forceinline__ void state_flux(const Consts& k, const double* u, double* f) {
+  if (plain_range(u[0])) {
+    const double ir = recip(u[0]);
+    double ke2 = 0.0, va = 0.0;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const double v = u[1 + d] * ir;
+      ke2 = d == 0 ? u[1] * v : ke2 + u[1 + d] * v;
+      if (d == A) va = v;
+    }
+    const double p = (u[ND + 1] - .5 * ke2) * k.gm1;
+    f[0] = u[1 + A];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) f[1 + d] = u[1 + d] * va;
+    f[1 + A] = f[1 + A] + p;
+    f[ND + 1] = va * (u[ND + 1] + p);
+  } else if (fabs(u[0]) < kTiny) {
+#pragma unroll
+    for (int c = 0; c < ND + 2; ++c) f[c] = 0.0;
+  } else {
+    flux_of<ND, A, double>(k, u, f);
+  }
+}
+
+// The limited slope of limit_one for omega = 0, where xi_R = 2 / (1 + r) and
+// d = (dL + dR) / 2 make xi_R d = dR, so that few branches divide:
+//   r = dL / dR <= 0 (or no number)   0
+//   |dL| > |dR| (r > 1)               dR: every limiter takes its xi_R d
+//   otherwise                         van Leer dL (2 r / (1 + r) d),
+//                                     minmod r d,
+//                                     van Albada r (1 + r) / (1 + r^2) d,
+//                                     superbee d for r > 1/2, else 2 r d
+template <int LIM>
+__device__ __forceinline__ double slope_of(int type, double dL, double dR) {
+  const int t = LIM ? LIM : type;
+  const double a = fabs(dL), b = fabs(dR);
+  if (!((dL > 0.0 && dR > 0.0) || (dL < 0.0 && dR < 0.0))) return 0.0;
+  if (b < kTiny) return 0.0;
+  if (t == 1) return a > b ? dR : dL;
+  if (a > b) return dR;
+  const double d = .5 * (dL + dR);
+  switch (t) {
+    case 2:
+      return dL / dR * d;
+    case 3: {
+      const double r = dL / dR;
+      return r * (1.0 + r) * recip(1.0 + r * r) * d;
+    }
+    case 4:
+      if (a > .5 * b) return d;
+      return 2.0 * (dL / dR) * d;
+    default:
+      return 0.0;
+  }
+}
+
 // rhyme_muscl_hancock_half_step_extrapolation.f90:15-21: slope from the
 // three cells um, u, up along axis A, then the half-step states l and r.
 template <int ND, int A, int LIM = 0, typename R = double>
 __device__ __forceinline__ void half_step(const Consts& k, const R* um, const R* u, const R* up,
                                           R hdtdx, R* l, R* r) {
   constexpr int NV = ND + 2;
+  constexpr bool kF64 = sizeof(R) == sizeof(double);
   R fl[NV], fr[NV];
   const R w = R(k.omega);
+  if (kF64 && w == R(0)) {
 #pragma unroll
-  for (int c = 0; c < NV; ++c) {
-    R delta = limit_one<LIM, R>(k.limiter, w, um[c], u[c], up[c]);
-    l[c] = u[c] - R(.5) * delta;
-    r[c] = u[c] + R(.5) * delta;
+    for (int c = 0; c < NV; ++c) {
+      const R h = R(.5) * (R)slope_of<LIM>(k.limiter, u[c] - um[c], up[c] - u[c]);
+      l[c] = u[c] - h;
+      r[c] = u[c] + h;
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+      const R delta = limit_one<LIM, R>(k.limiter, w, um[c], u[c], up[c]);
+      l[c] = u[c] - R(.5) * delta;
+      r[c] = u[c] + R(.5) * delta;
+    }
   }
-  flux<ND, A, R>(k, l, fl);
-  flux<ND, A, R>(k, r, fr);
+  if constexpr (kF64) {
+    state_flux<ND, A>(k, l, fl);
+    state_flux<ND, A>(k, r, fr);
+  } else {
+    flux<ND, A, R>(k, l, fl);
+    flux<ND, A, R>(k, r, fr);
+  }
 #pragma unroll
   for (int c = 0; c < NV; ++c) {
     R df = fl[c] - fr[c];
@@ -272,6 +395,7 @@ __device__ __forceinline__ void half_step(const Consts& k, const R* um, const R*
 // IEEE division and sqrt.
 struct PowLib {
   static constexpr bool kFast = false;
+  static constexpr bool kStar = false;  // star_sample (below) for the walks' faces
   static constexpr bool kDefer = false;
   __device__ __forceinline__ static double dv(double a, double b) { return a / b; }
   __device__ __forceinline__ static double sq(double x) { return sqrt(x); }
@@ -291,6 +415,7 @@ struct PowLib {
 // results as two pw calls.
 struct PowFast {
   static constexpr bool kFast = false;
+  static constexpr bool kStar = true;
   static constexpr bool kDefer = false;
   __device__ __forceinline__ static double dv(double a, double b) { return a / b; }
   __device__ __forceinline__ static double sq(double x) { return sqrt(x); }
@@ -382,6 +507,7 @@ struct PowFast {
 // take the IEEE operation.
 struct MixedMath : PowFast {
   static constexpr bool kFast = true;
+  static constexpr bool kStar = false;
   __device__ __forceinline__ static double dv(double a, double b) {
     const double ab = fabs(b);
     if (!(ab > 0x1p-1000 && ab < 0x1p+1000)) return a / b;
@@ -707,9 +833,9 @@ __device__ __forceinline__ void side_prims(const Consts& k, const RI* s, double*
 // branch of the reference ends in conv_prim_vars_to_cons of the state chosen
 // here.
 template <int ND, int A, class PW, typename RI>
-__device__ __forceinline__ void riemann_sample(const Consts& k, const RI* l, const RI* r,
-                                               double dxdt, double& srho, double* sv,
-                                               double& sp) {
+__device__ __forceinline__ void riemann_sample_ref(const Consts& k, const RI* l, const RI* r,
+                                                   double dxdt, double& srho, double* sv,
+                                                   double& sp) {
   const double l_rho = dmax((double)l[0], k.w_rho);
   const double r_rho = dmax((double)r[0], k.w_rho);
   const double e_rho = k.e_rho;
@@ -822,29 +948,291 @@ __device__ __forceinline__ void riemann_sample(const Consts& k, const RI* l, con
   }
 }
 
-// The conserved state sampled at x/t = dxdt (FP64 unit-level solve).
+// ------------------------------------------ star state of the walks ----
+//
+// irs_exec, rp_star and rp_sampling for two ordinary states (no vacuum,
+// every quantity in plain_range): the reference's guess, Newton iterates,
+// stopping rule and sampling, in terms arranged for few divisions and powers:
+//   * shock side: f = (p - p_K) / sqrt(rho_K ((g+1) p + (g-1) p_K) / 2), one
+//     reciprocal root (sqrt(A/(p+B)) with A, B written out), whose square
+//     also gives f';
+//   * rarefaction side: y = (p/p_K)^z, z = (g-1)/2g, f = 2 c_K/(g-1) (y - 1)
+//     and f' = y p_K / (rho_K c_K p): one power instead of two;
+//   * 1/z = 2g/(g-1) is 5, 7 or 8 for the monatomic, diatomic and polyatomic
+//     gas, so y is a root that a single-precision estimate and one Halley
+//     step give to an ulp (root_z), and x^(1/z) and the fan's powers are
+//     products; any other gamma takes exp(y log x);
+//   * the two-rarefaction guess needs one of its two equal terms
+//     p_K x_K^(1/z), and quotients over one divisor share its reciprocal.
+//
+// Returns false where the reference leaves this path (vacuum generated, a
+// Newton iterate below zero, a state out of range): the caller then takes
+// riemann_sample_ref, or defers the face to the fixup kernel, which does.
+
+// b^5, b^7 or b^8
+__device__ __forceinline__ double pow_n(int n, double b) {
+  const double b2 = b * b, b4 = b2 * b2;
+  return b4 * (n == 5 ? b : n == 7 ? b2 * b : b4);
+}
+
+// x^z, z = (gamma-1)/2gamma, x > 0.  n = 1/z: y0 = x^(1/n) in FP32 (relative
+// error 2^-22), then Halley's y = y0 + 2 y0 (x - y0^n) / ((n+1) y0^n + (n-1) x),
+// whose error is of order y0's cubed.
+__device__ __forceinline__ double root_z(const Consts& k, double x) {
+  if (k.nroot > 0 && x > 0x1p-100 && x < 0x1p100) {
+    const float e = __builtin_amdgcn_logf((float)x) * (float)k.gm1_2g;
+    const double y = (double)__builtin_amdgcn_exp2f(e);
+    const double yn = pow_n(k.nroot, y);
+    const double n = (double)k.nroot;
+    const double den = __builtin_fma(n + 1.0, yn, (n - 1.0) * x);
+    double q = __builtin_amdgcn_rcp(den);
+    q = __builtin_fma(__builtin_fma(-den, q, 1.0), q, q);
+    return __builtin_fma((y + y) * (x - yn), q, y);
+  }
+  return PowFast::ex(k.gm1_2g * PowFast::ln(x));
+}
+
+// x^(1/z), x > 0
+__device__ __forceinline__ double pow_inv_z(const Consts& k, double x) {
+  return k.nroot > 0 ? pow_n(k.nroot, x) : PowFast::ex(k.inv_z * PowFast::ln(x));
+}
+
+// f_K(p) and its derivative; prc = p_K / (rho_K c_K), ipk = 1 / p_K, ip = 1 / p
+__device__ __forceinline__ void wave_terms(const Consts& k, double p, double ip, double rho,
+                                           double pk, double ipk, double c, double prc, double& f,
+                                           double& fp) {
+  if (p > pk) {
+    const double y = rsqrt_of(0.5 * rho * (k.gp1 * p + k.gm1 * pk));
+    const double d = p - pk;
+    f = d * y;
+    fp = y * (1.0 - k.qgp1 * rho * d * (y * y));
+  } else {
+    const double y = root_z(k, p * ipk);
+    f = k.c2g * c * (y - 1.0);
+    fp = y * prc * ip;
+  }
+}
+
+template <int ND, int A>
+__device__ __forceinline__ bool star_sample(const Consts& k, double lr, const double* lv, double lp,
+                                            double lc, double rr, const double* rv, double rp,
+                                            double rc, double& srho, double* sv, double& sp) {
+  const double du = rv[A] - lv[A];
+  if (k.c2g * (lc + rc) < du) return false;  // vacuum generated (:83-98)
+  const double ipp = recip(lp * rp);
+  const double ilp = rp * ipp, irp = lp * ipp;
+  double p, lf = 0.0, rf = 0.0;
+  // guess 1 (rhyme_irs_guess_p_star.f90:14-39)
+  const double ppv =
+      dmax(0.5 * (lp + rp) - 0.5 * du * (0.25 * (lr + rr) * (lc + rc)), 0.0);
+  const double p_min = dmin(lp, rp), p_max = dmax(lp, rp);
+  if (p_max <= 2.0 * p_min && p_min < ppv && ppv < p_max) {
+    p = ppv;
+  } else if (ppv < p_min) {
+    const double pq = root_z(k, lp * irp);
+    const double um = (pq * lv[A] * rc + rv[A] * lc + k.c2g * (pq - 1.0) * (lc * rc)) *
+                      recip(pq * rc + lc);
+    const double x = 1.0 + k.hgm1 * (lv[A] - um) * recip(lc);
+    if (!(x > 0x1p-30)) return false;
+    p = lp * pow_inv_z(k, x);
+  } else {
+    const double gl = rsqrt_of(0.5 * lr * (k.gm1 * lp + k.gp1 * ppv));
+    const double gr = rsqrt_of(0.5 * rr * (k.gm1 * rp + k.gp1 * ppv));
+    p = (gl * lp + gr * rp - du) * recip(gl + gr);
+  }
+  if (!plain_range(p) || !(p > 0.0)) return false;
+  // p_K / (rho_K c_K) of both sides
+  const double lrc = lr * lc, rrc = rr * rc;
+  const double irc = recip(lrc * rrc);
+  const double lprc = lp * rrc * irc, rprc = rp * lrc * irc;
+  // rhyme_irs_exec.f90:25-39
+  double prev = p;
+  for (int i = 1; i <= k.n_iter; ++i) {
+    double lfp, rfp;
+    const double ip = recip(p);
+    wave_terms(k, p, ip, lr, lp, ilp, lc, lprc, lf, lfp);
+    wave_terms(k, p, ip, rr, rp, irp, rc, rprc, rf, rfp);
+    p = prev - (lf + rf + du) * recip(lfp + rfp);
+    if (!(p > 0x1p-300)) return false;
+    if (2.0 * fabs(p - prev) < k.tol * (p + prev)) break;
+    prev = p;
+  }
+  if (!plain_range(p)) return false;
+  if (p < k.w_p) p = k.w_p;
+  const double us = 0.5 * ((rv[A] + lv[A]) + (rf - lf));
+  // sampling (rhyme_riemann_problem_sampling.f90:13-47) on the side K of the
+  // point x/t = 0 with the signed sound speed sc = +c_R or -c_L, as riemann_sample_ref
+  const bool right = 0.0 > us;
+  const double kp = right ? rp : lp, kc = right ? rc : lc;
+  const double sc = right ? rc : -lc;
+  const double x = p * (right ? irp : ilp);
+  srho = right ? rr : lr;
+  sp = kp;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) sv[d] = right ? rv[d] : lv[d];
+  if (p > kp) {
+    const double speed = sv[A] + sc * sqrt_of(k.gp1_2g * x + k.gm1_2g);
+    if (right ? 0.0 < speed : 0.0 > speed) {
+      srho = srho * (k.gm1_gp1 + x) * recip(k.gm1_gp1 * x + 1.0);
+      sv[A] = us;
+      sp = p;
+    }
+  } else {
+    const double y = root_z(k, x);
+    const double fan_cs = kc * y;
+    const double head = sv[A] + sc;
+    const double tail = us + (right ? fan_cs : -fan_cs);
+    if (right ? 0.0 < tail : 0.0 > tail) {
+      // x^(1/gamma) = x / x^(2 z)
+      srho = srho * (x * recip(y * y));
+      sv[A] = us;
+      sp = p;
+    } else if (right ? 0.0 < head : 0.0 > head) {  // w_kfan_prim
+      const double b = k.two_gp1 - k.gm1_gp1 * sv[A] * recip(sc);
+      if (!(b > 0x1p-30)) return false;
+      if (k.nroot > 0) {  // 2 / (gamma-1) = 1/z - 2
+        const double bn = pow_n(k.nroot, b);
+        srho = srho * (bn * recip(b * b));
+        sp = kp * bn;
+      } else {
+        const double l = PowFast::ln(b);
+        srho = srho * PowFast::ex(k.c2g * l);
+        sp = kp * PowFast::ex(k.inv_z * l);
+      }
+      sv[A] = k.two_gp1 * (k.hgm1 * sv[A] - sc);
+    }
+  }
+  return true;
+}
+
+// The FP64 state sampled at x/t = 0: side states, exact contacts (these need
+// no sound speed: both sides carry the upwind side's rho and v with p* = p,
+// u* = u), then star_sample; vacuum, pressures at or under the floor and
+// whatever star_sample refuses through riemann_sample_ref or the fixup.
+template <int ND, int A, class PW>
+__device__ __forceinline__ void riemann_sample(const Consts& k, const double* l, const double* r,
+                                               double& srho, double* sv, double& sp) {
+  if constexpr (!PW::kStar) {
+    riemann_sample_ref<ND, A, PW, double>(k, l, r, 0.0, srho, sv, sp);
+    return;
+  } else {
+    bool ok = plain_range(l[0]) && plain_range(r[0]) && l[0] >= k.e_rho && r[0] >= k.e_rho;
+    if (ok) {
+      const double il = recip(l[0]), ir = recip(r[0]);
+      double lv[ND], rv[ND], lk = 0.0, rk = 0.0;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        lv[d] = l[1 + d] * il;
+        rv[d] = r[1 + d] * ir;
+        lk = d == 0 ? l[1] * lv[0] : lk + l[1 + d] * lv[d];
+        rk = d == 0 ? r[1] * rv[0] : rk + r[1 + d] * rv[d];
+      }
+      const double lp = (l[ND + 1] - .5 * lk) * k.gm1;
+      const double rp = (r[ND + 1] - .5 * rk) * k.gm1;
+      ok = lp > k.w_p && rp > k.w_p && plain_range(lp) && plain_range(rp);
+#if RHY_CONTACT_EXACT
+      if (ok && lp == rp && lv[A] == rv[A]) {
+        const bool right = 0.0 > lv[A];
+        srho = right ? r[0] : l[0];
+        sp = lp;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) sv[d] = right ? rv[d] : lv[d];
+        return;
+      }
+#endif
+      // c^2 = gamma p / rho
+      if (ok)
+        ok = star_sample<ND, A>(k, l[0], lv, lp, sqrt_of(k.g * (lp * il)), r[0], rv, rp,
+                                sqrt_of(k.g * (rp * ir)), srho, sv, sp);
+    } else if (l[0] < k.e_rho && r[0] < k.e_rho) {  // vacuum on both sides
+      srho = k.w_rho;
+      sp = k.w_p;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) sv[d] = 0.0;
+      return;
+    }
+    if (!ok) {
+      if constexpr (PW::kDefer) {
+        defer_mark();
+        srho = 1.0;
+        sp = 1.0;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) sv[d] = 0.0;
+      } else {
+        riemann_sample_ref<ND, A, PW, double>(k, l, r, 0.0, srho, sv, sp);
+      }
+    }
+  }
+}
+
+// The conserved state sampled at x/t = dxdt (FP64 unit-level solve, the
+// reference's forms).
 template <int ND, int A, class PW = PowLib>
 __device__ __forceinline__ void riemann_state(const Consts& k, const double* l, const double* r,
                                               double dxdt, double* u) {
   double srho, sv[ND], sp;
-  riemann_sample<ND, A, PW, double>(k, l, r, dxdt, srho, sv, sp);
+  riemann_sample_ref<ND, A, PW, double>(k, l, r, dxdt, srho, sv, sp);
   prim_to_cons<ND, double>(k, srho, sv, sp, u);
 }
 
 // Riemann solve + calc_flux of the sampled state
-// (…_solve_memory_intensive.f90:110-116): the intercell flux.  R is the
-// type of the half states and of the flux (double: FP64 throughout; float:
-// the mixed form, whose conversions to and from primitive variables and
-// flux run in FP32 around the FP64 star-state solve and sampling).
+// (…_solve_memory_intensive.f90:110-116): the intercell flux.
+//
+// FP64: the flux is formed from the sampled primitive state,
+// F = (rho v_A, rho v_A v + p, v_A (rho v^2 / 2 + p g / (g-1))), rather than
+// through the conserved state and back: no division, and a gas at rest
+// passes on its p bit for bit.
+//
+// FP32 (the mixed form): primitive variables, conserved state and flux in
+// FP32 around the FP64 star state.  A wave whose faces are all exact
+// contacts takes the upwind states without the sound speeds, the vacuum tests
+// and the sampling, which round to those same FP32 states.
 template <int ND, int A, class PW, typename R>
 __device__ __forceinline__ void riemann_flux(const Consts& k, const R* l, const R* r, R* F) {
-  double srho, sv[ND], sp;
-  riemann_sample<ND, A, PW, R>(k, l, r, 0.0, srho, sv, sp);
-  R v[ND], u[ND + 2];
+  if constexpr (sizeof(R) == sizeof(double)) {
+    double rho, v[ND], p;
+    riemann_sample<ND, A, PW>(k, l, r, rho, v, p);
+    if (fabs(rho) < kTiny) {
 #pragma unroll
-  for (int d = 0; d < ND; ++d) v[d] = (R)sv[d];
-  prim_to_cons<ND, R>(k, (R)srho, v, (R)sp, u);
-  flux<ND, A, R>(k, u, F);
+      for (int c = 0; c < ND + 2; ++c) F[c] = 0.0;
+      return;
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) s = d == 0 ? v[0] * v[0] : s + v[d] * v[d];
+    const double m = rho * v[A];
+    F[0] = m;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) F[1 + d] = m * v[d];
+    F[1 + A] = F[1 + A] + p;
+    F[ND + 1] = v[A] * (.5 * rho * s + p * k.g_gm1);
+  } else {
+    R v[ND], rho, p, u[ND + 2];
+    bool contact = false;
+#if RHY_CONTACT_EXACT
+    const R lp = pressure<ND, R>(k, l), lva = rdiv<R>(l[1 + A], l[0]);
+    contact = wave_all(lp == pressure<ND, R>(k, r) && lva == rdiv<R>(r[1 + A], r[0]) &&
+                       (double)lp > k.w_p && lp < R(INFINITY) && (double)l[0] >= k.e_rho &&
+                       (double)r[0] >= k.e_rho);
+    if (contact) {
+      const bool right = R(0) > lva;
+      rho = right ? r[0] : l[0];
+      p = lp;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) v[d] = rdiv<R>(right ? r[1 + d] : l[1 + d], rho);
+    }
+#endif
+    if (!contact) {
+      double srho, sv[ND], sp;
+      riemann_sample_ref<ND, A, PW, R>(k, l, r, 0.0, srho, sv, sp);
+      rho = (R)srho;
+      p = (R)sp;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) v[d] = (R)sv[d];
+    }
+    prim_to_cons<ND, R>(k, rho, v, p, u);
+    flux<ND, A, R>(k, u, F);
+  }
 }
 
 }  // namespace rhy
