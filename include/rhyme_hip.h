@@ -200,8 +200,9 @@ int rhy_box_last_dts(rhy_box_t *box, int32_t n, double *dts);
  * nothing else, so that the events (a few microseconds each) perturb only
  * the sampled steps; on = 0: off.  rhy_box_kernel_stats returns, for kernel
  * index kidx (0: the flux kernels, 1: update, 2: bc, 3: cfl, 4: dt, 5: the
- * deferred-face list reset and fixup), the number of launches timed and their
- * summed milliseconds.  RHY_ERR_ARG for on < 0. */
+ * deferred-face list reset and fixup), the number of launches timed (0: of
+ * axis walks; a kernel that walks two axes counts as two) and their summed
+ * milliseconds.  RHY_ERR_ARG for on < 0. */
 int rhy_box_set_profiling(rhy_box_t *box, int32_t on);
 int rhy_box_kernel_stats(rhy_box_t *box, int32_t kidx, int64_t *launches,
                          double *total_ms);
@@ -479,10 +480,9 @@ int rhy_batch_last_deferred(rhy_batch_t *batch, int64_t *n);
  *   levels); for callers of the hierarchy.  The coarse step as the ghost
  *   fill and one step with the given dt (rhy_bc_set_boundaries +
  *   rhy_mh_solve, bit for bit) through the accumulating walks of rhy_run
- *   instead of the flux planes: only the x fluxes stay in the flux planes,
- *   and the box keeps the state it stepped from in its second state buffer,
- *   from which rhy_amr_reflux forms the y/z coarse fluxes it needs (as the
- *   walks formed them, bit for bit).  Any later call that changes the box
+ *   instead of the flux planes: the box keeps the state it stepped from in
+ *   its second state buffer, from which rhy_amr_reflux forms the coarse
+ *   fluxes it needs (as the walks formed them, bit for bit).  Any later call that changes the box
  *   (upload, step, paint, draw, resize, unpack) ends that; the box's ghost
  *   faces are not filled after the step.  1D boxes take rhy_mh_solve.
  * The prolong, restrict, register and reflux calls wait for both sides'

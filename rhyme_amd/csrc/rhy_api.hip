@@ -58,6 +58,7 @@ constexpr int kNumKernelIds = 6;  // flux/step, update, bc, cfl, dt, deferred-fa
 struct TimedLaunch {
   int kidx;
   hipEvent_t a, b;
+  int axes = 1;  // axis walks the launch makes (walk_xy_kernel: 2)
 };
 
 }  // namespace
@@ -83,7 +84,7 @@ struct rhy_box {
   double* partial = nullptr;      // per-block CFL maxima of the last reduction
   int32_t partial_n = 0;          // partials of the stand-alone CFL pass
   int32_t acc_blocks = 0;         // partials of the last accumulating walk
-  int32_t nf_x = 8, acc_L = 16;   // walk lengths for this shape (choose_walks)
+  int32_t nf_x = 8, xy_L = 16, acc_L = 16;  // walk lengths for this shape (alloc_box_memory)
   int32_t partial_cap = 0;
   double* scalars = nullptr;      // [0] max_u, [16..16+6*RHY_MAX_CMP) inflow states
   double inflow_copied[6 * RHY_MAX_CMP] = {};  // what the device inflow slots hold
@@ -177,7 +178,7 @@ void collect_timings(rhy_box* b) {
   for (auto& tl : b->pending) {
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, tl.a, tl.b) == hipSuccess) {
-      b->launches[tl.kidx] += 1;
+      b->launches[tl.kidx] += tl.axes;
       b->total_ms[tl.kidx] += ms;
     }
     (void)hipEventDestroy(tl.a);
@@ -400,72 +401,69 @@ int ensure_dt_log(rhy_box* b, int32_t n) {
 // them with dt): scalars[8..14]
 double* step_consts(rhy_box* b) { return b->scalars + 8; }
 
-// The deferred-face list of axis a in the accumulating step.
-DeferList defer_list_axis(rhy_box* b, int a) {
+// The deferred-face lists of the accumulating step: of walk_xy (the x and y
+// axes' parts together) and of the z walk.
+DeferList defer_list_walk(rhy_box* b, bool z) {
   DeferList dl;
+  const int a = z ? 2 : 0;
+  const uint32_t room = z ? b->defer_cap_axis[2] : b->defer_cap_axis[0] + b->defer_cap_axis[1];
   dl.count = b->defer_count + a;
   dl.items = b->defer_items + b->defer_off_axis[a];
   const int64_t cap = defer_cap_setting();
-  dl.cap = cap >= 0 ? (uint32_t)std::min<int64_t>(cap, b->defer_cap_axis[a])
-                    : b->defer_cap_axis[a];
+  dl.cap = cap >= 0 ? (uint32_t)std::min<int64_t>(cap, room) : room;
   return dl;
 }
 
-// One accumulating walk (and its fixup) along A of an ND box: reads the
-// current state, writes Q (kAccMid) or the other state buffer (kAccLast).
-template <int ND, int A, int LIM, typename R, class PW, class P, int MODE>
-void launch_acc_axis(rhy_box* b, const Consts& k, const double* dx,
-                     int order) {
-  const Geom& G = b->geom;
-  const int nv = ND + 2;
-  const R* cur = static_cast<const R*>(b->cells);
-  const R* fx = static_cast<const R*>(b->flux);
-  R* q = static_cast<R*>(b->flux) + (int64_t)nv * G.plane;
-  R* other = static_cast<R*>(b->state[1 - b->cur]);
-  const R* acc = MODE == kAccLast && ND == 3 ? q : nullptr;
-  R* out = MODE == kAccMid ? q : other;
-  double* slot = b->partial + b->acc_blocks;
-  const DeferList dl = defer_list_axis(b, A);
-  TimedLaunch tl;
-  timed_begin(b, 0, tl);
-  hipLaunchKernelGGL((acc_walk_kernel<ND, A, LIM, R, PW, MODE>),
-                     dim3(grid_for(acc_threads(G, A, b->acc_L))), dim3(kThreads), 0, b->stream, k,
-                     G, cur, fx, acc, out, step_consts(b), b->acc_L, order, dl, b->partial);
-  timed_end(b, tl);
-  if constexpr (PW::kDefer) {
-    TimedLaunch tf;
-    timed_begin(b, 5, tf);
-    hipLaunchKernelGGL((acc_fixup_kernel<ND, A, R, P, MODE>), dim3(kFixupBlocks), dim3(kThreads),
-                       0, b->stream, k, G, cur, fx, acc, out, b->dt, dx[0], dx[A], order, dl,
-                       slot);
-    timed_end(b, tf);
-  }
+// The fixup of an accumulating walk.
+template <int WALK, typename R, class P>
+void launch_acc_fixup(rhy_box* b, const Consts& k, const double* dx, int order,
+                      const DeferList& dl, const R* acc, R* out) {
+  TimedLaunch tf;
+  timed_begin(b, 5, tf);
+  hipLaunchKernelGGL((acc_fixup_kernel<WALK, R, P>), dim3(kFixupBlocks), dim3(kThreads), 0,
+                     b->stream, k, b->geom, static_cast<const R*>(b->cells), acc, out, b->dt,
+                     dx[0], dx[1], WALK == kFixXy2 ? 1.0 : dx[2], order, dl,
+                     b->partial + b->acc_blocks);
+  timed_end(b, tf);
 }
 
-// One step of a 2D/3D box without the flux-plane update pass: the x walk's
-// fluxes into the first flux planes (and their fixup), then the
-// accumulating walks; the new state lands in the other state buffer.
+// One step of a 2D/3D box through the accumulating walks: x and y together
+// into Q (3D, the first flux planes) or the other state buffer (2D), then z
+// into the other state buffer, each followed by its fixup.
 template <int ND, int LIM, typename R, class PW, class P>
 void launch_acc_step_lim(rhy_box* b, const Consts& k, const double* dx,
                          int order) {
   static_assert(ND > 1, "1D boxes step through the flux planes");
   // the deferred-face counters and the fixup's partial slot were reset by
   // the step's dt_kernel (rhy_run) or set_step_kernel (rhy_amr_coarse_step)
-  const DeferList dlx = defer_list_axis(b, 0);
-  launch_flux_axis<ND, 0, LIM, R, PW>(b, k, dx, dlx);
-  if constexpr (PW::kDefer) {
-    TimedLaunch tf;
-    timed_begin(b, 5, tf);
-    hipLaunchKernelGGL((flux_fixup_kernel<ND, R, P>), dim3(kFixupBlocks), dim3(kThreads), 0,
-                       b->stream, k, b->geom, static_cast<const R*>(b->cells),
-                       static_cast<R*>(b->flux), b->dt, dx[0], dx[1], dx[2], dlx, 0);
-    timed_end(b, tf);
-  }
+  constexpr int MODE = ND == 3 ? kAccMid : kAccLast;
+  const Geom& G = b->geom;
+  const R* cur = static_cast<const R*>(b->cells);
+  R* q = static_cast<R*>(b->flux);
+  R* other = static_cast<R*>(b->state[1 - b->cur]);
+  R* xy = ND == 3 ? q : other;
+  const DeferList dlxy = defer_list_walk(b, false);
+  TimedLaunch tl;
+  timed_begin(b, 0, tl);
+  hipLaunchKernelGGL((walk_xy_kernel<ND, LIM, R, PW, MODE>),
+                     dim3(grid_for(xy_threads(G, b->xy_L))), dim3(kThreads), 0, b->stream, k, G,
+                     cur, xy, step_consts(b), b->xy_L, order, xy_waves(G), dlxy, b->partial);
+  tl.axes = 2;
+  timed_end(b, tl);
+  if constexpr (PW::kDefer)
+    launch_acc_fixup<ND == 3 ? kFixXy3 : kFixXy2, R, P>(b, k, dx, order, dlxy, (const R*)nullptr,
+                                                        xy);
   if constexpr (ND == 3) {
-    launch_acc_axis<ND, 1, LIM, R, PW, P, kAccMid>(b, k, dx, order);
-    launch_acc_axis<ND, 2, LIM, R, PW, P, kAccLast>(b, k, dx, order);
-  } else {
-    launch_acc_axis<ND, 1, LIM, R, PW, P, kAccLast>(b, k, dx, order);
+    const DeferList dlz = defer_list_walk(b, true);
+    tl.axes = 1;
+    timed_begin(b, 0, tl);
+    hipLaunchKernelGGL((acc_walk_kernel<LIM, R, PW>),
+                       dim3(grid_for(acc_threads(G, 2, b->acc_L))), dim3(kThreads), 0, b->stream,
+                       k, G, cur, (const R*)q, other, step_consts(b), b->acc_L, order, dlz,
+                       b->partial);
+    timed_end(b, tl);
+    if constexpr (PW::kDefer)
+      launch_acc_fixup<kFixZ, R, P>(b, k, dx, order, dlz, (const R*)q, other);
   }
   b->cur = 1 - b->cur;
   b->cells = b->state[b->cur];
@@ -584,15 +582,14 @@ int alloc_box_memory(rhy_box* b) {
   b->partial_n = (int32_t)grid_for(ncell);
   b->nf_x = kNfX;
   while (b->nf_x > 2 && flux_threads(b->geom, 0, b->nf_x) / 64 < kMinWavesX) b->nf_x /= 2;
-  b->acc_L = kAccL;
-  auto acc_waves = [&](int L) {
-    int64_t w = (int64_t)1 << 62;
-    for (int a = 1; a < b->ndim; ++a) w = std::min(w, acc_threads(b->geom, a, L) / 64);
-    return w;
-  };
-  while (b->ndim > 1 && b->acc_L > 4 && acc_waves(b->acc_L) < kMinWavesAcc) b->acc_L /= 2;
-  b->acc_blocks =
-      b->ndim > 1 ? (int32_t)grid_for(acc_threads(b->geom, b->ndim - 1, b->acc_L)) : 0;
+  b->xy_L = b->acc_L = kAccL;
+  while (b->ndim > 1 && b->xy_L > 4 && xy_threads(b->geom, b->xy_L) / 64 < kMinWavesAcc)
+    b->xy_L /= 2;
+  while (b->ndim > 2 && b->acc_L > 4 && acc_threads(b->geom, 2, b->acc_L) / 64 < kMinWavesAcc)
+    b->acc_L /= 2;
+  b->acc_blocks = b->ndim == 3   ? (int32_t)grid_for(acc_threads(b->geom, 2, b->acc_L))
+                  : b->ndim == 2 ? (int32_t)grid_for(xy_threads(b->geom, b->xy_L))
+                                 : 0;
   // one more slot: the CFL speeds of cells the fixup recomputed
   b->partial_cap = std::max(b->partial_n, b->acc_blocks) + 1;
   if (dev_alloc(&b->partial, sizeof(double) * (size_t)b->partial_cap) != hipSuccess) {
@@ -753,6 +750,7 @@ int rhy_box_resize(rhy_box_t* b, const int32_t dims[3]) {
   b->partial_n = t.partial_n;
   b->acc_blocks = t.acc_blocks;
   b->nf_x = t.nf_x;
+  b->xy_L = t.xy_L;
   b->acc_L = t.acc_L;
   b->partial_cap = t.partial_cap;
   b->defer_count = t.defer_count;
@@ -1199,7 +1197,7 @@ int rhy_amr_coarse_step(rhy_box_t* b, const rhy_params_t* p, const double dx[3],
                     : launch_acc_step<3>(b, k, dx, p->solver_type);
   if (rc) return rc;
   b->coarse_walked = true;  // after launch_acc_step: the state it stepped from is
-  b->coarse_k = k;          // state[1 - cur], its x fluxes in the first flux planes
+  b->coarse_k = k;          // state[1 - cur]
   b->coarse_dt = dt;
   for (int d = 0; d < 3; ++d) b->coarse_dx[d] = d < b->ndim ? dx[d] : 1.0;
   HIP_TRY(hipStreamSynchronize(b->stream));

@@ -570,10 +570,10 @@ __global__ __launch_bounds__(256) void amr_register_kernel(const AmrItem* __rest
 // Reflux of one (axis, side) pass: the coarse cell outside each listed face
 // takes dtdx (F_c - <F_f>) (low side) or dtdx (<F_f> - F_c) (high side),
 // <F_f> = register * 2^-ndim (the mean over 2 substeps and 2^(ndim-1) faces).
-// F_c from the coarse flux planes (FROM_STATE = 0), or, for a pass along
-// axis FROM_STATE > 0 after rhy_amr_coarse_step, formed from the pre-step
+// F_c from the coarse flux planes (FROM_STATE < 0), or, for a pass along
+// axis FROM_STATE after rhy_amr_coarse_step, formed from the pre-step
 // state `prev` with policy P, the step's constants k, dt and dx.
-template <int ND, typename R, int FROM_STATE = 0, class P = PowF64Fix>
+template <int ND, typename R, int FROM_STATE = -1, class P = PowF64Fix>
 __global__ __launch_bounds__(256) void amr_reflux_kernel(const AmrItem* __restrict__ items,
                                                          int nitems, int64_t total, int64_t base,
                                                          const double* __restrict__ reg,
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void amr_reflux_kernel(const AmrItem* __restri
   const int64_t oo = goff(GC, out[0], out[1], out[2]);
   const int64_t ol = goff(GC, low[0], low[1], low[2]);
   R Fs[ND + 2];
-  if constexpr (FROM_STATE > 0) {
+  if constexpr (FROM_STATE >= 0) {
     // the coarse face's flux formed again from the state the coarse step
     // started from, as the step's walk formed it
     face_flux<ND, FROM_STATE, R, P>(k, GC, prev, dt, dx, ol, Fs);
@@ -612,7 +612,7 @@ __global__ __launch_bounds__(256) void amr_reflux_kernel(const AmrItem* __restri
   for (int c = 0; c < ND + 2; ++c) {
     const double favg = r[c] * w;
     double fc;
-    if constexpr (FROM_STATE > 0)
+    if constexpr (FROM_STATE >= 0)
       fc = (double)Fs[c];
     else
       fc = (double)cflux[ol + (int64_t)a * (ND + 2) * GC.plane + c * GC.plane];
@@ -1954,16 +1954,20 @@ static int amr_reflux_v(const BoxView& vc, rhy_batch_t* f, const int32_t* lo, do
                      dim3(256), 0, f->stream, items, ni, f->reg_pt[pass], base, f->amr_reg,    \
                      vc.geom, static_cast<R*>(vc.cells), static_cast<const R*>(vc.flux), dtdx, \
                      vc.k, static_cast<const R*>(vc.prev), vc.step_dt, vc.step_dx[a])
-    if (vc.prev && a > 0) {  // y/z coarse fluxes of an accumulating coarse step
+    if (vc.prev) {  // coarse fluxes of an accumulating coarse step
       if (f->precision == RHY_MIXED) {
-        if (nd == 2) RHY_REFLUX_S(2, 1, float, MixedMath);
+        if (nd == 2) {
+          if (a == 0) RHY_REFLUX_S(2, 0, float, MixedMath);
+          else RHY_REFLUX_S(2, 1, float, MixedMath);
+        } else if (a == 0) RHY_REFLUX_S(3, 0, float, MixedMath);
         else if (a == 1) RHY_REFLUX_S(3, 1, float, MixedMath);
         else RHY_REFLUX_S(3, 2, float, MixedMath);
-      } else {
-        if (nd == 2) RHY_REFLUX_S(2, 1, double, PowF64Fix);
-        else if (a == 1) RHY_REFLUX_S(3, 1, double, PowF64Fix);
-        else RHY_REFLUX_S(3, 2, double, PowF64Fix);
-      }
+      } else if (nd == 2) {
+        if (a == 0) RHY_REFLUX_S(2, 0, double, PowF64Fix);
+        else RHY_REFLUX_S(2, 1, double, PowF64Fix);
+      } else if (a == 0) RHY_REFLUX_S(3, 0, double, PowF64Fix);
+      else if (a == 1) RHY_REFLUX_S(3, 1, double, PowF64Fix);
+      else RHY_REFLUX_S(3, 2, double, PowF64Fix);
     } else if (f->precision == RHY_MIXED) {
       if (nd == 1) RHY_REFLUX(1, float);
       else if (nd == 2) RHY_REFLUX(2, float);

@@ -94,7 +94,7 @@ __device__ __forceinline__ double* walk_ring() {
   return ring;
 }
 
-// The flux of the last face of each lane of a 256-thread workgroup (5
+// The flux of the last y or z face of each lane of a 256-thread workgroup (5
 // values), for the accumulating walks: the cell between two faces of a
 // walk takes both, and the lower one waits here across the Riemann solve of
 // the upper one instead of in registers.
@@ -149,7 +149,7 @@ inline Consts consts_of(const rhy_params_t* p) {
 // the box's stream).
 struct BoxView {
   void* cells;
-  void* flux;  // flux planes of the last rhy_mh_solve (the x planes after rhy_amr_coarse_step)
+  void* flux;  // flux planes of the last rhy_mh_solve
   void* prev;  // after rhy_amr_coarse_step: the state it stepped from, else nullptr
   Consts k;    // that step's constants, dt and dx (with prev)
   double step_dt, step_dx[3];
@@ -586,119 +586,220 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void flux_kernel(
 
 // ------------------------------------------------ accumulating walks ----
 //
-// The single-box step without a separate update pass.  The x walk stores
-// its fluxes F_x (flux_kernel).  Walking y and z, a lane takes a chunk of L
-// consecutive cells c0 .. c0+L-1 and solves the L+1 faces c0-1 .. c0+L-1
-// around them (one face more than the cells, shared with the neighbouring
-// chunk), so that every cell of the chunk has both its faces in the walk:
-//   kAccMid  (y of a 3D box): Q = A + B (memory_intensive) or (u + A) + B
-//            (cpu_intensive), A = dt/dx_x (F_x[c-1] - F_x[c]) from the F_x
-//            planes, B = dt/dx_y (F_y[c-1] - F_y[c]) from the walk;
-//   kAccLast (z of a 3D box, y of a 2D box): the new state u + (Q + C) or
-//            Q + C (3D), u + (A + B) or (u + A) + B (2D), written to the
-//            other state buffer (interior only: a ghost fill of the new
-//            state follows the step), and its CFL speed folded into the
-//            lane's maximum.
+// The single-box step without a separate update pass and without flux
+// planes.  walk_xy solves the x and y faces of a column of rows together and
+// forms what both contribute to a cell as soon as its upper y face is solved:
+//   kAccMid  (3D box): Q = A + B (memory_intensive) or (u + A) + B
+//            (cpu_intensive), A = dt/dx_x (F_x[c-1] - F_x[c]),
+//            B = dt/dx_y (F_y[c-1] - F_y[c]);
+//   kAccLast (2D box): the new state u + (A + B) or (u + A) + B.
+// In 3D, flux_walk_acc (kAccLast) then walks z: a lane takes a chunk of L
+// consecutive cells c0 .. c0+L-1 and solves the L+1 faces around them (one
+// more than the cells, shared with the neighbouring chunk), reads Q and
+// writes u + (Q + C) or Q + C.  The new state goes to the other state buffer
+// (interior only: a ghost fill of the new state follows the step), its CFL
+// speed into the lane's maximum.
 // These are the update's expressions operation for operation
 // (rhyme_muscl_hancock_solve_memory_intensive.f90:142-176,
 // …_solve_cpu_intensive.f90:117-136), so the state equals the flux-plane
 // path's bit for bit.  A cell beside a face the walk deferred gets a
-// placeholder here and no CFL speed; acc_fixup_kernel recomputes it.
+// placeholder here and no CFL speed; the walk's fixup kernel recomputes it.
 constexpr int kAccMid = 1, kAccLast = 2;
 
-// The accumulation of component value uc of one cell (q: its offset in the
-// component's plane) from its lower and upper face fluxes fl, fu along A;
-// stored to out[q] and returned.
-template <int ND, int A, typename R, int MODE>
-__device__ __forceinline__ R acc_one(const Geom& G, const R* __restrict__ fx,
-                                     const R* __restrict__ acc, R* __restrict__ out, int64_t q,
-                                     R uc, R fl, R fu, R dtdx0, R dtdxA, int order) {
-  const R b = dtdxA * (fl - fu);
-  R v;
-  if constexpr (MODE == kAccMid || ND == 2) {
-    const R a0 = dtdx0 * (fx[q - G.s[0]] - fx[q]);
-    if constexpr (MODE == kAccMid)
-      v = order == RHY_MEMORY_INTENSIVE ? a0 + b : (uc + a0) + b;
-    else
-      v = order == RHY_MEMORY_INTENSIVE ? uc + (a0 + b) : (uc + a0) + b;
-  } else {
-    v = order == RHY_MEMORY_INTENSIVE ? uc + (acc[q] + b) : acc[q] + b;
+// A cell's value from its state uc and the axes' contributions in the order
+// of the solver: the x and y ones (a0, b) to Q or, in 2D, the new state; Q
+// and the z one (q, c) to the new state.
+template <typename R, int MODE>
+__device__ __forceinline__ R acc_xy(R uc, R a0, R b, int order) {
+  if constexpr (MODE == kAccMid) return order == RHY_MEMORY_INTENSIVE ? a0 + b : (uc + a0) + b;
+  return order == RHY_MEMORY_INTENSIVE ? uc + (a0 + b) : (uc + a0) + b;
+}
+template <typename R>
+__device__ __forceinline__ R acc_z(R uc, R q, R c, int order) {
+  return order == RHY_MEMORY_INTENSIVE ? uc + (q + c) : q + c;
+}
+
+// Lane l gets lane l+1's value (lane 63 keeps its own): DPP wave_shl:1.
+__device__ __forceinline__ uint32_t wave_shl1(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x130, 0xf, 0xf, false);
+}
+__device__ __forceinline__ float lane_above(float x) {
+  return __builtin_bit_cast(float, wave_shl1(__builtin_bit_cast(uint32_t, x)));
+}
+__device__ __forceinline__ double lane_above(double x) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  const uint64_t lo = wave_shl1((uint32_t)b), hi = wave_shl1((uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, lo | (hi << 32));
+}
+
+// walk_xy: a wave takes 64 consecutive columns of the x rows at one y --
+// columns numbered row after row over z with all ghosts, n0 + 4 to a row, so
+// that they are consecutive in memory -- and walks L cells along y.  Each
+// lane's cells pass through its LDS ring (loaded from HBM once, the next one
+// during the half steps).  At a row, the x half steps take their stencil from
+// the neighbouring lanes' ring slots, the low side of the face (l-1, l) and
+// the flux of the face (l, l+1) come from the neighbouring lanes by DPP, so
+// that lanes 2..61 own a cell with both its x faces; the y half step and face
+// run on the owning lanes.  Nothing but the fluxes' differences leaves the
+// registers: no F_x planes (3D: 2.1 of 5.6 GB per 256^3 step saved).  Halo lanes
+// cost 4 in 64 and the row's ghosts 4 in n0 + 4, a chunk one y face and two
+// half steps more than its cells.
+constexpr int kXyOwn = 60;
+
+template <int ND, int LIM, typename R, class PW, int MODE>
+__device__ __forceinline__ double walk_xy(const Consts& k, const Geom& G,
+                                          const R* __restrict__ cells, R* __restrict__ out,
+                                          const double* __restrict__ sc, int L, int order,
+                                          int32_t wave, int32_t nwaves, const DeferList& dl) {
+  constexpr int NV = ND + 2;
+  defer_clear<PW>();
+  double smax = 0.0;
+  const int32_t rowlen = G.n[0] + 4;
+  const int32_t ncol = rowlen * G.n[2];
+  const int32_t chunk = wave / nwaves;
+  const int f0 = chunk * L;
+  if (f0 >= G.n[1]) return smax;  // the whole wave
+  const int nc = G.n[1] - f0 < L ? G.n[1] - f0 : L;  // cells f0+1 .. f0+nc
+  const int lane = threadIdx.x & 63;
+  int32_t q = (wave - chunk * nwaves) * kXyOwn + lane;
+  const bool valid = q < ncol;
+  q = valid ? q : ncol - 1;
+  const int32_t row = q / rowlen;
+  const int ci = q - row * rowlen - 1;  // x index, -1 .. n0+2
+  const bool own = valid && lane >= 2 && lane <= 61 && ci >= 1 && ci <= G.n[0];
+  const bool xhalf = valid && lane >= 1 && lane <= 62 && ci >= 0 && ci <= G.n[0] + 1;
+  const bool xface = valid && lane >= 2 && lane <= 62 && ci >= 1 && ci <= G.n[0] + 1;
+  const int64_t o = goff(G, ci, f0, row + 1);
+  const int64_t s = G.s[1];
+  const R dtdx0 = (R)sc[1], dtdx1 = (R)sc[2];
+  const R hdtdx0 = (R)sc[4], hdtdx1 = (R)sc[5];
+  R* ring = reinterpret_cast<R*>(walk_ring()) + threadIdx.x;
+  R* fprev = reinterpret_cast<R*>(walk_fprev()) + threadIdx.x;
+  auto put = [&](int j, const R* v) {
+#pragma unroll
+    for (int c = 0; c < NV; ++c) ring[((j & 3) * NV + c) * kWalkLanes] = v[c];
+  };
+  auto get = [&](int j, int at, R* v) {
+#pragma unroll
+    for (int c = 0; c < NV; ++c) v[c] = ring[((j & 3) * NV + c) * kWalkLanes + at];
+  };
+  R rp[NV];
+  {
+    R um[NV], u0[NV], up[NV], lw[NV], nx[NV];
+    load_state<ND, R>(cells, G.plane, o - s, um);
+    load_state<ND, R>(cells, G.plane, o, u0);
+    load_state<ND, R>(cells, G.plane, o + s, up);
+    load_state<ND, R>(cells, G.plane, o + 2 * s, nx);
+    put(0, u0);
+    put(1, up);
+    put(2, nx);
+#pragma unroll
+    for (int c = 0; c < NV; ++c) rp[c] = R(0);
+    if (own) half_step<ND, 1, LIM, R>(k, um, u0, up, hdtdx1, lw, rp);
   }
-  out[q] = v;
-  return v;
-}
-
-// All components of one cell (offset oc, state uc, face fluxes fl, fu);
-// the new values also into un.
-template <int ND, int A, typename R, int MODE>
-__device__ __forceinline__ void acc_cell(const Geom& G, const R* __restrict__ fx,
-                                         const R* __restrict__ acc, R* __restrict__ out,
-                                         int64_t oc, const R* uc, const R* fl, const R* fu,
-                                         R dtdx0, R dtdxA, int order, R* un) {
+  bool dyp = false;  // face m - 1 deferred
+#pragma unroll 1
+  for (int m = 0; m <= nc; ++m) {  // face m, between cells f0 + m and f0 + m + 1
+    R nx[NV], a0[NV];
+    if (m < nc) load_state<ND, R>(cells, G.plane, o + (m + 3) * s, nx);
+    bool dx = false;  // an x face of the cell deferred
+    if (m > 0) {
+      // neighbouring lanes' slots are read below: their stores come first
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      R um[NV], u0[NV], up[NV], lx[NV], rx[NV], F[NV];
 #pragma unroll
-  for (int c = 0; c < ND + 2; ++c)
-    un[c] = acc_one<ND, A, R, MODE>(G, fx, acc, out, oc + c * G.plane, uc[c], fl[c], fu[c],
-                                    dtdx0, dtdxA, order);
-}
-
-// What the epilogue of one cell reads from HBM: F_x at the cell and below
-// it (kAccMid, and kAccLast of a 2D box), or Q at the cell (kAccLast, 3D).
-template <int ND, typename R, int MODE>
-struct AccLoads {
-  static constexpr bool kFx = MODE == kAccMid || ND == 2;
-  R a[ND + 2];  // F_x[c - 1] or Q[c]
-  R b[ND + 2];  // F_x[c]
-  __device__ __forceinline__ void load(const Geom& G, const R* __restrict__ fx,
-                                       const R* __restrict__ acc, int64_t oc) {
+      for (int c = 0; c < NV; ++c) lx[c] = rx[c] = F[c] = R(0);
+      if (xhalf) {
+        get(m, -1, um);
+        get(m, 0, u0);
+        get(m, 1, up);
+        half_step<ND, 0, LIM, R>(k, um, u0, up, hdtdx0, lx, rx);
+      }
 #pragma unroll
-    for (int c = 0; c < ND + 2; ++c) {
-      const int64_t q = oc + c * G.plane;
-      if constexpr (kFx) {
-        a[c] = fx[q - G.s[0]];
-        b[c] = fx[q];
-      } else {
-        a[c] = acc[q];
+      for (int c = 0; c < NV; ++c) rx[c] = lane_below(rx[c]);
+      uint32_t dlo = 0;
+      if (xface) {
+        riemann_flux<ND, 0, PW, R>(k, rx, lx, F);
+        dlo = defer_take<PW>(k, dl, 0u, 0, o + (int64_t)m * s - 1) ? 1u : 0u;
+      }
+#pragma unroll
+      for (int c = 0; c < NV; ++c) a0[c] = dtdx0 * (F[c] - lane_above(F[c]));
+      if constexpr (PW::kDefer) dx = (dlo | wave_shl1(dlo)) != 0;
+    }
+    if (own) {
+      R um[NV], u0[NV], up[NV], lw[NV], rn[NV], F[NV];
+      get(m, 0, um);
+      get(m + 1, 0, u0);
+      get(m + 2, 0, up);
+      half_step<ND, 1, LIM, R>(k, um, u0, up, hdtdx1, lw, rn);
+      riemann_flux<ND, 1, PW, R>(k, rp, lw, F);
+      const bool dy = defer_take<PW>(k, dl, 0u, 1, o + (int64_t)m * s);
+      if (m > 0) {
+        const int64_t oc = o + (int64_t)m * s;
+        R un[NV];
+        get(m, 0, u0);
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          un[c] = acc_xy<R, MODE>(u0[c], a0[c], dtdx1 * (fprev[c * kWalkLanes] - F[c]), order);
+          out[oc + c * G.plane] = un[c];
+        }
+        if constexpr (MODE == kAccLast) {
+          if (!(dx || dy || dyp)) {  // deferred faces: the fixup's speed
+            double ud[NV];
+#pragma unroll
+            for (int c = 0; c < NV; ++c) ud[c] = (double)un[c];
+            const double sp = cfl_speed<ND>(k, ud);
+            smax = sp > smax ? sp : smax;
+          }
+        }
+      }
+      dyp = dy;
+#pragma unroll
+      for (int c = 0; c < NV; ++c) {
+        fprev[c * kWalkLanes] = F[c];
+        rp[c] = rn[c];
       }
     }
+    if (m < nc) put(m + 3, nx);
   }
-};
-
-// acc_one with the cell's loads already in registers (same arithmetic).
-template <int ND, typename R, int MODE>
-__device__ __forceinline__ R acc_one_loaded(R* __restrict__ out, int64_t q, R uc, R fl, R fu,
-                                            R xa, R xb, R dtdx0, R dtdxA, int order) {
-  const R b = dtdxA * (fl - fu);
-  R v;
-  if constexpr (MODE == kAccMid || ND == 2) {
-    const R a0 = dtdx0 * (xa - xb);
-    if constexpr (MODE == kAccMid)
-      v = order == RHY_MEMORY_INTENSIVE ? a0 + b : (uc + a0) + b;
-    else
-      v = order == RHY_MEMORY_INTENSIVE ? uc + (a0 + b) : (uc + a0) + b;
-  } else {
-    v = order == RHY_MEMORY_INTENSIVE ? uc + (xa + b) : xa + b;
-  }
-  out[q] = v;
-  return v;
+  return smax;
 }
 
-template <int ND, int A, int LIM, typename R, class PW, int MODE>
+// Waves across the columns of walk_xy.
+__host__ __device__ inline int32_t xy_waves(const Geom& G) {
+  return ((G.n[0] + 4) * G.n[2] - 4 + kXyOwn - 1) / kXyOwn;
+}
+// Threads of walk_xy with chunks of L cells.
+__host__ __device__ inline int64_t xy_threads(const Geom& G, int L) {
+  return (int64_t)xy_waves(G) * ((G.n[1] + L - 1) / L) * 64;
+}
+
+template <int ND, int LIM, typename R, class PW, int MODE>
+__global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void walk_xy_kernel(
+    Consts k, Geom G, const R* __restrict__ cells, R* __restrict__ out,
+    const double* __restrict__ sc, int L, int order, int32_t nwaves, DeferList dl,
+    double* __restrict__ partial) {
+  const int32_t wave =
+      __builtin_amdgcn_readfirstlane((int32_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
+  const double sp = walk_xy<ND, LIM, R, PW, MODE>(k, G, cells, out, sc, L, order, wave, nwaves, dl);
+  if constexpr (MODE == kAccLast) block_max_to_partial(sp, partial);
+}
+
+template <int LIM, typename R, class PW>
 __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
                                                 const R* __restrict__ cells,
-                                                const R* __restrict__ fx,
                                                 const R* __restrict__ acc, R* __restrict__ out,
                                                 const double* __restrict__ sc, int L,
                                                 int order, int64_t t, const DeferList& dl) {
-  static_assert(A > 0 && A < ND, "the accumulating walks run along y or z");
-  constexpr int NV = ND + 2;
+  constexpr int ND = 3, A = 2, NV = ND + 2;
   defer_clear<PW>();
   double smax = 0.0;
   const int nA = G.n[A];
   const int nchunk = (nA + L - 1) / L;
   const int e0 = G.n[0];
-  const int e1 = A == 1 ? nchunk : G.n[1];
-  const int e2 = A == 2 ? nchunk : G.n[2];
-  if (t >= (int64_t)e0 * e1 * e2) return smax;
+  const int e1 = G.n[1];
+  if (t >= (int64_t)e0 * e1 * nchunk) return smax;
   int idx[3];
   idx[0] = (int)(t % e0);
   const int64_t rr = t / e0;
@@ -714,7 +815,6 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
   // scalar registers)
   const R hdtdx = (R)sc[4 + A];
   const R dtdxA = (R)sc[1 + A];
-  const R dtdx0 = (R)sc[1];
   // cells of the walk through the lane's LDS ring (cell j from f0 in slot
   // j & 3, the next one loaded during the half step, as in flux_walk); the
   // lower face's flux of the next cell in the lane's walk_fprev slot
@@ -741,11 +841,11 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
   put(2, nx);
   // The walk is software-pipelined: the cell between faces m-2 and m-1 is
   // finished at face m, between that face's half step and its Riemann
-  // solve.  Its loads (AccLoads) are issued at the top of the iteration and
+  // solve.  Its loads of Q are issued at the top of the iteration and
   // arrive during the half step; its upper face's flux waits in registers
   // across the half step, its lower one in the lane's walk_fprev slot;
   // nothing more than a plain walk holds is live across a Riemann solve.
-  auto finish = [&](int j, const R* fu, const AccLoads<ND, R, MODE>& ld, bool deferred) {
+  auto finish = [&](int j, const R* fu, const R* qc, bool deferred) {
     const int64_t oc = o + (int64_t)j * s;
     R un[NV];
 #pragma unroll
@@ -753,18 +853,15 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
       const R fl = fprev[c * kWalkLanes + lane];
       fprev[c * kWalkLanes + lane] = fu[c];
       const R uc = ring[((j & 3) * NV + c) * kWalkLanes + lane];
-      un[c] = acc_one_loaded<ND, R, MODE>(out, oc + c * G.plane, uc, fl, fu[c], ld.a[c],
-                                          AccLoads<ND, R, MODE>::kFx ? ld.b[c] : R(0), dtdx0,
-                                          dtdxA, order);
+      un[c] = acc_z<R>(uc, qc[c], dtdxA * (fl - fu[c]), order);
+      out[oc + c * G.plane] = un[c];
     }
-    if constexpr (MODE == kAccLast) {
-      if (!deferred) {  // a deferred face: the fixup recomputes the speed
-        double ud[NV];
+    if (!deferred) {  // a deferred face: the fixup recomputes the speed
+      double ud[NV];
 #pragma unroll
-        for (int c = 0; c < NV; ++c) ud[c] = (double)un[c];
-        const double sp = cfl_speed<ND>(k, ud);
-        smax = sp > smax ? sp : smax;
-      }
+      for (int c = 0; c < NV; ++c) ud[c] = (double)un[c];
+      const double sp = cfl_speed<ND>(k, ud);
+      smax = sp > smax ? sp : smax;
     }
   };
   R fh[NV];         // flux of face m - 1, held for the finish at face m
@@ -772,15 +869,15 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
   bool dp = false;  // face m - 2 deferred (its flux in fprev)
 #pragma unroll 1
   for (int m = 0; m < nf; ++m) {
-    AccLoads<ND, R, MODE> ld;
-    if (m >= 2) ld.load(G, fx, acc, o + (int64_t)(m - 1) * s);
+    R qc[NV];
+    if (m >= 2) load_state<ND, R>(acc, G.plane, o + (int64_t)(m - 1) * s, qc);
     if (m + 1 < nf) load_state<ND, R>(cells, G.plane, o + (m + 3) * s, nx);
     get(m, um);
     get(m + 1, u0);
     get(m + 2, up);
     half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
     if (m >= 2) {  // cell f0 + m - 1 (its ring slot is overwritten by the put)
-      finish(m - 1, fh, ld, dp || dh);
+      finish(m - 1, fh, qc, dp || dh);
       dp = dh;
     }
     if (m + 1 < nf) put(m + 3, nx);
@@ -801,9 +898,9 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
       dh = dm;
   }
   {  // the last cell, f0 + nf - 1 (faces nf - 2 and nf - 1; nf >= 2)
-    AccLoads<ND, R, MODE> ld;
-    ld.load(G, fx, acc, o + (int64_t)(nf - 1) * s);
-    finish(nf - 1, fh, ld, dp || dh);
+    R qc[NV];
+    load_state<ND, R>(acc, G.plane, o + (int64_t)(nf - 1) * s, qc);
+    finish(nf - 1, fh, qc, dp || dh);
   }
   return smax;
 }
@@ -816,15 +913,13 @@ __host__ __device__ inline int64_t acc_threads(const Geom& G, int A, int L) {
   return n;
 }
 
-template <int ND, int A, int LIM, typename R, class PW, int MODE>
+template <int LIM, typename R, class PW>
 __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void acc_walk_kernel(
-    Consts k, Geom G, const R* __restrict__ cells, const R* __restrict__ fx,
-    const R* __restrict__ acc, R* __restrict__ out, const double* __restrict__ sc,
-    int L, int order, DeferList dl, double* __restrict__ partial) {
+    Consts k, Geom G, const R* __restrict__ cells, const R* __restrict__ acc, R* __restrict__ out,
+    const double* __restrict__ sc, int L, int order, DeferList dl, double* __restrict__ partial) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const double sp = flux_walk_acc<ND, A, LIM, R, PW, MODE>(k, G, cells, fx, acc, out, sc, L,
-                                                          order, t, dl);
-  if constexpr (MODE == kAccLast) block_max_to_partial(sp, partial);
+  block_max_to_partial(flux_walk_acc<LIM, R, PW>(k, G, cells, acc, out, sc, L, order, t, dl),
+                       partial);
 }
 
 // One face's flux from scratch: the half steps of its two cells (the
@@ -924,37 +1019,57 @@ __global__ __launch_bounds__(256) void flux_fixup_kernel(Consts k, Geom G,
   }
 }
 
-// The cells an accumulating walk along A left beside deferred faces,
-// recomputed with the full policy PW: both faces of each such cell from
-// scratch, then the walk's own accumulation (acc_cell); kAccLast also
-// folds the CFL speed into *slot (an extra
-// partial slot the dt reduction reads; speeds are >= 0, so their bit
-// patterns order as integers).  If the list overflowed, every cell of the
-// box.  Cells listed twice (two deferred faces) are written twice with the
-// same values.
-template <int ND, int A, typename R, class PW, int MODE>
+// The cells an accumulating walk left beside deferred faces, recomputed with
+// the full policy PW: the walk's faces of each such cell from scratch (x and
+// y, or z), then its own accumulation; where the walk writes the new state
+// (WALK kFixXy2, kFixZ) the CFL speed goes into *slot (an extra partial slot
+// the dt reduction reads; speeds are >= 0, so their bit patterns order as
+// integers).  If the list overflowed, every cell of the box.  Cells listed
+// twice (two deferred faces) are written twice with the same values.
+constexpr int kFixXy3 = 0, kFixXy2 = 1, kFixZ = 2;
+
+template <int WALK, typename R, class PW>
 __device__ __forceinline__ void acc_fix_cell(const Consts& k, const Geom& G,
                                              const R* __restrict__ cells,
-                                             const R* __restrict__ fx, const R* __restrict__ acc,
-                                             R* __restrict__ out, double dt,
-                                             double dx0, double dxA, int order, int64_t oc,
-                                             double* slot) {
-  constexpr int NV = ND + 2;
-  int ci[3];
+                                             const R* __restrict__ acc, R* __restrict__ out,
+                                             double dt, double dx0, double dx1, double dx2,
+                                             int order, int64_t oc, double* slot) {
+  constexpr int ND = WALK == kFixXy2 ? 2 : 3, NV = ND + 2;
   int64_t rem = oc;
+  bool inside = true;
 #pragma unroll
   for (int d = 2; d >= 0; --d) {
-    ci[d] = (int)(rem / G.s[d]) - G.g[d] + 1;
-    rem -= (int64_t)(ci[d] - 1 + G.g[d]) * G.s[d];
+    const int ci = (int)(rem / G.s[d]) - G.g[d] + 1;
+    rem -= (int64_t)(ci - 1 + G.g[d]) * G.s[d];
+    inside = inside && ci >= 1 && ci <= G.n[d];
   }
-  if (ci[A] < 1 || ci[A] > G.n[A]) return;
+  if (!inside) return;
   R fl[NV], fu[NV], uc[NV], un[NV];
-  face_flux<ND, A, R, PW>(k, G, cells, dt, dxA, oc - G.s[A], fl);
-  face_flux<ND, A, R, PW>(k, G, cells, dt, dxA, oc, fu);
   load_state<ND, R>(cells, G.plane, oc, uc);
-  acc_cell<ND, A, R, MODE>(G, fx, acc, out, oc, uc, fl, fu, (R)(dt / dx0), (R)(dt / dxA),
-                           order, un);
-  if constexpr (MODE == kAccLast) {
+  if constexpr (WALK == kFixZ) {
+    face_flux<3, 2, R, PW>(k, G, cells, dt, dx2, oc - G.s[2], fl);
+    face_flux<3, 2, R, PW>(k, G, cells, dt, dx2, oc, fu);
+    const R dtdx2 = (R)(dt / dx2);
+#pragma unroll
+    for (int c = 0; c < NV; ++c)
+      un[c] = acc_z<R>(uc[c], acc[oc + c * G.plane], dtdx2 * (fl[c] - fu[c]), order);
+  } else {
+    R a0[NV];
+    face_flux<ND, 0, R, PW>(k, G, cells, dt, dx0, oc - G.s[0], fl);
+    face_flux<ND, 0, R, PW>(k, G, cells, dt, dx0, oc, fu);
+    const R dtdx0 = (R)(dt / dx0), dtdx1 = (R)(dt / dx1);
+#pragma unroll
+    for (int c = 0; c < NV; ++c) a0[c] = dtdx0 * (fl[c] - fu[c]);
+    face_flux<ND, 1, R, PW>(k, G, cells, dt, dx1, oc - G.s[1], fl);
+    face_flux<ND, 1, R, PW>(k, G, cells, dt, dx1, oc, fu);
+#pragma unroll
+    for (int c = 0; c < NV; ++c)
+      un[c] = acc_xy<R, WALK == kFixXy3 ? kAccMid : kAccLast>(uc[c], a0[c],
+                                                              dtdx1 * (fl[c] - fu[c]), order);
+  }
+#pragma unroll
+  for (int c = 0; c < NV; ++c) out[oc + c * G.plane] = un[c];
+  if constexpr (WALK != kFixXy3) {
     double ud[NV];
 #pragma unroll
     for (int c = 0; c < NV; ++c) ud[c] = (double)un[c];
@@ -965,33 +1080,29 @@ __device__ __forceinline__ void acc_fix_cell(const Consts& k, const Geom& G,
   }
 }
 
-template <int ND, int A, typename R, class PW, int MODE>
+template <int WALK, typename R, class PW>
 __global__ __launch_bounds__(256) void acc_fixup_kernel(
-    Consts k, Geom G, const R* __restrict__ cells, const R* __restrict__ fx,
-    const R* __restrict__ acc, R* __restrict__ out, const double* __restrict__ dtp,
-    double dx0, double dxA, int order, DeferList dl, double* slot) {
+    Consts k, Geom G, const R* __restrict__ cells, const R* __restrict__ acc, R* __restrict__ out,
+    const double* __restrict__ dtp, double dx0, double dx1, double dx2, int order, DeferList dl,
+    double* slot) {
   const uint32_t n = *dl.count;
   if (n == 0) return;
   const double dt = *dtp;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n <= dl.cap) {
-    for (int64_t i = t0; i < (int64_t)n; i += stride) {
-      const int64_t of = (int64_t)(dl.items[i] & ((1ull << 40) - 1));
-      acc_fix_cell<ND, A, R, PW, MODE>(k, G, cells, fx, acc, out, dt, dx0, dxA, order, of,
-                                       slot);
-      acc_fix_cell<ND, A, R, PW, MODE>(k, G, cells, fx, acc, out, dt, dx0, dxA, order,
-                                       of + G.s[A], slot);
-    }
-    return;
-  }
   const int64_t total = (int64_t)G.n[0] * G.n[1] * G.n[2];
-  for (int64_t q = t0; q < total; q += stride) {
-    const int i = (int)(q % G.n[0]) + 1;
-    const int64_t r = q / G.n[0];
-    acc_fix_cell<ND, A, R, PW, MODE>(k, G, cells, fx, acc, out, dt, dx0, dxA, order,
-                                     goff(G, i, (int)(r % G.n[1]) + 1, (int)(r / G.n[1]) + 1),
-                                     slot);
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const bool listed = n <= dl.cap;
+  // the list's faces name two cells each; past its capacity, every cell
+  const int64_t work = listed ? 2 * (int64_t)n : total;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < work; i += stride) {
+    int64_t oc;
+    if (listed) {
+      const uint64_t it = dl.items[i >> 1];
+      oc = (int64_t)(it & ((1ull << 40) - 1)) + ((i & 1) ? G.s[(it >> 40) & 3] : 0);
+    } else {
+      const int64_t r = i / G.n[0];
+      oc = goff(G, (int)(i % G.n[0]) + 1, (int)(r % G.n[1]) + 1, (int)(r / G.n[1]) + 1);
+    }
+    acc_fix_cell<WALK, R, PW>(k, G, cells, acc, out, dt, dx0, dx1, dx2, order, oc, slot);
   }
 }
 
