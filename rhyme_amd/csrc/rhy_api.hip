@@ -84,7 +84,8 @@ struct rhy_box {
   double* partial = nullptr;      // per-block CFL maxima of the last reduction
   int32_t partial_n = 0;          // partials of the stand-alone CFL pass
   int32_t acc_blocks = 0;         // partials of the last accumulating walk
-  int32_t nf_x = 8, xy_L = 16, acc_L = 16;  // walk lengths for this shape (alloc_box_memory)
+  int32_t nf[3] = {8, 8, 8};      // walk lengths for this shape (choose_walks): the
+  int32_t xy_L = 16, acc_L = 16;  // flux walks', walk_xy's and the z walk's
   int32_t partial_cap = 0;
   double* scalars = nullptr;      // [0] max_u, [16..16+6*RHY_MAX_CMP) inflow states
   double inflow_copied[6 * RHY_MAX_CMP] = {};  // what the device inflow slots hold
@@ -187,32 +188,6 @@ void collect_timings(rhy_box* b) {
   b->pending.clear();
 }
 
-// Steps of 64 row cells per wave along x (the wave-cooperative walk) and
-// faces walked per thread along y and z (lanes consecutive in x).
-#ifndef RHY_NF_X
-#define RHY_NF_X 8
-#endif
-#ifndef RHY_NF_YZ
-#define RHY_NF_YZ 8
-#endif
-constexpr int kNfX = RHY_NF_X;
-constexpr int kNfYZ = RHY_NF_YZ;
-
-// Cells walked per thread by the accumulating y/z walks of rhy_run.
-#ifndef RHY_ACC_L
-#define RHY_ACC_L 16
-#endif
-constexpr int kAccL = RHY_ACC_L;
-
-// The walk lengths of a box: kNfX steps per x wave and kAccL cells per y/z
-// chunk, halved (down to 2 and 4) while a walk would have fewer waves than
-// fill the chip a few times over (256 CUs x 4 SIMDs x 3 waves = 3072 at a
-// time).  Longer walks repeat less work (a warm-up half step per x wave,
-// one extra face per chunk); more waves hide more latency.  Measured on
-// the 2D 1024^2 spheres: 8 / 16 -> 2 / 4 took 3.2e9 to 4.9e9 zone-updates/s
-// (FP64); at 3D 256^3 the longest lengths already give 33k and 16k waves.
-constexpr int64_t kMinWavesX = 8192, kMinWavesAcc = 4096;
-
 // Faces of axis a a step solves (faces 0..n_a along a, interior across).
 int64_t axis_faces(const Geom& G, int a) {
   int64_t n = (int64_t)G.n[a] + 1;
@@ -221,6 +196,18 @@ int64_t axis_faces(const Geom& G, int a) {
   return n;
 }
 
+
+// The walk lengths of a box's shape (walk_length).
+void choose_walks(rhy_box* b) {
+  const Geom& G = b->geom;
+  for (int a = 0; a < b->ndim; ++a)
+    b->nf[a] = walk_length(a == 0 ? 8 : G.n[a] + 1, 0.7,
+                           [&](int L) { return flux_threads(G, a, L) / 64; });
+  if (b->ndim > 1)
+    b->xy_L = walk_length(G.n[1], 1.0, [&](int L) { return xy_threads(G, L) / 64; });
+  if (b->ndim > 2)
+    b->acc_L = walk_length(G.n[2], 1.0, [&](int L) { return acc_threads(G, 2, L) / 64; });
+}
 
 DeferList defer_list(rhy_box* b) {
   DeferList dl;
@@ -234,7 +221,7 @@ DeferList defer_list(rhy_box* b) {
 template <int ND, int A, int LIM, typename R, class PW>
 void launch_flux_axis(rhy_box* b, const Consts& k, const double* dx, const DeferList& dl) {
   const Geom& G = b->geom;
-  const int nf = A == 0 ? b->nf_x : kNfYZ;
+  const int nf = b->nf[A];
   const int64_t nthreads = flux_threads(G, A, nf);
   R* F = static_cast<R*>(b->flux) + (int64_t)A * (ND + 2) * G.plane;
   TimedLaunch tl;
@@ -580,13 +567,7 @@ int alloc_box_memory(rhy_box* b) {
   }
   const int64_t ncell = (int64_t)b->geom.n[0] * b->geom.n[1] * b->geom.n[2];
   b->partial_n = (int32_t)grid_for(ncell);
-  b->nf_x = kNfX;
-  while (b->nf_x > 2 && flux_threads(b->geom, 0, b->nf_x) / 64 < kMinWavesX) b->nf_x /= 2;
-  b->xy_L = b->acc_L = kAccL;
-  while (b->ndim > 1 && b->xy_L > 4 && xy_threads(b->geom, b->xy_L) / 64 < kMinWavesAcc)
-    b->xy_L /= 2;
-  while (b->ndim > 2 && b->acc_L > 4 && acc_threads(b->geom, 2, b->acc_L) / 64 < kMinWavesAcc)
-    b->acc_L /= 2;
+  choose_walks(b);
   b->acc_blocks = b->ndim == 3   ? (int32_t)grid_for(acc_threads(b->geom, 2, b->acc_L))
                   : b->ndim == 2 ? (int32_t)grid_for(xy_threads(b->geom, b->xy_L))
                                  : 0;
@@ -749,7 +730,7 @@ int rhy_box_resize(rhy_box_t* b, const int32_t dims[3]) {
   b->partial = t.partial;
   b->partial_n = t.partial_n;
   b->acc_blocks = t.acc_blocks;
-  b->nf_x = t.nf_x;
+  for (int a = 0; a < 3; ++a) b->nf[a] = t.nf[a];
   b->xy_L = t.xy_L;
   b->acc_L = t.acc_L;
   b->partial_cap = t.partial_cap;
@@ -1272,6 +1253,7 @@ int rhy_mh_solve_noalloc(const rhy_params_t* p, int32_t ndim, const int32_t dims
   const size_t list_bytes = align256(sizeof(uint64_t) * (size_t)b.defer_cap);
   b.defer_count = reinterpret_cast<uint32_t*>(base + flux_bytes + list_bytes);
   b.dt = reinterpret_cast<double*>(base + flux_bytes + list_bytes + 256);
+  choose_walks(&b);
   b.profiling = false;
   rc = mh_solve_enqueue(&b, p, dx, dt);
   b.cells = b.flux = nullptr;  // nothing here is the view's to free

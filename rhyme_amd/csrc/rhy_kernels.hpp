@@ -922,6 +922,33 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void acc_walk_kernel(
                        partial);
 }
 
+// Cells (or faces, or 64-cell steps) a lane walks, of n along the axis:
+// waves(L) waves walk L each at the cost of `extra` more for a wave's start
+// (its first loads, half step and face).  A longer walk repeats less work, a
+// shorter one gives the chip's 1024 SIMDs more waves, of which each holds 3.
+// With w waves per SIMD a wave's step takes max(0.68 + 0.16 (w - 1), w / 3) of
+// what it takes beside two others: the chain of dependent operations of one
+// wave, or the SIMD's issue.  Measured on 1024^2 (walk_xy, FP64, ms per pass
+// of 100 steps): 32 cells 35.5, 16 23.4, 9 14.5, 7 13.4, 6 11.9 (3078 waves),
+// 4 12.6 (4608); on 40 x 33 x 27 one solve takes 114 us with 1 face per lane
+// and 199 us with 8; 256^3 does not care between 6 and 32, where 16 re-reads
+// less than shorter walks and is the limit.
+template <class W>
+inline int walk_length(int n, double extra, W waves) {
+  int best = 1;
+  double best_cost = 0.0;
+  for (int L = 1; L <= 16 && L <= n; ++L) {
+    const double w = (double)waves(L) / 1024.0;
+    const double alone = w > 1.0 ? 0.68 + 0.16 * (w - 1.0) : 0.68;
+    const double cost = (L + extra) * (w / 3.0 > alone ? w / 3.0 : alone);
+    if (L == 1 || cost < best_cost) {
+      best = L;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 // One face's flux from scratch: the half steps of its two cells (the
 // stencil of four cells along A) and the Riemann solve with policy PW, the
 // computation the flux walks make for it.  of: offset of the low cell.
