@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librhyme_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["rhy_api.hip", "rhy_batch.hip"]
+SOURCES = ["rhy_api.hip", "rhy_batch.hip", "rhy_transfer.hip"]
 
 FLAGS = [
     "--offload-arch=gfx950",

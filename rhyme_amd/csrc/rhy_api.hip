@@ -14,6 +14,7 @@
 
 #include "../../include/rhyme_hip.h"
 #include "rhy_kernels.hpp"
+#include "rhy_transfer.hpp"
 
 using namespace rhy;
 
@@ -677,11 +678,13 @@ int rhy_box_create(int32_t ndim, const int32_t dims[3], int32_t ncmp, int32_t pr
   if (precision != RHY_FP64 && precision != RHY_MIXED)
     return fail(RHY_ERR_ARG, "unsupported precision");
   rhy_box* b = new rhy_box();
+  transfer_user_add();
   b->ndim = ndim;
   for (int d = 0; d < 3; ++d) b->dims[d] = dims[d];
   b->ncmp = ncmp;
   b->precision = precision;
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) {
+    transfer_user_drop();
     delete b;
     return fail(RHY_ERR_HIP, "stream creation failed");
   }
@@ -756,6 +759,7 @@ int rhy_box_destroy(rhy_box_t* b) {
   if (b->diag) (void)hipFree(b->diag);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
+  transfer_user_drop();
   return RHY_OK;
 }
 
@@ -766,37 +770,14 @@ namespace {
 // Host array (ncmp planes, hydro first) to or from the box's current hydro
 // buffer and its other-component planes.
 int box_copy(rhy_box* b, const double* in, double* out) {
-  const size_t P = (size_t)b->geom.plane;
   const size_t nv = (size_t)(b->ndim + 2);
-  const size_t n = P * b->ncmp;
-  const size_t nh = P * nv;
-  const hipMemcpyKind kind = in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
-  auto copy = [&](void* host, size_t esz) -> int {
-    unsigned char* h = static_cast<unsigned char*>(host);
-    void* dh = b->cells;
-    void* dx = b->extra;
-    if (in) {
-      HIP_TRY(hipMemcpyAsync(dh, h, esz * nh, kind, b->stream));
-      if (n > nh) HIP_TRY(hipMemcpyAsync(dx, h + esz * nh, esz * (n - nh), kind, b->stream));
-    } else {
-      HIP_TRY(hipMemcpyAsync(h, dh, esz * nh, kind, b->stream));
-      if (n > nh) HIP_TRY(hipMemcpyAsync(h + esz * nh, dx, esz * (n - nh), kind, b->stream));
-    }
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    return RHY_OK;
-  };
-  if (b->precision == RHY_MIXED) {
-    std::vector<float> tmp(n);
-    if (in) {
-      for (size_t i = 0; i < n; ++i) tmp[i] = (float)in[i];
-      return copy(tmp.data(), sizeof(float));
-    }
-    int rc = copy(tmp.data(), sizeof(float));
-    if (rc) return rc;
-    for (size_t i = 0; i < n; ++i) out[i] = (double)tmp[i];
-    return RHY_OK;
-  }
-  return copy(in ? const_cast<double*>(in) : out, sizeof(double));
+  const size_t n = (size_t)b->geom.plane * b->ncmp;
+  const size_t nh = (size_t)b->geom.plane * nv;
+  double* h = in ? const_cast<double*>(in) : out;
+  const HostSpan spans[2] = {{b->cells, h, nh}, {b->extra, h + nh, n - nh}};
+  HIP_TRY(copy_spans(b->stream, spans, n > nh ? 2 : 1, b->esz, b->precision == RHY_MIXED,
+                     in == nullptr));
+  return RHY_OK;
 }
 
 }  // namespace
@@ -869,8 +850,9 @@ static int box_snapshot(rhy_box_t* b, float* out, const float* in) {
     return fail(RHY_ERR_OOM, "snapshot staging allocation failed");
   }
   const dim3 grid = snapshot_grid(b->geom);
+  const HostSpan span = {b->snap, in ? const_cast<float*>(in) : out, bytes / sizeof(float)};
   if (in) {
-    HIP_TRY(hipMemcpyAsync(b->snap, in, bytes, hipMemcpyHostToDevice, b->stream));
+    HIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, false));
     if (b->precision == RHY_MIXED)
       hipLaunchKernelGGL(snapshot_unpack_kernel<float>, grid, dim3(kThreads), 0, b->stream,
                          b->geom, b->ncmp, b->ndim + 2, static_cast<float*>(b->cells),
@@ -890,7 +872,8 @@ static int box_snapshot(rhy_box_t* b, float* out, const float* in) {
                          b->geom, b->ncmp, b->ndim + 2, static_cast<const double*>(b->cells),
                          static_cast<const double*>(b->extra), b->snap);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(out, b->snap, bytes, hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, true));
+    return RHY_OK;
   }
   HIP_TRY(hipStreamSynchronize(b->stream));
   return RHY_OK;

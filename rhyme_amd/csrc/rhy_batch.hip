@@ -26,6 +26,7 @@
 
 #include "../../include/rhyme_hip.h"
 #include "rhy_kernels.hpp"
+#include "rhy_transfer.hpp"
 
 using namespace rhy;
 
@@ -1045,6 +1046,7 @@ rhy_batch* new_batch(int32_t ndim, int32_t ncmp, int32_t precision, int64_t aren
     return nullptr;
   }
   rhy_batch* b = new rhy_batch();
+  transfer_user_add();
   b->ndim = ndim;
   b->ncmp = ncmp;
   b->precision = precision;
@@ -1091,6 +1093,12 @@ void launch_paint(rhy_batch* b, const Geom& G, const PaintIC& ic, int64_t off) {
                        static_cast<double*>(b->arena) + xo);
 }
 
+// n values of the arena from element off on, and the caller's doubles.
+hipError_t copy_state(rhy_batch* b, int64_t off, int64_t n, double* host, bool to_host) {
+  const HostSpan span = {static_cast<char*>(b->arena) + off * (int64_t)b->esz, host, (size_t)n};
+  return copy_spans(b->stream, &span, 1, b->esz, b->precision == RHY_MIXED, to_host);
+}
+
 // Place a box: its state from host `cells`, painted from `ic`, or zero.
 int add_box(rhy_batch* b, const int32_t* dims, const double* dx, const double* cells,
             const PaintIC* ic, int32_t limiter, const int32_t* bc_types, int32_t* slot_out) {
@@ -1112,18 +1120,7 @@ int add_box(rhy_batch* b, const int32_t* dims, const double* dx, const double* c
   // the state first; the slot becomes active only once it is written
   hipError_t e = hipSuccess;
   if (cells) {
-    const size_t n = (size_t)G.plane * b->ncmp;
-    if (b->precision == RHY_MIXED) {
-      std::vector<float> tmp(n);
-      for (size_t i = 0; i < n; ++i) tmp[i] = (float)cells[i];
-      e = hipMemcpyAsync(static_cast<float*>(b->arena) + off, tmp.data(), sizeof(float) * n,
-                         hipMemcpyHostToDevice, b->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    } else {
-      e = hipMemcpyAsync(static_cast<double*>(b->arena) + off, cells, sizeof(double) * n,
-                         hipMemcpyHostToDevice, b->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    }
+    e = copy_state(b, off, (int64_t)G.plane * b->ncmp, const_cast<double*>(cells), false);
   } else if (ic) {
     if (b->ndim == 1) launch_paint<1>(b, G, *ic, off);
     else if (b->ndim == 2) launch_paint<2>(b, G, *ic, off);
@@ -1273,6 +1270,7 @@ int rhy_batch_destroy(rhy_batch_t* b) {
     if (p) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
+  transfer_user_drop();
   return RHY_OK;
 }
 
@@ -1291,18 +1289,7 @@ int rhy_batch_upload(rhy_batch_t* b, int32_t box, const double* cells) {
   const BBox& B = b->slots[box].B;
   b->slots[box].needs_bc = true;
   b->partials_valid = false;
-  const size_t n = (size_t)B.G.plane * b->ncmp;
-  if (b->precision == RHY_MIXED) {
-    std::vector<float> tmp(n);
-    for (size_t i = 0; i < n; ++i) tmp[i] = (float)cells[i];
-    BHIP_TRY(hipMemcpyAsync(static_cast<float*>(b->arena) + B.cell_off, tmp.data(),
-                            sizeof(float) * n, hipMemcpyHostToDevice, b->stream));
-    BHIP_TRY(hipStreamSynchronize(b->stream));
-    return RHY_OK;
-  }
-  BHIP_TRY(hipMemcpyAsync(static_cast<double*>(b->arena) + B.cell_off, cells,
-                          sizeof(double) * n, hipMemcpyHostToDevice, b->stream));
-  BHIP_TRY(hipStreamSynchronize(b->stream));
+  BHIP_TRY(copy_state(b, B.cell_off, B.G.plane * b->ncmp, const_cast<double*>(cells), false));
   return RHY_OK;
 }
 
@@ -1336,9 +1323,8 @@ static int batch_snapshot(rhy_batch_t* b, float* out, const float* in) {
     }
     b->snap_elems = total;
   }
-  if (in)
-    BHIP_TRY(hipMemcpyAsync(b->snap, in, sizeof(float) * (size_t)total, hipMemcpyHostToDevice,
-                            b->stream));
+  const HostSpan span = {b->snap, in ? const_cast<float*>(in) : out, (size_t)total};
+  if (in) BHIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, false));
   int64_t ofs = 0;
   for (Slot& S : b->slots) {
     if (!S.active) continue;
@@ -1371,9 +1357,7 @@ static int batch_snapshot(rhy_batch_t* b, float* out, const float* in) {
   }
   BHIP_TRY(hipGetLastError());
   if (in) b->partials_valid = false;
-  if (out)
-    BHIP_TRY(hipMemcpyAsync(out, b->snap, sizeof(float) * (size_t)total, hipMemcpyDeviceToHost,
-                            b->stream));
+  if (out) BHIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, true));
   BHIP_TRY(hipStreamSynchronize(b->stream));
   return RHY_OK;
 }
@@ -1393,18 +1377,7 @@ int rhy_batch_snapshot_unpack(rhy_batch_t* b, const float* data) {
 int rhy_batch_download(rhy_batch_t* b, int32_t box, double* cells) {
   if (!slot_ok(b, box) || !cells) return bfail(RHY_ERR_ARG, "bad download");
   const BBox& B = b->slots[box].B;
-  const size_t n = (size_t)B.G.plane * b->ncmp;
-  if (b->precision == RHY_MIXED) {
-    std::vector<float> tmp(n);
-    BHIP_TRY(hipMemcpyAsync(tmp.data(), static_cast<float*>(b->arena) + B.cell_off,
-                            sizeof(float) * n, hipMemcpyDeviceToHost, b->stream));
-    BHIP_TRY(hipStreamSynchronize(b->stream));
-    for (size_t i = 0; i < n; ++i) cells[i] = (double)tmp[i];
-    return RHY_OK;
-  }
-  BHIP_TRY(hipMemcpyAsync(cells, static_cast<double*>(b->arena) + B.cell_off,
-                          sizeof(double) * n, hipMemcpyDeviceToHost, b->stream));
-  BHIP_TRY(hipStreamSynchronize(b->stream));
+  BHIP_TRY(copy_state(b, B.cell_off, B.G.plane * b->ncmp, cells, true));
   return RHY_OK;
 }
 
