@@ -479,8 +479,38 @@ int launch_acc_step(rhy_box* b, const Consts& k, const double* dx,
   return RHY_OK;
 }
 
-// The main loop's steps (src/main.f90:109-136) on the device.  1D boxes:
-// fluxes into planes, then the update with the fused epilogue (ghost
+// nsteps steps of a small 1D box by tube_run_kernel, its ghosts filled.
+// (A launch takes at most 4096 steps, some 30 ms.)
+template <typename R, class PW, class P>
+void launch_tube_r(rhy_box* b, const Consts& k, const BcTypes& bc, double dx, double cmdx,
+                   int nsteps, int threads) {
+  for (int s = 0; s < nsteps; s += 4096) {
+    const int m = std::min(nsteps - s, 4096);
+#define RHY_TUBE(L)                                                                          \
+  hipLaunchKernelGGL((tube_run_kernel<L, R, PW, P>), dim3(1), dim3(threads), 0, b->stream, k, \
+                     b->geom, bc, static_cast<R*>(b->cells), cmdx, dx, m, b->dt, b->dt_log + s, \
+                     b->defer_count)
+    switch (k.limiter) {
+      case 1: RHY_TUBE(1); break;
+      case 2: RHY_TUBE(2); break;
+      case 3: RHY_TUBE(3); break;
+      default: RHY_TUBE(4); break;
+    }
+#undef RHY_TUBE
+  }
+}
+
+void launch_tube(rhy_box* b, const Consts& k, const BcTypes& bc, double dx, double cmdx,
+                 int nsteps, int threads) {
+  if (b->precision == RHY_MIXED)
+    launch_tube_r<float, MixedTube, MixedMath>(b, k, bc, dx, cmdx, nsteps, threads);
+  else
+    launch_tube_r<double, PowF64Tube, PowF64Fix>(b, k, bc, dx, cmdx, nsteps, threads);
+}
+
+// The main loop's steps (src/main.f90:109-136) on the device.  Small 1D
+// boxes: all of them in one launch (tube_run_kernel; not while launches are
+// timed, which name the phases of a step).  Other 1D boxes: fluxes into planes, then the update with the fused epilogue (ghost
 // images and CFL partials of the new state).  2D/3D boxes: the
 // accumulating walks, whose last one writes the new state's interior and
 // CFL partials into the other state buffer (the buffers swap every step),
@@ -493,10 +523,18 @@ int run_steps(rhy_box* b, const rhy_params_t* p, const double* dx, int32_t nstep
   const BcTypes bc = make_bc(p);
   int rc;
   if ((rc = ensure_dt_log(b, nsteps > 0 ? nsteps : 1))) return rc;
+  const double cmdx = p->courant * min_dx(ND, dx);
+  const int tube = ND == 1 && b->prof_every == 0 ? tube_threads(b->geom.n[0]) : 0;
+  if (tube > 0) {
+    if ((rc = launch_bc<ND>(b, p, -1))) return rc;
+    launch_tube(b, k, bc, dx[0], cmdx, nsteps, tube);
+    b->last_nsteps = nsteps;
+    HIP_TRY(hipGetLastError());
+    return RHY_OK;
+  }
   // prologue: CFL of the current state and the ghost fill it is stepped with
   if ((rc = launch_cfl<ND>(b, k))) return rc;
   if ((rc = launch_bc<ND>(b, p, -1))) return rc;
-  const double cmdx = p->courant * min_dx(ND, dx);
   for (int32_t s = 0; s < nsteps; ++s) {
     if (b->prof_every > 1) b->profiling = s % b->prof_every == 0;
     // partials: the CFL pass's before the first step, the last walk's and

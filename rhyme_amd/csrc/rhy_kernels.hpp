@@ -179,7 +179,7 @@ template <class PW>
 __device__ __forceinline__ bool defer_take(const Consts& k, const DeferList& dl, uint32_t box,
                                            int axis, int64_t of) {
   if constexpr (PW::kDefer) {
-    uint32_t& f = defer_flag();
+    uint32_t& f = PW::flag();
     if (k.defer_every > 0 && of % k.defer_every == 0) f = 1u;
     if (f) {
       f = 0u;
@@ -193,7 +193,7 @@ __device__ __forceinline__ bool defer_take(const Consts& k, const DeferList& dl,
 
 template <class PW>
 __device__ __forceinline__ void defer_clear() {
-  if constexpr (PW::kDefer) defer_flag() = 0u;
+  if constexpr (PW::kDefer) PW::flag() = 0u;
 }
 
 // Writes the ghost images of an updated interior cell, i.e. what
@@ -1131,6 +1131,134 @@ __global__ __launch_bounds__(256) void acc_fixup_kernel(
     }
     acc_fix_cell<WALK, R, PW>(k, G, cells, acc, out, dt, dx0, dx1, dx2, order, oc, slot);
   }
+}
+
+// tube_run: nsteps steps of a small 1D box in one workgroup and one launch,
+// its state in LDS: a step through kernels of its own (the fluxes, their
+// fixup, the update, dt and a reset) is 20.5 us whatever its cells, most of
+// it launches and first loads; here it is 5.5 us at 64 cells, 8.7 at 766,
+// 12.4 at 1024 and 15.3 at 2040, the chain of dependent operations of one
+// half step and one Riemann solve for each round of cells.  A thread takes every blockDim-th cell; the
+// right half states of a strip of cells lie in `rf` for the cells above, and
+// a face's flux takes the slot of the half state that only it reads.  A face
+// that needs the policy's slow paths is solved again with P on the spot.
+// The arithmetic and its order are flux_xrows', update_kernel's and
+// dt_kernel's.
+constexpr int kTubeLanes = 768;  // 3 waves per SIMD: 168 VGPRs
+constexpr int kTubeCells = 2040;  // 4 rounds would be 19 us of the 20.5
+using PowF64Tube = typename WithLanes<PowF64Flux, kTubeLanes>::type;
+using MixedTube = typename WithLanes<MixedFlux, kTubeLanes>::type;
+
+template <int LIM, typename R, class PW, class P>
+__global__ __launch_bounds__(kTubeLanes) RHY_FLUX_OCCUPANCY void tube_run_kernel(
+    Consts k, Geom G, BcTypes bc, R* __restrict__ cells, double cmdx, double dx, int nsteps,
+    double* __restrict__ dt_out, double* __restrict__ dt_log, uint32_t* __restrict__ defer_count) {
+  constexpr int NV = 3;
+  __shared__ R u[NV * (kTubeCells + 4)];   // cells with ghosts, plane G.plane
+  __shared__ R rf[NV * (kTubeCells + 4)];  // right half states, then fluxes
+  __shared__ double wave_max[kTubeLanes / 64];
+  __shared__ uint32_t deferred;
+  const int n = G.n[0], P1 = n + 4;  // cell c (0..n+1) in slot c + 1
+  const int tid = (int)threadIdx.x, T = (int)blockDim.x;
+  for (int i = tid; i < P1; i += T)
+#pragma unroll
+    for (int c = 0; c < NV; ++c) u[c * P1 + i] = cells[c * G.plane + i];
+  if (tid == 0) deferred = 0u;
+  defer_clear<PW>();
+  double speed = 0.0;
+  auto speed_of = [&](const R* w) {
+    double ud[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) ud[c] = (double)w[c];
+    const double s = cfl_speed<1>(k, ud);
+    speed = s > speed ? s : speed;
+  };
+  __syncthreads();
+  for (int i = tid + 1; i <= n; i += T) {
+    R w[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) w[c] = u[c * P1 + i + 1];
+    speed_of(w);
+  }
+#pragma unroll 1
+  for (int s = 0; s < nsteps; ++s) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const double o = __shfl_xor(speed, off, 64);
+      speed = o > speed ? o : speed;
+    }
+    if ((tid & 63) == 0) wave_max[tid >> 6] = speed;
+    __syncthreads();
+    double m = 0.0;
+    for (int i = 0; i < T >> 6; ++i) m = wave_max[i] > m ? wave_max[i] : m;
+    const double dt = cmdx / m;
+    const R hdtdx = (R)(.5 * dt / dx), dtdx = (R)(dt / dx);
+    if (tid == 0) {
+      dt_log[s] = dt;
+      if (s == nsteps - 1) *dt_out = dt;
+    }
+    speed = 0.0;
+#pragma unroll 1
+    for (int i0 = 0; i0 < n + 2; i0 += T) {  // every thread: the barrier inside
+      const int i = i0 + tid;
+      const bool valid = i < n + 2;
+      R lw[NV];
+      if (valid) {
+        R um[NV], u0[NV], up[NV], rn[NV];
+#pragma unroll
+        for (int c = 0; c < NV; ++c) {
+          um[c] = u[c * P1 + i];
+          u0[c] = u[c * P1 + i + 1];
+          up[c] = u[c * P1 + i + 2];
+        }
+        half_step<1, 0, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+#pragma unroll
+        for (int c = 0; c < NV; ++c) rf[c * P1 + i] = rn[c];
+      }
+      __syncthreads();
+      if (valid && i > 0) {  // face i - 1, between cells i - 1 and i
+        R r[NV], F[NV];
+#pragma unroll
+        for (int c = 0; c < NV; ++c) r[c] = rf[c * P1 + i - 1];
+        riemann_flux<1, 0, PW, R>(k, r, lw, F);
+        if constexpr (PW::kDefer) {
+          uint32_t& f = PW::flag();
+          if (k.defer_every > 0 && i % k.defer_every == 0) f = 1u;  // i: the low cell's offset
+          if (f) {
+            f = 0u;
+            if (s == nsteps - 1) atomicAdd(&deferred, 1u);
+            riemann_flux<1, 0, P, R>(k, r, lw, F);
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < NV; ++c) rf[c * P1 + i - 1] = F[c];
+      }
+    }
+    __syncthreads();
+    for (int i = tid + 1; i <= n; i += T) {
+      R w[NV];
+#pragma unroll
+      for (int c = 0; c < NV; ++c) {
+        w[c] = u[c * P1 + i + 1] + dtdx * (rf[c * P1 + i - 1] - rf[c * P1 + i]);
+        u[c * P1 + i + 1] = w[c];
+      }
+      write_ghost_images<1, R>(G, bc, u, i, 1, 1, w);
+      speed_of(w);
+    }
+    __syncthreads();
+  }
+  for (int i = tid; i < P1; i += T)
+#pragma unroll
+    for (int c = 0; c < NV; ++c) cells[c * G.plane + i] = u[c * P1 + i];
+  if (tid < 4) defer_count[tid] = tid == 0 ? deferred : 0u;
+}
+
+// Threads of tube_run for n cells, 0 for more than it holds: the fewest rounds of at most kTubeLanes cells, evenly filled.
+inline int tube_threads(int n) {
+  if (n > kTubeCells) return 0;
+  const int rounds = (n + 2 + kTubeLanes - 1) / kTubeLanes;
+  const int per = (n + 2 + rounds - 1) / rounds;
+  return (per + 63) / 64 * 64;
 }
 
 // Empties the deferred-face counters of a step (and the extra CFL slot).

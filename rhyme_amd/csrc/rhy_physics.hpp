@@ -548,17 +548,16 @@ using PowF64 = PowLib;
 // for bit, and on every other face Deferring<P> computes what P computes.
 //
 // The flag is one LDS word per lane (a lane only touches its own word), so
-// policies need no state; kernels using it have at most 256 threads per
+// policies need no state; kernels using it have at most LANES threads per
 // workgroup and clear the flag when they start.
-__device__ __forceinline__ uint32_t& defer_flag() {
-  __shared__ uint32_t flags[256];
-  return flags[threadIdx.x];
-}
-__device__ __forceinline__ void defer_mark() { defer_flag() = 1u; }
-
-template <class P>
+template <class P, int LANES = 256>
 struct Deferring : P {
   static constexpr bool kDefer = true;
+  __device__ __forceinline__ static uint32_t& flag() {
+    __shared__ uint32_t flags[LANES];
+    return flags[threadIdx.x];
+  }
+  __device__ __forceinline__ static void defer_mark() { flag() = 1u; }
   __device__ __forceinline__ static double pw(double x, double y) {
     if (!(x > 0.0) || !(x < INFINITY)) {
       defer_mark();
@@ -615,6 +614,11 @@ using PowF64Flux = PowLib;
 using PowF64Fix = PowLib;
 #endif
 using MixedFlux = Deferring<MixedMath>;
+// the same with more lanes to a workgroup
+template <class PW, int LANES>
+struct WithLanes { using type = PW; };
+template <class P, int N, int LANES>
+struct WithLanes<Deferring<P, N>, LANES> { using type = Deferring<P, LANES>; };
 
 // rhyme_irs_nonlinear_wave_function.f90:13-23.  The terms that do not
 // depend on p (A_K, B_K of the shock branch, 2 c_K / (gamma-1) and
@@ -771,7 +775,7 @@ __device__ __forceinline__ double irs_exec(const Consts& k, double lr, double lv
   double p = newton<PW>(k, guess1<PW>(k, lr, lv, lp, lc, rr, rv, rp, rc), L, R, du, lf, rf);
   if (!(p > 0.0)) {
     if constexpr (PW::kDefer) {
-      defer_mark();  // guesses 2-6: the fixup kernel's work
+      PW::defer_mark();  // guesses 2-6: the fixup kernel's work
     } else {
       for (int gi = 1; gi < 6; ++gi) {
         p = newton<PW>(k, guess_n<PW>(k, gi, lr, lv, lp, lc, rr, rv, rp, rc), L, R, du, lf, rf);
@@ -1153,7 +1157,7 @@ __device__ __forceinline__ void riemann_sample(const Consts& k, const double* l,
     }
     if (!ok) {
       if constexpr (PW::kDefer) {
-        defer_mark();
+        PW::defer_mark();
         srho = 1.0;
         sp = 1.0;
 #pragma unroll
