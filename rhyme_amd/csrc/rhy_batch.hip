@@ -60,7 +60,7 @@ struct BBox {
 
 // A tile is one workgroup's share: `count` consecutive threads, starting
 // at `base`, of box `box`'s index space for phase `kind` (0..2: flux along
-// that axis, 3: update).
+// that axis, 3: update, 4: ghosts).
 struct BTile {
   int32_t box;
   int32_t kind;
@@ -71,7 +71,7 @@ struct BTile {
 // A segment is the run of tiles that covers one phase of one box: tiles
 // [start, next segment's start) take blockDim.x consecutive threads each of
 // the `threads` threads of box `box`'s phase `kind`.  Segments are stored in
-// tile order (all flux phases, then the updates), a few per box; a per-tile
+// tile order (all flux phases, then the updates, then the ghosts), a few per box; a per-tile
 // table of segment indices (4 bytes per tile) finds a tile's segment.
 struct BSeg {
   int32_t start;
@@ -103,7 +103,8 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void batch_flux_kernel(Cons
                                                          R* __restrict__ arena,
                                                          const double* __restrict__ dt,
                                                          int32_t nf_x, int32_t nf_yz,
-                                                         DeferList dl) {
+                                                         DeferList dl, int32_t* __restrict__ step) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *step = *step + 1;  // dt has been logged
   for (int32_t ti = blockIdx.x; ti < ntiles; ti += gridDim.x) {
     const BTile T = tile_of(segs, tile_seg, ti);
     if ((int32_t)threadIdx.x >= T.count) continue;
@@ -259,16 +260,59 @@ __global__ __launch_bounds__(256) void batch_cfl_kernel(Consts k, const BBox* __
   }
 }
 
+// Ghost cells of a box's faces, two per thread.
+inline int64_t face_cells(const Geom& G, int ndim) {
+  int64_t n = 0;
+  for (int a = 0; a < ndim; ++a) {
+    int64_t m = 2;
+    for (int d = 0; d < 3; ++d)
+      if (d != a) m *= G.n[d];
+    n += m;
+  }
+  return n;
+}
+
+// Ghost fill of every box.
+template <int ND, typename R>
+__global__ __launch_bounds__(256) void batch_bc_kernel(const BBox* __restrict__ boxes,
+                                                       const BSeg* __restrict__ segs,
+                                                       const int32_t* __restrict__ tile_seg,
+                                                       int32_t first, int32_t ntiles,
+                                                       R* __restrict__ arena,
+                                                       const double* __restrict__ inflow,
+                                                       int32_t ncmp) {
+  for (int32_t ti = first + blockIdx.x; ti < first + ntiles; ti += gridDim.x) {
+    const BTile T = tile_of(segs, tile_seg, ti);
+    if ((int32_t)threadIdx.x >= T.count) continue;
+    const BBox& B = boxes[T.box];
+    int64_t t = T.base + threadIdx.x;
+    int face = 0;
+    for (;; ++face) {
+      int64_t m = 1;
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+        if (d != face / 2) m *= B.G.n[d];
+      if (t < m) break;
+      t -= m;
+    }
+    R* c = arena + B.cell_off;
+    bc_face_cell<ND, R>(B.G, B.bc, inflow, ncmp, c, c + (int64_t)(ND + 2) * B.G.plane, face, t);
+  }
+}
+
 // dt of every active box (block b reduces the partials of box active[b]);
 // logs it at dtlog[*step * log_stride + box] while the step counter is
-// below the log size.
+// below the log size.  Also empties the step's deferred-face list (the flux
+// phase counts the step itself: launches of their own for the two were 8 us
+// of a step).
 __global__ __launch_bounds__(256) void batch_dt_kernel(const BBox* __restrict__ boxes,
                                                        const int32_t* __restrict__ active,
                                                        const double* __restrict__ partial,
                                                        double* __restrict__ dt,
                                                        double* __restrict__ dtlog,
                                                        const int32_t* __restrict__ step,
-                                                       int32_t log_steps, int32_t log_stride) {
+                                                       int32_t log_steps, int32_t log_stride,
+                                                       uint32_t* __restrict__ defer_count) {
   __shared__ double wave_max[4];
   const int b = active[blockIdx.x];
   const BBox& B = boxes[b];
@@ -287,11 +331,8 @@ __global__ __launch_bounds__(256) void batch_dt_kernel(const BBox* __restrict__ 
     dt[b] = d;
     const int32_t s = *step;
     if (dtlog && s < log_steps) dtlog[(int64_t)s * log_stride + b] = d;
+    if (defer_count && blockIdx.x == 0) *defer_count = 0u;
   }
-}
-
-__global__ void batch_step_counter_kernel(int32_t* step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step = *step + 1;
 }
 
 __global__ void batch_set_counter_kernel(int32_t* step, int32_t v) {
@@ -305,9 +346,11 @@ __global__ __launch_bounds__(256) void batch_set_dt_kernel(const int32_t* __rest
                                                            double* __restrict__ dt,
                                                            double* __restrict__ dtlog,
                                                            const int32_t* __restrict__ step,
-                                                           int32_t log_steps, int32_t log_stride) {
+                                                           int32_t log_steps, int32_t log_stride,
+                                                           uint32_t* __restrict__ defer_count) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= nactive) return;
+  if (i == 0) *defer_count = 0u;
   const int b = active[i];
   dt[b] = value;
   const int32_t s = *step;
@@ -646,7 +689,7 @@ struct rhy_batch {
   std::map<int64_t, int64_t> free_blocks;  // offset -> length, elements
   int64_t arena_elems = 0;
   std::vector<BSeg> hsegs;
-  int32_t nflux_tiles = 0, nupd_tiles = 0;
+  int32_t nflux_tiles = 0, nupd_tiles = 0, nbc_tiles = 0;
   int32_t block = 256, nf_x = 8, nf_yz = 8, grid_cap = 0;
   bool dirty = true;
   bool partials_valid = false;  // CFL partials match the state and tile table
@@ -784,6 +827,12 @@ int build_tiles(rhy_batch* b) {
     B.part_end = start - b->nflux_tiles;
   }
   b->nupd_tiles = start - b->nflux_tiles;
+  for (int i : b->active) {
+    const int64_t n = face_cells(b->slots[i].B.G, nd);
+    b->hsegs.push_back({start, i, 4, 0, n});
+    start += (int32_t)cdiv(n, b->block);
+  }
+  b->nbc_tiles = start - b->nflux_tiles - b->nupd_tiles;
   int rc;
   std::vector<int32_t> tseg((size_t)std::max(1, start));
   for (size_t i = 0; i < b->hsegs.size(); ++i) {
@@ -838,11 +887,10 @@ void launch_flux_phase(rhy_batch* b, const Consts& k, int lim) {
   const unsigned g = persistent_grid(b, b->nflux_tiles);
   R* a = static_cast<R*>(b->arena);
   const DeferList dl = defer_list(b);
-  hipLaunchKernelGGL(set_u32_kernel, dim3(1), dim3(64), 0, b->stream, b->defer_count, 0u);
 #define RHY_BATCH_FLUX(L)                                                                   \
   hipLaunchKernelGGL((batch_flux_kernel<ND, L, R, PW>), dim3(g), dim3(b->block), 0, b->stream, \
                      k, b->dboxes, b->dsegs, b->dtile_seg, b->nflux_tiles, a, b->dt, \
-                     b->nf_x, b->nf_yz, dl)
+                     b->nf_x, b->nf_yz, dl, b->step)
   switch (lim) {
     case 0: RHY_BATCH_FLUX(0); break;
     case 1: RHY_BATCH_FLUX(1); break;
@@ -876,14 +924,14 @@ void enqueue_step(rhy_batch* b, const Consts& k, int order, int lim, double fixe
   if (fixed_dt > 0.0)
     hipLaunchKernelGGL(batch_set_dt_kernel, dim3(cdiv((int64_t)b->active.size(), 256)), dim3(256),
                        0, b->stream, b->dactive, (int32_t)b->active.size(), fixed_dt, b->dt,
-                       b->dtlog, b->step, b->dtlog_steps, (int32_t)b->slots.size());
+                       b->dtlog, b->step, b->dtlog_steps, (int32_t)b->slots.size(),
+                       b->defer_count);
   else
     hipLaunchKernelGGL(batch_dt_kernel, dim3((unsigned)b->active.size()), dim3(256), 0,
                        b->stream, b->dboxes, b->dactive, b->partial, b->dt, b->dtlog, b->step,
-                       b->dtlog_steps, (int32_t)b->slots.size());
+                       b->dtlog_steps, (int32_t)b->slots.size(), b->defer_count);
   launch_flux_phase<ND, R, PW, P>(b, k, lim);
   launch_update_phase<ND, R>(b, k, order);
-  hipLaunchKernelGGL(batch_step_counter_kernel, dim3(1), dim3(64), 0, b->stream, b->step);
 }
 
 // Ghost fill, then CFL partials of the current state.  A fixed batch fills
@@ -894,22 +942,18 @@ void enqueue_step(rhy_batch* b, const Consts& k, int order, int lim, double fixe
 template <int ND, typename R>
 int prologue(rhy_batch* b, const Consts& k, bool need_partials) {
   R* a = static_cast<R*>(b->arena);
+  // (one launch for all boxes: the fill of one whose ghosts are current changes
+  // nothing, and a launch for each box is 2.7 us, 2.7 of the 38 ms of 40
+  // steps over 8 fine boxes, which are filled before every substep)
+  bool fill = !b->pool;
   for (int i : b->active) {
-    Slot& S = b->slots[i];
-    if (b->pool && !S.needs_bc) continue;
-    S.needs_bc = false;
-    const BBox& B = S.B;
-    int64_t maxface = 1;
-    for (int ax = 0; ax < ND; ++ax) {
-      int64_t m = 1;
-      for (int d = 0; d < 3; ++d)
-        if (d != ax) m *= B.G.n[d];
-      maxface = std::max(maxface, m);
-    }
-    hipLaunchKernelGGL((bc_kernel<ND, R>), dim3(cdiv(maxface, 256), 2 * ND), dim3(256), 0,
-                       b->stream, B.G, B.bc, b->inflow, b->ncmp, a + B.cell_off,
-                       a + B.cell_off + (int64_t)(ND + 2) * B.G.plane, -1);
+    fill = fill || b->slots[i].needs_bc;
+    b->slots[i].needs_bc = false;
   }
+  if (fill)
+    hipLaunchKernelGGL((batch_bc_kernel<ND, R>), dim3(persistent_grid(b, b->nbc_tiles)),
+                       dim3(b->block), 0, b->stream, b->dboxes, b->dsegs, b->dtile_seg,
+                       b->nflux_tiles + b->nupd_tiles, b->nbc_tiles, a, b->inflow, b->ncmp);
   if (need_partials && (!b->pool || !b->partials_valid)) {
     const unsigned g = persistent_grid(b, b->nupd_tiles);
     hipLaunchKernelGGL((batch_cfl_kernel<ND, R>), dim3(g), dim3(b->block), 0, b->stream, k,
@@ -980,7 +1024,7 @@ int run_t(rhy_batch* b, const rhy_params_t* p, int32_t nsteps, int32_t use_graph
   if (mode == 2) {
     hipLaunchKernelGGL(batch_dt_kernel, dim3((unsigned)b->active.size()), dim3(256), 0,
                        b->stream, b->dboxes, b->dactive, b->partial, b->dt, (double*)nullptr,
-                       b->step, 0, (int32_t)b->slots.size());
+                       b->step, 0, (int32_t)b->slots.size(), (uint32_t*)nullptr);
     BHIP_TRY(hipGetLastError());
     return RHY_OK;
   }

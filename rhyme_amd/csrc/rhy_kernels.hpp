@@ -1328,20 +1328,18 @@ __global__ __launch_bounds__(256) void update_kernel(Consts k, Geom G, R* __rest
   if (FUSED) block_max_to_partial(speed, partial);
 }
 
-// Stand-alone ghost fill, one thread per face cell; blockIdx.y = face
-// (rhyme_samr_bc_set_boundaries.f90:9-20 calls the faces in this order; the
-// faces are disjoint and read interior cells only, so they run together).
-template <int ND, typename R = double>
-__global__ __launch_bounds__(256) void bc_kernel(Geom G, BcTypes bc, const double* __restrict__ inflow,
-                                                 int32_t ncmp, R* __restrict__ cells,
-                                                 R* __restrict__ extra, int32_t face_only) {
-  const int face = face_only >= 0 ? face_only : (int)blockIdx.y;
+// Ghost fill of the t-th cell of a face: its two ghost cells
+// (rhyme_samr_bc_set_boundaries.f90:9-20 calls the faces in order; they are
+// disjoint and read interior cells only, so they run together).
+template <int ND, typename R>
+__device__ __forceinline__ void bc_face_cell(const Geom& G, const BcTypes& bc,
+                                             const double* __restrict__ inflow, int32_t ncmp,
+                                             R* __restrict__ cells, R* __restrict__ extra,
+                                             int face, int64_t t) {
   const int a = face / 2, side = face % 2;
-  if (a >= ND) return;
   const int o1 = a == 0 ? 1 : 0;
   const int o2 = a == 2 ? 1 : 2;
   const int n1 = G.n[o1], n2 = G.n[o2];
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)n1 * n2) return;
   int idx[3];
   idx[o1] = (int)(t % n1) + 1;
@@ -1386,6 +1384,17 @@ __global__ __launch_bounds__(256) void bc_kernel(Geom G, BcTypes bc, const doubl
     cells[og0 + c * G.plane] = v0;
     cells[og1 + c * G.plane] = v1;
   }
+}
+
+// Stand-alone ghost fill, one thread per face cell; blockIdx.y = face.
+template <int ND, typename R = double>
+__global__ __launch_bounds__(256) void bc_kernel(Geom G, BcTypes bc, const double* __restrict__ inflow,
+                                                 int32_t ncmp, R* __restrict__ cells,
+                                                 R* __restrict__ extra, int32_t face_only) {
+  const int face = face_only >= 0 ? face_only : (int)blockIdx.y;
+  if (face / 2 >= ND) return;
+  bc_face_cell<ND, R>(G, bc, inflow, ncmp, cells, extra, face,
+                      (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // max over the interior of |v| + c_s (rhyme_cfl_time_step.f90:40-47).
@@ -1495,9 +1504,6 @@ __device__ __forceinline__ double strided_max(const double* __restrict__ p, int6
   }
 }
 
-[[maybe_unused]] static __global__ void set_u32_kernel(uint32_t* dst, uint32_t v) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *dst = v;
-}
 
 // -------------------------------------------------------- diagnostics ----
 
