@@ -205,9 +205,11 @@ void choose_walks(rhy_box* b) {
     b->nf[a] = walk_length(a == 0 ? 8 : G.n[a] + 1, 0.7,
                            [&](int L) { return flux_threads(G, a, L) / 64; });
   if (b->ndim > 1)
-    b->xy_L = walk_length(G.n[1], 1.0, [&](int L) { return xy_threads(G, L) / 64; });
+    b->xy_L = even_length(
+        G.n[1], walk_length(G.n[1], 1.0, [&](int L) { return xy_threads(G, L) / 64; }));
   if (b->ndim > 2)
-    b->acc_L = walk_length(G.n[2], 1.0, [&](int L) { return acc_threads(G, 2, L) / 64; });
+    b->acc_L = even_length(
+        G.n[2], walk_length(G.n[2], 1.0, [&](int L) { return acc_threads(G, 2, L) / 64; }));
 }
 
 DeferList defer_list(rhy_box* b) {

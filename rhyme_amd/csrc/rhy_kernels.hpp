@@ -925,28 +925,32 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void acc_walk_kernel(
 // Cells (or faces, or 64-cell steps) a lane walks, of n along the axis:
 // waves(L) waves walk L each at the cost of `extra` more for a wave's start
 // (its first loads, half step and face).  A longer walk repeats less work, a
-// shorter one gives the chip's 1024 SIMDs more waves, of which each holds 3.
-// With w waves per SIMD a wave's step takes max(0.68 + 0.16 (w - 1), w / 3) of
-// what it takes beside two others: the chain of dependent operations of one
-// wave, or the SIMD's issue.  Measured on 1024^2 (walk_xy, FP64, ms per pass
-// of 100 steps): 32 cells 35.5, 16 23.4, 9 14.5, 7 13.4, 6 11.9 (3078 waves),
-// 4 12.6 (4608); on 40 x 33 x 27 one solve takes 114 us with 1 face per lane
-// and 199 us with 8; 256^3 does not care between 6 and 32, where 16 re-reads
-// less than shorter walks and is the limit.
+// shorter one gives the chip's 1024 SIMDs, which hold 3 waves each, more and
+// evener shares: with w waves per SIMD a wave's steps take w / 3 rounds of
+// three, and 0.6 of a round passes while the last ones end alone, each a
+// chain of dependent operations.  Measured (us a step): 1024^2 3 cells 113,
+// 4 117, 5 124, 6 117, 7 136, 10 149; 1203 x 517 mixed 3 104, 6 123, 10 173;
+// 131 x 97 x 118 4 281, 5 280, 7 290, 9 279, 12 304; one solve of 40 x 33 x 27
+// 114 with 1 face per lane, 199 with 8.  256^3 does not care between 6 and
+// 32, where 16 re-reads less than shorter walks and is the limit.
 template <class W>
 inline int walk_length(int n, double extra, W waves) {
   int best = 1;
   double best_cost = 0.0;
   for (int L = 1; L <= 16 && L <= n; ++L) {
-    const double w = (double)waves(L) / 1024.0;
-    const double alone = w > 1.0 ? 0.68 + 0.16 * (w - 1.0) : 0.68;
-    const double cost = (L + extra) * (w / 3.0 > alone ? w / 3.0 : alone);
+    const double cost = (L + extra) * ((double)waves(L) / 3072.0 + 0.6);
     if (L == 1 || cost < best_cost) {
       best = L;
       best_cost = cost;
     }
   }
   return best;
+}
+
+// The same number of chunks of n, evenly filled.
+inline int even_length(int n, int L) {
+  const int chunks = (n + L - 1) / L;
+  return (n + chunks - 1) / chunks;
 }
 
 // One face's flux from scratch: the half steps of its two cells (the
