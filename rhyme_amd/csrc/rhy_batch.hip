@@ -109,21 +109,20 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void batch_flux_kernel(Cons
     const BTile T = tile_of(segs, tile_seg, ti);
     if ((int32_t)threadIdx.x >= T.count) continue;
     const BBox& B = boxes[T.box];
-    Consts kb = k;
-    if (LIM == 0) kb.limiter = B.limiter;
+    const int type = LIM ? LIM : B.limiter;
     const int64_t t = T.base + threadIdx.x;
     const R* c = arena + B.cell_off;
     R* F = arena + B.flux_off + (int64_t)T.kind * (ND + 2) * B.G.plane;
     const double d = dt[T.box];
     const uint32_t bx = (uint32_t)T.box;
     if (T.kind == 0)
-      flux_walk<ND, 0, LIM, R, PW, false>(kb, B.G, c, F, d, B.dx[0], nf_x, t, dl, bx);
+      flux_walk<ND, 0, LIM, R, PW, false>(type, B.G, c, F, d, B.dx[0], nf_x, t, dl, bx);
     if constexpr (ND > 1)
       if (T.kind == 1)
-        flux_walk<ND, 1, LIM, R, PW, false>(kb, B.G, c, F, d, B.dx[1], nf_yz, t, dl, bx);
+        flux_walk<ND, 1, LIM, R, PW, false>(type, B.G, c, F, d, B.dx[1], nf_yz, t, dl, bx);
     if constexpr (ND > 2)
       if (T.kind == 2)
-        flux_walk<ND, 2, LIM, R, PW, false>(kb, B.G, c, F, d, B.dx[2], nf_yz, t, dl, bx);
+        flux_walk<ND, 2, LIM, R, PW, false>(type, B.G, c, F, d, B.dx[2], nf_yz, t, dl, bx);
   }
 }
 

@@ -302,6 +302,20 @@ __device__ __forceinline__ double lane_below(double x) {
   return __builtin_bit_cast(double, lo | (hi << 32));
 }
 
+// The Consts a kernel was launched with (its first parameter), read from the
+// kernel's arguments where they are used.  Held in scalar registers across a
+// walk, their 60 registers beside the masks of the Riemann solve were spilled
+// to vector lanes: 420 v_readlane in walk_xy, one VALU instruction in ten of a
+// moving gas, and 4 to 13 vector registers to memory, whose reloads wait for
+// the walk's stores.  The scalar loads hit the scalar cache; the empty asm
+// keeps them from being moved out of the walk's loop.
+__device__ __forceinline__ const Consts& kernel_consts() {
+  typedef const __attribute__((address_space(4))) Consts* Args;
+  Args p = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Consts*)p;
+}
+
 // Intercell flux on every face normal to axis A that the interior update
 // reads: face f in [0, n_A] sits between cells f and f+1, the other indices
 // run over the interior (the faces-only range the update consumes,
@@ -314,7 +328,7 @@ __device__ __forceinline__ double lane_below(double x) {
 // R is the storage/bulk type (double: the FP64 drop-in; float: the mixed
 // form, whose half step and the conversions around the Riemann solve run in
 // FP32 while the star-state solve and the sampling run in FP64 with the
-// MixedMath policy).  LIM is the slope limiter (slid).  PW is the policy of
+// MixedMath policy).  LIM is the slope limiter (slid; 0: `type`).  PW is the policy of
 // the Riemann solve; with Deferring<P> the faces that need P's slow paths
 // are listed in dl, tagged with `box`, for the fixup kernel.
 //
@@ -328,7 +342,7 @@ __device__ __forceinline__ double lane_below(double x) {
 // loads and flux stores are contiguous along x, and each half step is formed
 // once (plus one warm-up step per wave).
 template <int ND, int LIM, typename R, class PW>
-__device__ __forceinline__ void flux_xrows(const Consts& k, const Geom& G,
+__device__ __forceinline__ void flux_xrows(int type, const Geom& G,
                                            const R* __restrict__ cells, R* __restrict__ F,
                                            double dt, double dx, int steps, int64_t t,
                                            const DeferList& dl, uint32_t box) {
@@ -375,7 +389,7 @@ __device__ __forceinline__ void flux_xrows(const Consts& k, const Geom& G,
       load_state<ND, R>(cells, G.plane, o - 1, um);
       load_state<ND, R>(cells, G.plane, o, u0);
       load_state<ND, R>(cells, G.plane, o + 1, up);
-      half_step<ND, 0, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+      half_step<ND, 0, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rn, type);
     } else {
 #pragma unroll
       for (int c = 0; c < NV; ++c) lw[c] = rn[c] = R(0);
@@ -389,10 +403,10 @@ __device__ __forceinline__ void flux_xrows(const Consts& k, const Geom& G,
     }
     if (m >= 0 && valid && ci >= 1) {  // face ci - 1, between cells ci - 1 and ci
       R Fr[NV];
-      riemann_flux<ND, 0, PW, R>(k, rp, lw, Fr);
+      riemann_flux<ND, 0, PW, R>(kernel_consts(), rp, lw, Fr);
 #pragma unroll
       for (int c = 0; c < NV; ++c) F[o - 1 + c * G.plane] = Fr[c];
-      defer_take<PW>(k, dl, box, 0, o - 1);
+      defer_take<PW>(kernel_consts(), dl, box, 0, o - 1);
     }
   }
 }
@@ -406,12 +420,12 @@ __device__ __forceinline__ void flux_xrows(const Consts& k, const Geom& G,
 // ring, FP64 cells through the ring without the early load, which keeps the
 // kernel within 3 waves per SIMD unspilled.
 template <int ND, int A, int LIM, typename R, class PW, bool WINDOW = true>
-__device__ __forceinline__ void flux_walk(const Consts& k, const Geom& G,
+__device__ __forceinline__ void flux_walk(int type, const Geom& G,
                                           const R* __restrict__ cells, R* __restrict__ F,
                                           double dt, double dx, int nf_max, int64_t t,
                                           const DeferList& dl, uint32_t box) {
   if constexpr (A == 0) {
-    flux_xrows<ND, LIM, R, PW>(k, G, cells, F, dt, dx, nf_max, t, dl, box);
+    flux_xrows<ND, LIM, R, PW>(type, G, cells, F, dt, dx, nf_max, t, dl, box);
     return;
   }
   constexpr int NV = ND + 2;
@@ -438,7 +452,7 @@ __device__ __forceinline__ void flux_walk(const Consts& k, const Geom& G,
   load_state<ND, R>(cells, G.plane, o - s, um);
   load_state<ND, R>(cells, G.plane, o, u0);
   load_state<ND, R>(cells, G.plane, o + s, up);
-  half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rp);
+  half_step<ND, A, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rp, type);
   if constexpr (sizeof(R) == sizeof(float) && WINDOW) {
     // FP32 cells: a sliding window carries two cells to the next half step
     // and loads one new cell, issued before the Riemann solve so that its
@@ -454,17 +468,17 @@ __device__ __forceinline__ void flux_walk(const Consts& k, const Geom& G,
         u0[c] = up[c];
         up[c] = nx[c];
       }
-      half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+      half_step<ND, A, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rn, type);
       if (m + 1 < nf) load_state<ND, R>(cells, G.plane, o + (m + 3) * s, nx);
       R Fr[NV];
-      riemann_flux<ND, A, PW, R>(k, rp, lw, Fr);
+      riemann_flux<ND, A, PW, R>(kernel_consts(), rp, lw, Fr);
       const int64_t of = o + m * s;
 #pragma unroll
       for (int c = 0; c < NV; ++c) {
         F[of + c * G.plane] = Fr[c];
         rp[c] = rn[c];
       }
-      defer_take<PW>(k, dl, box, A, of);
+      defer_take<PW>(kernel_consts(), dl, box, A, of);
     }
   } else if constexpr (RHY_LDS_WALK && (sizeof(R) == sizeof(double) ? WINDOW : !WINDOW)) {
     // Cells through a lane-private ring of 4 cells in LDS (cell j of the
@@ -495,17 +509,17 @@ __device__ __forceinline__ void flux_walk(const Consts& k, const Geom& G,
       get(m, um);
       get(m + 1, u0);
       get(m + 2, up);
-      half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+      half_step<ND, A, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rn, type);
       if (m + 1 < nf) put(m + 3, nx);
       R Fr[NV];
-      riemann_flux<ND, A, PW, R>(k, rp, lw, Fr);
+      riemann_flux<ND, A, PW, R>(kernel_consts(), rp, lw, Fr);
       const int64_t of = o + m * s;
 #pragma unroll
       for (int c = 0; c < NV; ++c) {
         F[of + c * G.plane] = Fr[c];
         rp[c] = rn[c];
       }
-      defer_take<PW>(k, dl, box, A, of);
+      defer_take<PW>(kernel_consts(), dl, box, A, of);
     }
   } else if constexpr (RHY_LDS_WALK && sizeof(R) == sizeof(double)) {
     // Batched FP64 walks: the ring without the early load, so no registers
@@ -527,16 +541,16 @@ __device__ __forceinline__ void flux_walk(const Consts& k, const Geom& G,
         u0[c] = ring[(((m + 1) & 3) * NV + c) * kWalkLanes + lane];
         ring[(((m + 2) & 3) * NV + c) * kWalkLanes + lane] = up[c];
       }
-      half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+      half_step<ND, A, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rn, type);
       R Fr[NV];
-      riemann_flux<ND, A, PW, R>(k, rp, lw, Fr);
+      riemann_flux<ND, A, PW, R>(kernel_consts(), rp, lw, Fr);
       const int64_t of = o + m * s;
 #pragma unroll
       for (int c = 0; c < NV; ++c) {
         F[of + c * G.plane] = Fr[c];
         rp[c] = rn[c];
       }
-      defer_take<PW>(k, dl, box, A, of);
+      defer_take<PW>(kernel_consts(), dl, box, A, of);
     }
   } else {
     // Without the LDS ring (RHY_LDS_WALK=0): only rp (the right state of the
@@ -549,16 +563,16 @@ __device__ __forceinline__ void flux_walk(const Consts& k, const Geom& G,
       load_state<ND, R>(cells, G.plane, oc - s, um);
       load_state<ND, R>(cells, G.plane, oc, u0);
       load_state<ND, R>(cells, G.plane, oc + s, up);
-      half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+      half_step<ND, A, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rn, type);
       R Fr[NV];
-      riemann_flux<ND, A, PW, R>(k, rp, lw, Fr);
+      riemann_flux<ND, A, PW, R>(kernel_consts(), rp, lw, Fr);
       const int64_t of = o + m * s;
 #pragma unroll
       for (int c = 0; c < NV; ++c) {
         F[of + c * G.plane] = Fr[c];
         rp[c] = rn[c];
       }
-      defer_take<PW>(k, dl, box, A, of);
+      defer_take<PW>(kernel_consts(), dl, box, A, of);
     }
   }
 }
@@ -581,7 +595,7 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void flux_kernel(
     Consts k, Geom G, const R* __restrict__ cells, R* __restrict__ F,
     const double* __restrict__ dtp, double dx, int nf, DeferList dl) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  flux_walk<ND, A, LIM, R, PW>(k, G, cells, F, *dtp, dx, nf, t, dl, 0u);
+  flux_walk<ND, A, LIM, R, PW>(LIM, G, cells, F, *dtp, dx, nf, t, dl, 0u);
 }
 
 // ------------------------------------------------ accumulating walks ----
@@ -647,7 +661,7 @@ __device__ __forceinline__ double lane_above(double x) {
 constexpr int kXyOwn = 60;
 
 template <int ND, int LIM, typename R, class PW, int MODE>
-__device__ __forceinline__ double walk_xy(const Consts& k, const Geom& G,
+__device__ __forceinline__ double walk_xy(const Geom& G,
                                           const R* __restrict__ cells, R* __restrict__ out,
                                           const double* __restrict__ sc, int L, int order,
                                           int32_t wave, int32_t nwaves, const DeferList& dl) {
@@ -695,7 +709,7 @@ __device__ __forceinline__ double walk_xy(const Consts& k, const Geom& G,
     put(2, nx);
 #pragma unroll
     for (int c = 0; c < NV; ++c) rp[c] = R(0);
-    if (own) half_step<ND, 1, LIM, R>(k, um, u0, up, hdtdx1, lw, rp);
+    if (own) half_step<ND, 1, LIM, R>(kernel_consts(), um, u0, up, hdtdx1, lw, rp);
   }
   bool dyp = false;  // face m - 1 deferred
 #pragma unroll 1
@@ -714,14 +728,14 @@ __device__ __forceinline__ double walk_xy(const Consts& k, const Geom& G,
         get(m, -1, um);
         get(m, 0, u0);
         get(m, 1, up);
-        half_step<ND, 0, LIM, R>(k, um, u0, up, hdtdx0, lx, rx);
+        half_step<ND, 0, LIM, R>(kernel_consts(), um, u0, up, hdtdx0, lx, rx);
       }
 #pragma unroll
       for (int c = 0; c < NV; ++c) rx[c] = lane_below(rx[c]);
       uint32_t dlo = 0;
       if (xface) {
-        riemann_flux<ND, 0, PW, R>(k, rx, lx, F);
-        dlo = defer_take<PW>(k, dl, 0u, 0, o + (int64_t)m * s - 1) ? 1u : 0u;
+        riemann_flux<ND, 0, PW, R>(kernel_consts(), rx, lx, F);
+        dlo = defer_take<PW>(kernel_consts(), dl, 0u, 0, o + (int64_t)m * s - 1) ? 1u : 0u;
       }
 #pragma unroll
       for (int c = 0; c < NV; ++c) a0[c] = dtdx0 * (F[c] - lane_above(F[c]));
@@ -732,9 +746,9 @@ __device__ __forceinline__ double walk_xy(const Consts& k, const Geom& G,
       get(m, 0, um);
       get(m + 1, 0, u0);
       get(m + 2, 0, up);
-      half_step<ND, 1, LIM, R>(k, um, u0, up, hdtdx1, lw, rn);
-      riemann_flux<ND, 1, PW, R>(k, rp, lw, F);
-      const bool dy = defer_take<PW>(k, dl, 0u, 1, o + (int64_t)m * s);
+      half_step<ND, 1, LIM, R>(kernel_consts(), um, u0, up, hdtdx1, lw, rn);
+      riemann_flux<ND, 1, PW, R>(kernel_consts(), rp, lw, F);
+      const bool dy = defer_take<PW>(kernel_consts(), dl, 0u, 1, o + (int64_t)m * s);
       if (m > 0) {
         const int64_t oc = o + (int64_t)m * s;
         R un[NV];
@@ -749,7 +763,7 @@ __device__ __forceinline__ double walk_xy(const Consts& k, const Geom& G,
             double ud[NV];
 #pragma unroll
             for (int c = 0; c < NV; ++c) ud[c] = (double)un[c];
-            const double sp = cfl_speed<ND>(k, ud);
+            const double sp = cfl_speed<ND>(kernel_consts(), ud);
             smax = sp > smax ? sp : smax;
           }
         }
@@ -782,12 +796,12 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void walk_xy_kernel(
     double* __restrict__ partial) {
   const int32_t wave =
       __builtin_amdgcn_readfirstlane((int32_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
-  const double sp = walk_xy<ND, LIM, R, PW, MODE>(k, G, cells, out, sc, L, order, wave, nwaves, dl);
+  const double sp = walk_xy<ND, LIM, R, PW, MODE>(G, cells, out, sc, L, order, wave, nwaves, dl);
   if constexpr (MODE == kAccLast) block_max_to_partial(sp, partial);
 }
 
 template <int LIM, typename R, class PW>
-__device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
+__device__ __forceinline__ double flux_walk_acc(const Geom& G,
                                                 const R* __restrict__ cells,
                                                 const R* __restrict__ acc, R* __restrict__ out,
                                                 const double* __restrict__ sc, int L,
@@ -833,7 +847,7 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
   load_state<ND, R>(cells, G.plane, o - s, um);
   load_state<ND, R>(cells, G.plane, o, u0);
   load_state<ND, R>(cells, G.plane, o + s, up);
-  half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rp);
+  half_step<ND, A, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rp);
   put(0, u0);
   put(1, up);
   R nx[NV];
@@ -860,7 +874,7 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
       double ud[NV];
 #pragma unroll
       for (int c = 0; c < NV; ++c) ud[c] = (double)un[c];
-      const double sp = cfl_speed<ND>(k, ud);
+      const double sp = cfl_speed<ND>(kernel_consts(), ud);
       smax = sp > smax ? sp : smax;
     }
   };
@@ -875,27 +889,19 @@ __device__ __forceinline__ double flux_walk_acc(const Consts& k, const Geom& G,
     get(m, um);
     get(m + 1, u0);
     get(m + 2, up);
-    half_step<ND, A, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+    half_step<ND, A, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rn);
     if (m >= 2) {  // cell f0 + m - 1 (its ring slot is overwritten by the put)
       finish(m - 1, fh, qc, dp || dh);
-      dp = dh;
-    }
-    if (m + 1 < nf) put(m + 3, nx);
-    R Fr[NV];
-    riemann_flux<ND, A, PW, R>(k, rp, lw, Fr);
-    const bool dm = defer_take<PW>(k, dl, 0u, A, o + (int64_t)m * s);
+    } else if (m == 1) {  // the first face: no cell below
 #pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      rp[c] = rn[c];
-      if (m == 0)
-        fprev[c * kWalkLanes + lane] = Fr[c];
-      else
-        fh[c] = Fr[c];
+      for (int c = 0; c < NV; ++c) fprev[c * kWalkLanes + lane] = fh[c];
     }
-    if (m == 0)
-      dp = dm;
-    else
-      dh = dm;
+    dp = dh;
+    if (m + 1 < nf) put(m + 3, nx);
+    riemann_flux<ND, A, PW, R>(kernel_consts(), rp, lw, fh);
+    dh = defer_take<PW>(kernel_consts(), dl, 0u, A, o + (int64_t)m * s);
+#pragma unroll
+    for (int c = 0; c < NV; ++c) rp[c] = rn[c];
   }
   {  // the last cell, f0 + nf - 1 (faces nf - 2 and nf - 1; nf >= 2)
     R qc[NV];
@@ -918,7 +924,7 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void acc_walk_kernel(
     Consts k, Geom G, const R* __restrict__ cells, const R* __restrict__ acc, R* __restrict__ out,
     const double* __restrict__ sc, int L, int order, DeferList dl, double* __restrict__ partial) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  block_max_to_partial(flux_walk_acc<LIM, R, PW>(k, G, cells, acc, out, sc, L, order, t, dl),
+  block_max_to_partial(flux_walk_acc<LIM, R, PW>(G, cells, acc, out, sc, L, order, t, dl),
                        partial);
 }
 
@@ -969,9 +975,9 @@ __device__ __noinline__ void face_flux(const Consts& k, const Geom& G,
   load_state<ND, R>(cells, G.plane, of - s, um);
   load_state<ND, R>(cells, G.plane, of, u0);
   load_state<ND, R>(cells, G.plane, of + s, up);
-  half_step<ND, A, 0, R>(k, um, u0, up, hdtdx, l0, r0);
+  half_step<ND, A, 0, R>(k, um, u0, up, hdtdx, l0, r0, k.limiter);
   load_state<ND, R>(cells, G.plane, of + 2 * s, um);
-  half_step<ND, A, 0, R>(k, u0, up, um, hdtdx, l1, r1);
+  half_step<ND, A, 0, R>(k, u0, up, um, hdtdx, l1, r1, k.limiter);
   riemann_flux<ND, A, PW, R>(k, r0, l1, Fr);
 }
 
@@ -1174,7 +1180,7 @@ __global__ __launch_bounds__(kTubeLanes) RHY_FLUX_OCCUPANCY void tube_run_kernel
     double ud[NV];
 #pragma unroll
     for (int c = 0; c < NV; ++c) ud[c] = (double)w[c];
-    const double s = cfl_speed<1>(k, ud);
+    const double s = cfl_speed<1>(kernel_consts(), ud);
     speed = s > speed ? s : speed;
   };
   __syncthreads();
@@ -1215,7 +1221,7 @@ __global__ __launch_bounds__(kTubeLanes) RHY_FLUX_OCCUPANCY void tube_run_kernel
           u0[c] = u[c * P1 + i + 1];
           up[c] = u[c * P1 + i + 2];
         }
-        half_step<1, 0, LIM, R>(k, um, u0, up, hdtdx, lw, rn);
+        half_step<1, 0, LIM, R>(kernel_consts(), um, u0, up, hdtdx, lw, rn);
 #pragma unroll
         for (int c = 0; c < NV; ++c) rf[c * P1 + i] = rn[c];
       }
@@ -1224,14 +1230,14 @@ __global__ __launch_bounds__(kTubeLanes) RHY_FLUX_OCCUPANCY void tube_run_kernel
         R r[NV], F[NV];
 #pragma unroll
         for (int c = 0; c < NV; ++c) r[c] = rf[c * P1 + i - 1];
-        riemann_flux<1, 0, PW, R>(k, r, lw, F);
+        riemann_flux<1, 0, PW, R>(kernel_consts(), r, lw, F);
         if constexpr (PW::kDefer) {
           uint32_t& f = PW::flag();
           if (k.defer_every > 0 && i % k.defer_every == 0) f = 1u;  // i: the low cell's offset
           if (f) {
             f = 0u;
             if (s == nsteps - 1) atomicAdd(&deferred, 1u);
-            riemann_flux<1, 0, P, R>(k, r, lw, F);
+            riemann_flux<1, 0, P, R>(kernel_consts(), r, lw, F);
           }
         }
 #pragma unroll

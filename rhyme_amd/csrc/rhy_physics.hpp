@@ -347,9 +347,10 @@ __device__ __forceinline__ double slope_of(int type, double dL, double dR) {
 
 // rhyme_muscl_hancock_half_step_extrapolation.f90:15-21: slope from the
 // three cells um, u, up along axis A, then the half-step states l and r.
+// LIM == 0: with the limiter `type`.
 template <int ND, int A, int LIM = 0, typename R = double>
 __device__ __forceinline__ void half_step(const Consts& k, const R* um, const R* u, const R* up,
-                                          R hdtdx, R* l, R* r) {
+                                          R hdtdx, R* l, R* r, int type = 0) {
   constexpr int NV = ND + 2;
   constexpr bool kF64 = sizeof(R) == sizeof(double);
   R fl[NV], fr[NV];
@@ -357,14 +358,14 @@ __device__ __forceinline__ void half_step(const Consts& k, const R* um, const R*
   if (kF64 && w == R(0)) {
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
-      const R h = R(.5) * (R)slope_of<LIM>(k.limiter, u[c] - um[c], up[c] - u[c]);
+      const R h = R(.5) * (R)slope_of<LIM>(type, u[c] - um[c], up[c] - u[c]);
       l[c] = u[c] - h;
       r[c] = u[c] + h;
     }
   } else {
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
-      const R delta = limit_one<LIM, R>(k.limiter, w, um[c], u[c], up[c]);
+      const R delta = limit_one<LIM, R>(type, w, um[c], u[c], up[c]);
       l[c] = u[c] - R(.5) * delta;
       r[c] = u[c] + R(.5) * delta;
     }
