@@ -319,13 +319,7 @@ int launch_update(rhy_box* b, const Consts& k, const double* dx, int order, bool
 template <int ND>
 int launch_bc(rhy_box* b, const rhy_params_t* p, int face_only, void* hydro = nullptr) {
   const Geom& G = b->geom;
-  int64_t maxface = 1;
-  for (int a = 0; a < ND; ++a) {
-    int64_t m = 1;
-    for (int d = 0; d < 3; ++d)
-      if (d != a) m *= G.n[d];
-    maxface = m > maxface ? m : maxface;
-  }
+  const int64_t maxface = bc_threads(G, ND);
   // inflow states travel in device memory; they are copied only when they
   // change, after the box's queued work (which may still read them) is done,
   // so nothing refers to the caller's parameters once this call returns
@@ -339,15 +333,16 @@ int launch_bc(rhy_box* b, const rhy_params_t* p, int face_only, void* hydro = nu
   }
   TimedLaunch tl;
   timed_begin(b, 2, tl);
-  dim3 grid(grid_for(maxface), face_only >= 0 ? 1 : 2 * ND);
+  const int32_t gaps = face_only < 0 && (int64_t)G.n[1] * G.n[2] >= kGapRows;
+  dim3 grid(grid_for(maxface), face_only >= 0 ? 1 : 2 * ND - gaps);
   if (b->precision == RHY_MIXED)
     hipLaunchKernelGGL((bc_kernel<ND, float>), grid, dim3(kThreads), 0, b->stream, G, make_bc(p),
                        dinf, b->ncmp, static_cast<float*>(hydro ? hydro : b->cells),
-                       static_cast<float*>(b->extra), face_only);
+                       static_cast<float*>(b->extra), face_only, gaps);
   else
     hipLaunchKernelGGL((bc_kernel<ND, double>), grid, dim3(kThreads), 0, b->stream, G, make_bc(p),
                        dinf, b->ncmp, static_cast<double*>(hydro ? hydro : b->cells),
-                       static_cast<double*>(b->extra), face_only);
+                       static_cast<double*>(b->extra), face_only, gaps);
   timed_end(b, tl);
   HIP_TRY(hipGetLastError());
   return RHY_OK;

@@ -259,10 +259,10 @@ __global__ __launch_bounds__(256) void batch_cfl_kernel(Consts k, const BBox* __
   }
 }
 
-// Ghost cells of a box's faces, two per thread.
-inline int64_t face_cells(const Geom& G, int ndim) {
-  int64_t n = 0;
-  for (int a = 0; a < ndim; ++a) {
+// Threads of a box's ghost fill: its x gaps, then its y and z faces.
+inline int64_t fill_threads(const Geom& G, int ndim) {
+  int64_t n = (int64_t)(G.n[1] + 1) * G.n[2];
+  for (int a = 1; a < ndim; ++a) {
     int64_t m = 2;
     for (int d = 0; d < 3; ++d)
       if (d != a) m *= G.n[d];
@@ -285,17 +285,24 @@ __global__ __launch_bounds__(256) void batch_bc_kernel(const BBox* __restrict__ 
     if ((int32_t)threadIdx.x >= T.count) continue;
     const BBox& B = boxes[T.box];
     int64_t t = T.base + threadIdx.x;
-    int face = 0;
-    for (;; ++face) {
-      int64_t m = 1;
+    R* c = arena + B.cell_off;
+    R* x = c + (int64_t)(ND + 2) * B.G.plane;
+    int64_t m = (int64_t)(B.G.n[1] + 1) * B.G.n[2];
+    if (t < m) {
+      bc_x_gap<ND, R>(B.G, B.bc, inflow, ncmp, c, x, (uint32_t)t);
+      continue;
+    }
+    for (int face = 2; face < 2 * ND; ++face) {
+      t -= m;
+      m = 1;
 #pragma unroll
       for (int d = 0; d < 3; ++d)
         if (d != face / 2) m *= B.G.n[d];
-      if (t < m) break;
-      t -= m;
+      if (t < m) {
+        bc_face_cell<ND, R>(B.G, B.bc, inflow, ncmp, c, x, face, (uint32_t)t);
+        break;
+      }
     }
-    R* c = arena + B.cell_off;
-    bc_face_cell<ND, R>(B.G, B.bc, inflow, ncmp, c, c + (int64_t)(ND + 2) * B.G.plane, face, t);
   }
 }
 
@@ -827,7 +834,7 @@ int build_tiles(rhy_batch* b) {
   }
   b->nupd_tiles = start - b->nflux_tiles;
   for (int i : b->active) {
-    const int64_t n = face_cells(b->slots[i].B.G, nd);
+    const int64_t n = fill_threads(b->slots[i].B.G, nd);
     b->hsegs.push_back({start, i, 4, 0, n});
     start += (int32_t)cdiv(n, b->block);
   }

@@ -1338,73 +1338,139 @@ __global__ __launch_bounds__(256) void update_kernel(Consts k, Geom G, R* __rest
   if (FUSED) block_max_to_partial(speed, partial);
 }
 
-// Ghost fill of the t-th cell of a face: its two ghost cells
-// (rhyme_samr_bc_set_boundaries.f90:9-20 calls the faces in order; they are
-// disjoint and read interior cells only, so they run together).
+// Ghost fill (rhyme_samr_bc_set_boundaries.f90:9-20 calls the faces in order;
+// they are disjoint and read interior cells only, so they run together).
+// The two ghost cells beside one cell of a face, and the cells they copy.
+struct FaceGhosts {
+  int type;  // 0: nothing to fill
+  int64_t g0, g1, s0, s1;
+};
+
+// i1, i2: the cell's interior indices along the other two axes.
+__device__ __forceinline__ FaceGhosts face_ghosts(const Geom& G, const BcTypes& bc, int face,
+                                                  int i1, int i2) {
+  const int a = face / 2, side = face % 2;
+  int gi[3];
+  gi[a == 0 ? 1 : 0] = i1;
+  gi[a == 2 ? 1 : 2] = i2;
+  const int n = G.n[a];
+  FaceGhosts f;
+  f.type = bc.t[face];
+  if (f.type < 1 || f.type > 4) f.type = 0;
+  gi[a] = 1;
+  const int64_t first = goff(G, gi[0], gi[1], gi[2]);  // cell 1 of the axis
+  const int64_t s = G.s[a];
+  const int c0 = f.type == 3 ? (side ? 1 : n) : (side ? n : 1);
+  const int c1 = f.type == 3 ? (side ? 2 : n - 1) : (side ? n - 1 : 2);
+  f.g0 = first + (side ? n : -1) * s;
+  f.g1 = first + (side ? n + 1 : -2) * s;
+  f.s0 = first + (c0 - 1) * s;
+  f.s1 = first + (c1 - 1) * s;
+  return f;
+}
+
+template <int ND, typename R>
+__device__ __forceinline__ void ghosts_load(const Geom& G, const FaceGhosts& f,
+                                            const R* __restrict__ cells, R* v0, R* v1) {
+#pragma unroll
+  for (int c = 0; c < ND + 2; ++c) {  // interior cells whatever the type: no branch to wait at
+    v0[c] = cells[f.s0 + c * G.plane];
+    v1[c] = cells[f.s1 + c * G.plane];
+  }
+}
+
+template <int ND, typename R>
+__device__ __forceinline__ void ghosts_store(const Geom& G, const FaceGhosts& f, int face,
+                                             const double* __restrict__ inflow, int32_t ncmp,
+                                             R* __restrict__ cells, R* __restrict__ extra,
+                                             const R* v0, const R* v1) {
+  if (f.type == 4) {
+    for (int c = 0; c < ncmp; ++c) {
+      R* pc = comp_plane<R>(cells, extra, ND + 2, c, G.plane);
+      pc[f.g0] = (R)inflow[face * 16 + c];
+      pc[f.g1] = (R)inflow[face * 16 + c];
+    }
+  } else if (f.type) {
+    const bool flip = f.type == 1;
+#pragma unroll
+    for (int c = 0; c < ND + 2; ++c) {
+      const bool m = flip && c == 1 + face / 2;
+      cells[f.g0 + c * G.plane] = m ? -v0[c] : v0[c];
+      cells[f.g1 + c * G.plane] = m ? -v1[c] : v1[c];
+    }
+  }
+}
+
+// The t-th cell of a face.
 template <int ND, typename R>
 __device__ __forceinline__ void bc_face_cell(const Geom& G, const BcTypes& bc,
                                              const double* __restrict__ inflow, int32_t ncmp,
                                              R* __restrict__ cells, R* __restrict__ extra,
-                                             int face, int64_t t) {
-  const int a = face / 2, side = face % 2;
-  const int o1 = a == 0 ? 1 : 0;
-  const int o2 = a == 2 ? 1 : 2;
-  const int n1 = G.n[o1], n2 = G.n[o2];
-  if (t >= (int64_t)n1 * n2) return;
-  int idx[3];
-  idx[o1] = (int)(t % n1) + 1;
-  idx[o2] = (int)(t / n1) + 1;
-  const int n = G.n[a];
-  const int type = bc.t[face];
-  const int g0 = side ? n + 1 : 0, g1 = side ? n + 2 : -1;
-  int gi[3] = {idx[0], idx[1], idx[2]};
-  gi[a] = g0;
-  const int64_t og0 = goff(G, gi[0], gi[1], gi[2]);
-  gi[a] = g1;
-  const int64_t og1 = goff(G, gi[0], gi[1], gi[2]);
-  if (type == 4) {
-    for (int c = 0; c < ncmp; ++c) {
-      R* pc = comp_plane<R>(cells, extra, ND + 2, c, G.plane);
-      pc[og0] = (R)inflow[face * 16 + c];
-      pc[og1] = (R)inflow[face * 16 + c];
-    }
-    return;
-  }
-  if (type < 1 || type > 3) return;
-  int s0, s1;
-  if (type == 3) {
-    s0 = side ? 1 : n;
-    s1 = side ? 2 : n - 1;
-  } else {
-    s0 = side ? n : 1;
-    s1 = side ? n - 1 : 2;
-  }
-  gi[a] = s0;
-  const int64_t os0 = goff(G, gi[0], gi[1], gi[2]);
-  gi[a] = s1;
-  const int64_t os1 = goff(G, gi[0], gi[1], gi[2]);
-#pragma unroll
-  for (int c = 0; c < ND + 2; ++c) {
-    R v0 = cells[os0 + c * G.plane];
-    R v1 = cells[os1 + c * G.plane];
-    if (type == 1 && c == 1 + a) {
-      v0 = -v0;
-      v1 = -v1;
-    }
-    cells[og0 + c * G.plane] = v0;
-    cells[og1 + c * G.plane] = v1;
-  }
+                                             int face, uint32_t t) {
+  const uint32_t n1 = face / 2 == 0 ? G.n[1] : G.n[0], n2 = face / 2 == 2 ? G.n[1] : G.n[2];
+  if (t >= n1 * n2) return;  // a box has fewer than 2^31 cells
+  const uint32_t q = n2 == 1 ? 0u : t / n1;
+  const FaceGhosts f = face_ghosts(G, bc, face, (int)(t - q * n1) + 1, (int)q + 1);
+  R v0[ND + 2], v1[ND + 2];
+  ghosts_load<ND, R>(G, f, cells, v0, v1);
+  ghosts_store<ND, R>(G, f, face, inflow, ncmp, cells, extra, v0, v1);
 }
 
-// Stand-alone ghost fill, one thread per face cell; blockIdx.y = face.
+// The t-th gap between x rows: the ghosts above row j (x right) and below
+// row j + 1 (x left), j = 0 .. n1, which lie beside each other in memory, so
+// that the cells of a gap are one or two cache lines instead of two or four.
+// All loads come before the stores: an x face is bound by the lines it
+// touches, a lane to each.  256^3 44 -> 37 us,
+// mixed 250 x 192 x 129 26 -> 19 us.
+template <int ND, typename R>
+__device__ __forceinline__ void bc_x_gap(const Geom& G, const BcTypes& bc,
+                                         const double* __restrict__ inflow, int32_t ncmp,
+                                         R* __restrict__ cells, R* __restrict__ extra, uint32_t t) {
+  const uint32_t gaps = G.n[1] + 1;
+  if (t >= gaps * (uint32_t)G.n[2]) return;
+  const uint32_t q = G.n[2] == 1 ? 0u : t / gaps;
+  const int j = (int)(t - q * gaps), k = (int)q + 1;
+  FaceGhosts r = face_ghosts(G, bc, 1, j > 0 ? j : 1, k);
+  FaceGhosts l = face_ghosts(G, bc, 0, j < G.n[1] ? j + 1 : j, k);
+  if (j == 0) r.type = 0;
+  if (j == G.n[1]) l.type = 0;
+  R r0[ND + 2], r1[ND + 2], l0[ND + 2], l1[ND + 2];
+  ghosts_load<ND, R>(G, r, cells, r0, r1);
+  ghosts_load<ND, R>(G, l, cells, l0, l1);
+  ghosts_store<ND, R>(G, r, 1, inflow, ncmp, cells, extra, r0, r1);
+  ghosts_store<ND, R>(G, l, 0, inflow, ncmp, cells, extra, l0, l1);
+}
+
+// Stand-alone ghost fill, blockIdx.y: the faces, or (gaps) the gaps of the x
+// rows, then the faces of y and z; face_only >= 0: that face.  Gaps from
+// kGapRows rows on: a thread's 20 loads take longer than the 10 of a face
+// (40 x 33 x 27 8.5 us against 7.7, 1024^2 6.8 against 6.2, 131 x 97 x 118
+// the same) until the lines count.
+constexpr int64_t kGapRows = 16384;
 template <int ND, typename R = double>
 __global__ __launch_bounds__(256) void bc_kernel(Geom G, BcTypes bc, const double* __restrict__ inflow,
                                                  int32_t ncmp, R* __restrict__ cells,
-                                                 R* __restrict__ extra, int32_t face_only) {
-  const int face = face_only >= 0 ? face_only : (int)blockIdx.y;
+                                                 R* __restrict__ extra, int32_t face_only,
+                                                 int32_t gaps) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (gaps && blockIdx.y == 0) {
+    bc_x_gap<ND, R>(G, bc, inflow, ncmp, cells, extra, t);
+    return;
+  }
+  const int face = face_only >= 0 ? face_only : (int)blockIdx.y + gaps;
   if (face / 2 >= ND) return;
-  bc_face_cell<ND, R>(G, bc, inflow, ncmp, cells, extra, face,
-                      (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+  bc_face_cell<ND, R>(G, bc, inflow, ncmp, cells, extra, face, t);
+}
+// Its grid for every face: threads across the largest of them.
+inline int64_t bc_threads(const Geom& G, int ndim) {
+  int64_t m = (int64_t)(G.n[1] + 1) * G.n[2];
+  for (int a = 1; a < ndim; ++a) {
+    int64_t f = 1;
+    for (int d = 0; d < 3; ++d)
+      if (d != a) f *= G.n[d];
+    m = f > m ? f : m;
+  }
+  return m;
 }
 
 // max over the interior of |v| + c_s (rhyme_cfl_time_step.f90:40-47).
