@@ -88,7 +88,8 @@ struct rhy_box {
   int32_t nf[3] = {8, 8, 8};      // walk lengths for this shape (choose_walks): the
   int32_t xy_L = 16, acc_L = 16;  // flux walks', walk_xy's and the z walk's
   int32_t partial_cap = 0;
-  double* scalars = nullptr;      // [0] max_u, [16..16+6*RHY_MAX_CMP) inflow states
+  double* host_max = nullptr;     // pinned: the wave speed of rhy_cfl_time_step (lazy)
+  double* scalars = nullptr;      // [16..16+6*RHY_MAX_CMP) inflow states
   double inflow_copied[6 * RHY_MAX_CMP] = {};  // what the device inflow slots hold
   bool inflow_valid = false;
   double* dt = nullptr;           // current dt
@@ -201,9 +202,12 @@ int64_t axis_faces(const Geom& G, int a) {
 // The walk lengths of a box's shape (walk_length).
 void choose_walks(rhy_box* b) {
   const Geom& G = b->geom;
-  for (int a = 0; a < b->ndim; ++a)
-    b->nf[a] = walk_length(a == 0 ? 8 : G.n[a] + 1, 0.7,
-                           [&](int L) { return flux_threads(G, a, L) / 64; });
+  for (int a = 0; a < b->ndim; ++a)  // the axes' walks share a launch
+    b->nf[a] = walk_length(a == 0 ? 8 : G.n[a] + 1, 0.7, [&](int L) {
+      int64_t w = 0;
+      for (int d = 0; d < b->ndim; ++d) w += flux_threads(G, d, L) / 64;
+      return w;
+    });
   if (b->ndim > 1)
     b->xy_L = even_length(
         G.n[1], walk_length(G.n[1], 1.0, [&](int L) { return xy_threads(G, L) / 64; }));
@@ -221,38 +225,32 @@ DeferList defer_list(rhy_box* b) {
   return dl;
 }
 
-template <int ND, int A, int LIM, typename R, class PW>
-void launch_flux_axis(rhy_box* b, const Consts& k, const double* dx, const DeferList& dl) {
+template <int ND, int LIM, typename R, class PW>
+void launch_flux_lim(rhy_box* b, const Consts& k, const double* dx, const DeferList& dl) {
   const Geom& G = b->geom;
-  const int nf = b->nf[A];
-  const int64_t nthreads = flux_threads(G, A, nf);
-  R* F = static_cast<R*>(b->flux) + (int64_t)A * (ND + 2) * G.plane;
+  FluxPlan plan{};
+  for (int a = 0; a < 3; ++a) {
+    plan.first[a + 1] = plan.first[a];
+    if (a >= ND) continue;
+    plan.first[a + 1] += grid_for(flux_threads(G, a, b->nf[a]));
+    plan.nf[a] = b->nf[a];
+    plan.dx[a] = dx[a];
+  }
   TimedLaunch tl;
   timed_begin(b, 0, tl);
-  hipLaunchKernelGGL((flux_kernel<ND, A, LIM, R, PW>), dim3(grid_for(nthreads)),
-                     dim3(kThreads), 0, b->stream, k, G, static_cast<const R*>(b->cells), F, b->dt,
-                     dx[A], nf, dl);
+  hipLaunchKernelGGL((flux_kernel<ND, LIM, R, PW>), dim3(plan.first[3]), dim3(kThreads), 0,
+                     b->stream, k, G, static_cast<const R*>(b->cells), static_cast<R*>(b->flux),
+                     b->dt, plan, dl);
+  tl.axes = ND;
   timed_end(b, tl);
 }
 
-template <int ND, int LIM, typename R, class PW>
-void launch_flux_lim(rhy_box* b, const Consts& k, const double* dx, const DeferList& dl) {
-  launch_flux_axis<ND, 0, LIM, R, PW>(b, k, dx, dl);
-  if constexpr (ND > 1) launch_flux_axis<ND, 1, LIM, R, PW>(b, k, dx, dl);
-  if constexpr (ND > 2) launch_flux_axis<ND, 2, LIM, R, PW>(b, k, dx, dl);
-}
-
-// The flux kernels run with policy PW (Deferring<P> unless built with libm
-// pow) and list the faces that need P's slow paths; the fixup kernel then
-// recomputes those with P.  The list is emptied before the first axis.
+// The flux kernel runs with policy PW (Deferring<P> unless built with libm
+// pow) and lists the faces that need P's slow paths; the fixup kernel then
+// recomputes those with P.  The list was emptied with the step's dt.
 template <int ND, typename R, class PW, class P>
 void launch_flux_r(rhy_box* b, const Consts& k, const double* dx) {
   const DeferList dl = defer_list(b);
-  TimedLaunch tr;
-  timed_begin(b, 5, tr);
-  hipLaunchKernelGGL(step_reset_kernel, dim3(1), dim3(64), 0, b->stream, b->defer_count, 4,
-                     (double*)nullptr);
-  timed_end(b, tr);
   switch (k.limiter) {
     case 1: launch_flux_lim<ND, 1, R, PW>(b, k, dx, dl); break;
     case 2: launch_flux_lim<ND, 2, R, PW>(b, k, dx, dl); break;
@@ -541,7 +539,7 @@ int run_steps(rhy_box* b, const rhy_params_t* p, const double* dx, int32_t nstep
     timed_begin(b, 4, tl);
     hipLaunchKernelGGL(dt_kernel, dim3(1), dim3(1024), 0, b->stream, b->partial, np, cmdx, b->dt,
                        b->dt_log + s, (double*)nullptr, dx[0], dx[1], dx[2], step_consts(b),
-                       ND > 1 ? b->defer_count : (uint32_t*)nullptr,
+                       b->defer_count,
                        ND > 1 ? b->partial + b->acc_blocks : (double*)nullptr);
     timed_end(b, tl);
     if constexpr (ND > 1) {
@@ -789,6 +787,7 @@ int rhy_box_destroy(rhy_box_t* b) {
   collect_timings(b);
   free_box_memory(b);
   if (b->scalars) (void)hipFree(b->scalars);
+  if (b->host_max) (void)hipHostFree(b->host_max);
   if (b->dt) (void)hipFree(b->dt);
   if (b->dt_log) (void)hipFree(b->dt_log);
   if (b->diag) (void)hipFree(b->diag);
@@ -1124,13 +1123,19 @@ int rhy_cfl_time_step(rhy_box_t* b, const rhy_params_t* p, const double dx[3], d
   else if (b->ndim == 2) rc = launch_cfl<2>(b, k);
   else rc = launch_cfl<3>(b, k);
   if (rc) return rc;
+  // the speed goes straight to host memory: a copy of 8 bytes is a launch of
+  // its own
+  if (!b->host_max &&
+      hipHostMalloc(reinterpret_cast<void**>(&b->host_max), sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();
+    b->host_max = nullptr;
+    return fail(RHY_ERR_OOM, "host memory for the wave speed");
+  }
   hipLaunchKernelGGL(dt_kernel, dim3(1), dim3(1024), 0, b->stream, b->partial, b->partial_n, 0.0,
-                     (double*)nullptr, (double*)nullptr, b->scalars);
+                     (double*)nullptr, (double*)nullptr, b->host_max);
   HIP_TRY(hipGetLastError());
-  double maxu = 0.0;
-  HIP_TRY(hipMemcpyAsync(&maxu, b->scalars, sizeof(maxu), hipMemcpyDeviceToHost, b->stream));
   HIP_TRY(hipStreamSynchronize(b->stream));
-  *dt = p->courant * min_dx(b->ndim, dx) / maxu;
+  *dt = p->courant * min_dx(b->ndim, dx) / *b->host_max;
   return RHY_OK;
 }
 
@@ -1147,7 +1152,7 @@ int mh_solve_enqueue(rhy_box* b, const rhy_params_t* p, const double* dx, double
   if (p->solver_type != RHY_CPU_INTENSIVE && p->solver_type != RHY_MEMORY_INTENSIVE)
     return fail(RHY_ERR_SOLVER, "Unknown solver type");
   const Consts k = consts_of(p);
-  hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(64), 0, b->stream, b->dt, dt);
+  hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(64), 0, b->stream, b->dt, dt, b->defer_count);
   const BcTypes bc = make_bc(p);
   if (b->ndim == 1) {
     if ((rc = launch_flux<1>(b, k, dx))) return rc;
