@@ -80,19 +80,15 @@ def load_pmc_summary():
 # rocprofv3 prints them; kernels shared by the legs of both precisions,
 # such as dt_kernel, enter at their mean over all dispatches).
 STEP_KERNELS = {
-    "fp64": r"^void rhy::(flux_kernel<3, 0, \d, double|acc_walk_kernel<3, \d, \d, double|"
-            r"acc_fixup_kernel<3, \d, double|flux_fixup_kernel<3, double|update_kernel<3, \d, \w+, "
-            r"double|bc_kernel<3, double)|^rhy::(dt_kernel|step_reset_kernel)",
-    "mixed": r"^void rhy::(flux_kernel<3, 0, \d, float|acc_walk_kernel<3, \d, \d, float|"
-             r"acc_fixup_kernel<3, \d, float|flux_fixup_kernel<3, float|update_kernel<3, \d, \w+, "
-             r"float|bc_kernel<3, float)|^rhy::(dt_kernel|step_reset_kernel)",
-    "batched_fp64": r"batch_(flux|fixup|update)_kernel<3, [^>]*double|batch_dt_kernel|"
-                    r"batch_step_counter_kernel|^rhy::set_u32_kernel",
-    "batched_mixed": r"batch_(flux|fixup|update)_kernel<3, [^>]*float|batch_dt_kernel|"
-                     r"batch_step_counter_kernel|^rhy::set_u32_kernel",
+    "fp64": r"^void rhy::(walk_xy_kernel<3, \d, double|acc_walk_kernel<\d, double|"
+            r"acc_fixup_kernel<[02], double|bc_kernel<3, double)|^rhy::dt_kernel",
+    "mixed": r"^void rhy::(walk_xy_kernel<3, \d, float|acc_walk_kernel<\d, float|"
+             r"acc_fixup_kernel<[02], float|bc_kernel<3, float)|^rhy::dt_kernel",
+    "batched_fp64": r"batch_(flux|fixup|update)_kernel<3, [^>]*double|batch_dt_kernel",
+    "batched_mixed": r"batch_(flux|fixup|update)_kernel<3, [^>]*float|batch_dt_kernel",
 }
 # the kernels that walk faces (VALU-issue bound) in each leg
-WALK_KERNELS = r"flux_kernel<|acc_walk_kernel<|batch_flux_kernel<"
+WALK_KERNELS = r"flux_kernel<|walk_xy_kernel<|acc_walk_kernel<|batch_flux_kernel<"
 # kernels the run also launches for other (smaller) boxes: only their
 # dispatches of at least half the largest size enter the summary
 LARGEST_ONLY = r"bc_kernel<"
@@ -489,9 +485,8 @@ def main():
     zu = zones * a.steps / g["elapsed"]
     ms_step = 1e3 * g["elapsed"] / a.steps
     st = g["stats"]
-    # kernels of one step: dt (4), deferred-face list reset and fixup (5),
-    # x flux walk and y/z accumulating walks (0), update (1, 1D boxes only),
-    # ghost fill of the new state (2)
+    # kernels of one step: dt (4), fixups (5), the x/y and z accumulating walks
+    # (0), update (1, 1D boxes only), ghost fill of the new state (2)
     kern_ms = sum(st[k][1] for k in (0, 1, 2, 4, 5)) / max(st[4][0], 1)  # per timed step
     flux_ms = st[0][1] / max(st[0][0], 1)
     bytes_alg = 80.0 * zones
@@ -508,10 +503,9 @@ def main():
                     achieved_wall=achieved_wall, frac_wall=achieved_wall / HBM_PEAK_GBS,
                     flux_kernel_bound="valu issue",
                     flux_kernel_valu_issue_frac=pmc["fp64"]["walk_valu_issue"] if pmc else None,
-                    kernel="one step: dt_kernel + deferred-list reset + x flux walk + its fixup "
-                           "+ y and z accumulating walks + their fixups + ghost fill (achieved: "
-                           "over the HIP-event sum of these kernels; achieved_wall: over "
-                           "ms_per_step)",
+                    kernel="one step: dt_kernel + the x/y and the z accumulating walk, each "
+                           "with its fixup, + ghost fill (achieved: over the HIP-event sum of "
+                           "these kernels; achieved_wall: over ms_per_step)",
                     events="HIP events on the box stream around every launch of timed steps "
                            "0, %d, %d, ... (%d of the %d)" % (a.event_every, 2 * a.event_every,
                                                               st[4][0], a.steps),
