@@ -29,8 +29,18 @@ constexpr size_t kChunk = (size_t)2 << 20;  // staging bytes of one chunk, at mo
 constexpr size_t kMinChunk = (size_t)256 << 10;
 constexpr int kWorkers = 8;
 constexpr int kSlots = 2 * kWorkers;
-// Below this the threads cost more than they give.
-constexpr size_t kMinStaged = (size_t)2 << 20;
+
+// Whether a copy of `bytes` device bytes is staged: from the size on where the
+// threads give more than they cost (a queued copy and an event for each chunk,
+// the helpers' wakes), by direction and conversion.  Direct against staged, us:
+//   from the host      24 MiB 676 / 742   32 MiB 914 / 908    64 MiB 2304 / 1729
+//   to the host         6 MiB 344 / 406    8 MiB 455 / 450    32 MiB 1885 / 946
+//   narrowed (mixed)    6 MiB 365 / 383    8 MiB 476 / 427    32 MiB 3993 / 942
+//   widened (mixed)     3 MiB 287 / 295    4 MiB 430 / 377    32 MiB 4655 / 1027
+inline bool worth_staging(size_t bytes, bool as_double, bool to_host) {
+  const size_t mib = as_double ? (to_host ? 4 : 8) : (to_host ? 8 : 32);
+  return bytes >= mib << 20;
+}
 
 // The helpers of a copy: threads that wait for work(index), index 1 .. n.
 // (Starting threads for each copy takes as long as a copy of 4 MB.)
@@ -266,7 +276,7 @@ hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t es
                 bool to_host) {
   size_t bytes = 0;
   for (int i = 0; i < nspans; ++i) bytes += spans[i].count * esz;
-  StagingHold held(bytes >= kMinStaged);
+  StagingHold held(worth_staging(bytes, as_double, to_host));
   if (!held.staging) return copy_direct(stream, spans, nspans, esz, as_double, to_host);
   Job job;
   hipError_t e = hipGetDevice(&job.device);
