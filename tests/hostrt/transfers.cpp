@@ -55,6 +55,17 @@ int main(int argc, char** argv) {
     std::printf("copies %d ", hostrt::copies);
     rhy::transfer_user_drop();
   }
+  if (what == "pinned") {  // caller memory the runtime knows
+    std::vector<double> dev((size_t)8 << 20), host((size_t)8 << 20, 1.5);
+    hostrt::pinned_lo = host.data();
+    hostrt::pinned_hi = host.data() + host.size();
+    const rhy::HostSpan span = {dev.data(), host.data(), host.size()};
+    rhy::transfer_user_add();
+    ok = rhy::copy_spans(&s, &span, 1, 8, false, false) == hipSuccess && dev == host &&
+         rhy::copy_spans(&s, &span, 1, 8, false, true) == hipSuccess;
+    rhy::transfer_user_drop();
+    std::printf("copies %d ", hostrt::copies);
+  }
   std::printf("ok %d events %d pinned %zu\n", ok, hostrt::events, hostrt::pinned_bytes);
   return ok ? 0 : 1;
 }

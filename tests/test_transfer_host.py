@@ -38,3 +38,7 @@ def test_staged_only_where_it_is_faster(program, kind, way, least):
         got = call(program, "route", kib, kind, way)
         assert (got["copies"] > 1) == staged, (kib, kind, way, got)
         assert got["events"] == 0 and got["pinned"] == 0  # all given back
+
+
+def test_pinned_caller_memory_is_copied_directly(program):
+    assert call(program, "pinned")["copies"] == 2
