@@ -292,7 +292,11 @@ hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t es
   StagingHold held(staged);
   if (!held.staging) return copy_direct(stream, spans, nspans, esz, as_double, to_host);
   Job job;
-  hipError_t e = hipGetDevice(&job.device);
+  // the workers' events belong to the stream's device, which need not be the
+  // caller's current one
+  int current = 0;
+  hipError_t e = hipGetDevice(&current);
+  if (e == hipSuccess) e = hipStreamGetDevice(stream, &job.device);
   if (e == hipSuccess) {
     job.stream = stream;
     job.esz = esz;
@@ -315,6 +319,7 @@ hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t es
     const std::function<void(int)> work = [&job](int w) { job.work(w); };
     g_helpers->run(workers - 1, work);
     e = (hipError_t)job.error.load();
+    (void)hipSetDevice(current);  // worker 0 was this thread
     const hipError_t es = hipStreamSynchronize(stream);
     if (e == hipSuccess) e = es;
   }

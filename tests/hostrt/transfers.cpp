@@ -66,6 +66,13 @@ int main(int argc, char** argv) {
     rhy::transfer_user_drop();
     std::printf("copies %d ", hostrt::copies);
   }
+  if (what == "device") {  // a box of device 0 while the caller's is device 1
+    hostrt::device = 1;
+    rhy::transfer_user_add();
+    ok = round_trip((size_t)8 << 20, false, true, true, &s) && hostrt::copies > 2;
+    rhy::transfer_user_drop();
+    std::printf("current %d ", hostrt::device);
+  }
   std::printf("ok %d events %d pinned %zu\n", ok, hostrt::events, hostrt::pinned_bytes);
   return ok ? 0 : 1;
 }

@@ -42,3 +42,7 @@ def test_staged_only_where_it_is_faster(program, kind, way, least):
 
 def test_pinned_caller_memory_is_copied_directly(program):
     assert call(program, "pinned")["copies"] == 2
+
+
+def test_box_on_another_device_than_the_current_one(program):
+    assert call(program, "device")["current"] == 1
