@@ -15,10 +15,10 @@
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -58,7 +58,7 @@ struct Helpers {
     for (int i = 1; i < kWorkers; ++i) {
       try {
         threads.emplace_back([this, i] { loop(i); });
-      } catch (const std::system_error&) {
+      } catch (const std::exception&) {  // no thread or no memory for one
         break;  // the ones there are take the chunks
       }
     }
@@ -117,7 +117,11 @@ unsigned char* staging_take() {
   std::lock_guard<std::mutex> hold(g_lock);
   if (g_taken) return nullptr;
   if (!g_staging) {
-    if (!g_helpers) g_helpers = new Helpers;
+    try {
+      if (!g_helpers) g_helpers = new Helpers;
+    } catch (const std::bad_alloc&) {
+      return nullptr;
+    }
     void* p = nullptr;
     if (hipHostMalloc(&p, kChunk * kSlots, hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();
@@ -219,6 +223,17 @@ struct Job {
   std::atomic<size_t> next{0};
   std::atomic<int> error{(int)hipSuccess};
 
+  // The chunks: two for each worker, within [kMinChunk, kChunk].
+  void cut(const HostSpan* spans, int nspans, size_t bytes, size_t esz, bool as_double) {
+    const size_t part = std::min(std::max(bytes / kSlots, kMinChunk), kChunk);
+    const size_t per = part / esz, hsz = as_double ? sizeof(double) : esz;
+    for (int i = 0; i < nspans; ++i)
+      for (size_t at = 0; at < spans[i].count; at += per)
+        chunks.push_back({static_cast<unsigned char*>(spans[i].dev) + at * esz,
+                          static_cast<unsigned char*>(spans[i].host) + at * hsz,
+                          std::min(spans[i].count - at, per)});
+  }
+
   void fail(hipError_t e) {
     int ok = (int)hipSuccess;
     error.compare_exchange_strong(ok, (int)e);
@@ -292,6 +307,11 @@ hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t es
   StagingHold held(staged);
   if (!held.staging) return copy_direct(stream, spans, nspans, esz, as_double, to_host);
   Job job;
+  try {
+    job.cut(spans, nspans, bytes, esz, as_double);
+  } catch (const std::bad_alloc&) {  // nothing has been queued by then
+    return copy_direct(stream, spans, nspans, esz, as_double, to_host);
+  }
   // the workers' events belong to the stream's device, which need not be the
   // caller's current one
   int current = 0;
@@ -303,17 +323,6 @@ hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t es
     job.as_double = as_double;
     job.to_host = to_host;
     job.staging = held.staging;
-    // two chunks for each worker, within [kMinChunk, kChunk]
-    const size_t part = std::min(std::max(bytes / kSlots, kMinChunk), kChunk);
-    const size_t per = part / esz;
-    for (int i = 0; i < nspans; ++i) {
-      const size_t hsz = as_double ? sizeof(double) : esz;
-      for (size_t at = 0; at < spans[i].count; at += per) {
-        const size_t n = spans[i].count - at < per ? spans[i].count - at : per;
-        job.chunks.push_back({static_cast<unsigned char*>(spans[i].dev) + at * esz,
-                              static_cast<unsigned char*>(spans[i].host) + at * hsz, n});
-      }
-    }
     const size_t half = (job.chunks.size() + 1) / 2;
     const int workers = half < (size_t)kWorkers ? (int)half : kWorkers;
     const std::function<void(int)> work = [&job](int w) { job.work(w); };

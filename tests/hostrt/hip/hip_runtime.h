@@ -85,13 +85,14 @@ inline hipError_t hipStreamSynchronize(hipStream_t) {
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   std::lock_guard<std::mutex> hold(hostrt::lock);
   ++hostrt::events;
-  *e = new FakeEvent{hostrt::device};
+  *e = static_cast<FakeEvent*>(std::malloc(sizeof(FakeEvent)));
+  (*e)->device = hostrt::device;
   return hipSuccess;
 }
 inline hipError_t hipEventDestroy(hipEvent_t e) {
   std::lock_guard<std::mutex> hold(hostrt::lock);
   --hostrt::events;
-  delete e;
+  std::free(e);
   return hipSuccess;
 }
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {

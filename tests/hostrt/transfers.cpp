@@ -1,10 +1,22 @@
 // One call of the transfers a line of arguments, on the host runtime beside
 // this file; prints what the call did.
+#include <atomic>
 #include <cstdio>
+#include <new>
 #include <string>
 #include <vector>
 
 #include "rhy_transfer.hip"
+
+// The allocation that fails: counted down by every one while at or above 0.
+static std::atomic<int> g_fail_at{-1};
+void* operator new(size_t n) {
+  if (g_fail_at.load() >= 0 && g_fail_at.fetch_sub(1) == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace {
 
@@ -72,6 +84,21 @@ int main(int argc, char** argv) {
     ok = round_trip((size_t)8 << 20, false, true, true, &s) && hostrt::copies > 2;
     rhy::transfer_user_drop();
     std::printf("current %d ", hostrt::device);
+  }
+  if (what == "memory") {  // every allocation of a first copy fails in turn
+    const size_t n = (size_t)8 << 20;
+    std::vector<double> dev(n), host(n);
+    ok = true;
+    for (int at = 0; at < 40 && ok; ++at) {
+      for (size_t i = 0; i < n; i += 997) host[i] = (double)at + 1.0;
+      const rhy::HostSpan span = {dev.data(), host.data(), n};
+      rhy::transfer_user_add();
+      g_fail_at = at;
+      ok = rhy::copy_spans(&s, &span, 1, 8, false, false) == hipSuccess;
+      g_fail_at = -1;
+      ok = ok && dev == host;
+      rhy::transfer_user_drop();
+    }
   }
   std::printf("ok %d events %d pinned %zu\n", ok, hostrt::events, hostrt::pinned_bytes);
   return ok ? 0 : 1;

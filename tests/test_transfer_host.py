@@ -46,3 +46,9 @@ def test_pinned_caller_memory_is_copied_directly(program):
 
 def test_box_on_another_device_than_the_current_one(program):
     assert call(program, "device")["current"] == 1
+
+
+def test_no_memory_on_the_way(program):
+    """Whichever allocation fails, the copy is made, in one piece or in chunks."""
+    got = call(program, "memory")
+    assert got["events"] == 0 and got["pinned"] == 0
