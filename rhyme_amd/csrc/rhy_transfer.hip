@@ -107,16 +107,27 @@ struct Helpers {
 // One staging area (32 MB) and set of helpers per process, used by one copy at
 // a time: a copy that finds them taken goes the direct way.  They go with the
 // last box or batch; in a process that ends before, with the process.
+//
+// To pin the memory, start the threads and give both back is about 0.5 ms, which
+// a program that makes a box, copies a little and drops it again would pay each
+// time.  So the first copies of the objects alive go the direct way, until
+// staging them would have saved that much: 29 us for each MiB to the host or
+// converted, at least, and half of it from the host.
+constexpr size_t kWorth = (size_t)32 << 20;
 std::mutex g_lock;
 unsigned char* g_staging = nullptr;
 Helpers* g_helpers = nullptr;
-bool g_taken = false;
+bool g_taken = false, g_refused = false;
+size_t g_missed = 0;  // what direct copies missed since the last giving back
 int g_users = 0;
 
-unsigned char* staging_take() {
+// saves: what staging saves a copy, in bytes to the host.
+unsigned char* staging_take(size_t saves) {
   std::lock_guard<std::mutex> hold(g_lock);
-  if (g_taken) return nullptr;
+  if (g_taken || g_refused) return nullptr;
   if (!g_staging) {
+    g_missed += saves;
+    if (g_missed < kWorth) return nullptr;
     try {
       if (!g_helpers) g_helpers = new Helpers;
     } catch (const std::bad_alloc&) {
@@ -125,6 +136,7 @@ unsigned char* staging_take() {
     void* p = nullptr;
     if (hipHostMalloc(&p, kChunk * kSlots, hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();
+      g_refused = true;  // not asked for again until the last object has gone
       return nullptr;
     }
     g_staging = static_cast<unsigned char*>(p);
@@ -139,6 +151,8 @@ void staging_free_if_idle() {  // with g_lock held
   g_staging = nullptr;
   delete g_helpers;
   g_helpers = nullptr;
+  g_refused = false;
+  g_missed = 0;
 }
 
 void staging_give() {
@@ -149,7 +163,7 @@ void staging_give() {
 
 struct StagingHold {
   unsigned char* staging;
-  explicit StagingHold(bool wanted) : staging(wanted ? staging_take() : nullptr) {}
+  explicit StagingHold(size_t saves) : staging(saves ? staging_take(saves) : nullptr) {}
   ~StagingHold() {
     if (staging) staging_give();
   }
@@ -304,7 +318,7 @@ hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t es
   for (int i = 0; i < nspans; ++i) bytes += spans[i].count * esz;
   bool staged = worth_staging(bytes, as_double, to_host);
   for (int i = 0; i < nspans && staged && !as_double; ++i) staged = !pinned(spans[i].host);
-  StagingHold held(staged);
+  StagingHold held(!staged ? 0 : to_host || as_double ? bytes : bytes / 2);
   if (!held.staging) return copy_direct(stream, spans, nspans, esz, as_double, to_host);
   Job job;
   try {

@@ -67,6 +67,29 @@ int main(int argc, char** argv) {
     std::printf("copies %d ", hostrt::copies);
     rhy::transfer_user_drop();
   }
+  if (what == "short") {  // objects that copy 12 MiB to the host and go
+    ok = true;
+    for (int i = 0; i < 20 && ok; ++i) {
+      rhy::transfer_user_add();
+      ok = round_trip((size_t)3 << 19, false, false, true, &s);
+      rhy::transfer_user_drop();
+    }
+    std::printf("asked %d ", hostrt::pinned_calls);
+  }
+  if (what == "long") {  // one that makes the same copies
+    ok = true;
+    rhy::transfer_user_add();
+    for (int i = 0; i < 20 && ok; ++i) ok = round_trip((size_t)3 << 19, false, false, true, &s);
+    std::printf("asked %d held %d ", hostrt::pinned_calls, hostrt::pinned_bytes > 0);
+    rhy::transfer_user_drop();
+  }
+  if (what == "refused") {  // no pinned memory to be had
+    hostrt::refuse_pinned = ok = true;
+    rhy::transfer_user_add();
+    for (int i = 0; i < 5 && ok; ++i) ok = round_trip((size_t)8 << 20, false, true, true, &s);
+    std::printf("asked %d copies %d ", hostrt::pinned_calls, hostrt::copies);
+    rhy::transfer_user_drop();
+  }
   if (what == "pinned") {  // caller memory the runtime knows
     std::vector<double> dev((size_t)8 << 20), host((size_t)8 << 20, 1.5);
     hostrt::pinned_lo = host.data();
@@ -81,7 +104,7 @@ int main(int argc, char** argv) {
   if (what == "device") {  // a box of device 0 while the caller's is device 1
     hostrt::device = 1;
     rhy::transfer_user_add();
-    ok = round_trip((size_t)8 << 20, false, true, true, &s) && hostrt::copies > 2;
+    ok = round_trip((size_t)8 << 20, false, true, true, &s) && hostrt::copies > 2;  // 64 MiB
     rhy::transfer_user_drop();
     std::printf("current %d ", hostrt::device);
   }

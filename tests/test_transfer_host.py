@@ -52,3 +52,14 @@ def test_no_memory_on_the_way(program):
     """Whichever allocation fails, the copy is made, in one piece or in chunks."""
     got = call(program, "memory")
     assert got["events"] == 0 and got["pinned"] == 0
+
+
+def test_short_lived_objects_do_not_pay_for_staging(program):
+    assert call(program, "short")["asked"] == 0
+    got = call(program, "long")
+    assert got["asked"] == 1 and got["held"] == 1 and got["pinned"] == 0
+
+
+def test_refused_pinned_memory_is_asked_for_once(program):
+    got = call(program, "refused")
+    assert got["asked"] == 1 and got["copies"] == 10
