@@ -886,7 +886,7 @@ static int box_snapshot(rhy_box_t* b, float* out, const float* in) {
   const dim3 grid = snapshot_grid(b->geom);
   const HostSpan span = {b->snap, in ? const_cast<float*>(in) : out, bytes / sizeof(float)};
   if (in) {
-    HIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, false));
+    HIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, false, false));
     if (b->precision == RHY_MIXED)
       hipLaunchKernelGGL(snapshot_unpack_kernel<float>, grid, dim3(kThreads), 0, b->stream,
                          b->geom, b->ncmp, b->ndim + 2, static_cast<float*>(b->cells),

@@ -1374,7 +1374,7 @@ static int batch_snapshot(rhy_batch_t* b, float* out, const float* in) {
     b->snap_elems = total;
   }
   const HostSpan span = {b->snap, in ? const_cast<float*>(in) : out, (size_t)total};
-  if (in) BHIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, false));
+  if (in) BHIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, false, false));
   int64_t ofs = 0;
   for (Slot& S : b->slots) {
     if (!S.active) continue;
@@ -1405,10 +1405,12 @@ static int batch_snapshot(rhy_batch_t* b, float* out, const float* in) {
     }
     ofs += blen * b->ncmp;
   }
+  if (in) {  // the caller's array is read until then
+    b->partials_valid = false;
+    BHIP_TRY(hipStreamSynchronize(b->stream));
+  }
   BHIP_TRY(hipGetLastError());
-  if (in) b->partials_valid = false;
   if (out) BHIP_TRY(copy_spans(b->stream, &span, 1, sizeof(float), false, true));
-  BHIP_TRY(hipStreamSynchronize(b->stream));
   return RHY_OK;
 }
 

@@ -203,7 +203,7 @@ void fill(void* to, const void* host, size_t count, size_t esz, bool as_double) 
 
 // A span at a time through the runtime, converted in a host buffer.
 hipError_t copy_direct(hipStream_t stream, const HostSpan* spans, int nspans, size_t esz,
-                       bool as_double, bool to_host) {
+                       bool as_double, bool to_host, bool wait) {
   std::vector<std::vector<float>> tmp(as_double ? (size_t)nspans : 0);
   for (int i = 0; as_double && i < nspans; ++i) tmp[i].resize(spans[i].count);
   for (int i = 0; i < nspans; ++i) {
@@ -221,6 +221,7 @@ hipError_t copy_direct(hipStream_t stream, const HostSpan* spans, int nspans, si
       return e;
     }
   }
+  if (!wait && !as_double) return hipSuccess;
   const hipError_t e = hipStreamSynchronize(stream);
   if (e == hipSuccess && as_double && to_host)
     for (int i = 0; i < nspans; ++i) unload(tmp[i].data(), spans[i].host, spans[i].count, esz, true);
@@ -313,18 +314,18 @@ struct Job {
 };
 
 hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t esz, bool as_double,
-                bool to_host) {
+                bool to_host, bool wait) {
   size_t bytes = 0;
   for (int i = 0; i < nspans; ++i) bytes += spans[i].count * esz;
   bool staged = worth_staging(bytes, as_double, to_host);
   for (int i = 0; i < nspans && staged && !as_double; ++i) staged = !pinned(spans[i].host);
   StagingHold held(!staged ? 0 : to_host || as_double ? bytes : bytes / 2);
-  if (!held.staging) return copy_direct(stream, spans, nspans, esz, as_double, to_host);
+  if (!held.staging) return copy_direct(stream, spans, nspans, esz, as_double, to_host, wait);
   Job job;
   try {
     job.cut(spans, nspans, bytes, esz, as_double);
   } catch (const std::bad_alloc&) {  // nothing has been queued by then
-    return copy_direct(stream, spans, nspans, esz, as_double, to_host);
+    return copy_direct(stream, spans, nspans, esz, as_double, to_host, wait);
   }
   // the workers' events belong to the stream's device, which need not be the
   // caller's current one
@@ -352,9 +353,9 @@ hipError_t copy(hipStream_t stream, const HostSpan* spans, int nspans, size_t es
 }  // namespace
 
 hipError_t copy_spans(hipStream_t stream, const HostSpan* spans, int nspans, size_t esz,
-                      bool as_double, bool to_host) {
+                      bool as_double, bool to_host, bool wait) {
   try {
-    return copy(stream, spans, nspans, esz, as_double, to_host);
+    return copy(stream, spans, nspans, esz, as_double, to_host, wait);
   } catch (const std::bad_alloc&) {  // no copy has been queued by then
     return hipErrorOutOfMemory;
   }

@@ -17,9 +17,11 @@ struct HostSpan {
 
 // Copies every span on `stream` and waits for it.  Device values take esz
 // bytes; host values the same, or, with as_double, are doubles of device
-// floats.  to_host gives the direction.
+// floats.  to_host gives the direction.  wait = false: the caller waits for the
+// stream itself before it returns, so that a copy that needs nothing from the
+// host once queued does not (4 us of a snapshot's way in).
 hipError_t copy_spans(hipStream_t stream, const HostSpan* spans, int nspans, size_t esz,
-                      bool as_double, bool to_host);
+                      bool as_double, bool to_host, bool wait = true);
 
 // Objects that may copy (boxes, batches): the staging memory is given back
 // when the last one goes.

@@ -90,6 +90,14 @@ int main(int argc, char** argv) {
     std::printf("asked %d copies %d ", hostrt::pinned_calls, hostrt::copies);
     rhy::transfer_user_drop();
   }
+  if (what == "wait") {  // a caller that waits for the stream itself
+    std::vector<double> dev(1000), host(1000, 1.5);
+    const rhy::HostSpan span = {dev.data(), host.data(), host.size()};
+    ok = rhy::copy_spans(&s, &span, 1, 8, false, false, false) == hipSuccess;
+    std::printf("unwaited %d ", hostrt::waits);
+    ok = ok && rhy::copy_spans(&s, &span, 1, 8, false, false) == hipSuccess;
+    std::printf("waited %d ", hostrt::waits);
+  }
   if (what == "pinned") {  // caller memory the runtime knows
     std::vector<double> dev((size_t)8 << 20), host((size_t)8 << 20, 1.5);
     hostrt::pinned_lo = host.data();

@@ -63,3 +63,8 @@ def test_short_lived_objects_do_not_pay_for_staging(program):
 def test_refused_pinned_memory_is_asked_for_once(program):
     got = call(program, "refused")
     assert got["asked"] == 1 and got["copies"] == 10
+
+
+def test_a_copy_whose_caller_waits_does_not_wait_too(program):
+    got = call(program, "wait")
+    assert got["unwaited"] == 0 and got["waited"] == 1
