@@ -420,6 +420,7 @@ struct PowLib {
 struct PowFast {
   static constexpr bool kFast = false;
   static constexpr bool kStar = true;
+  static constexpr bool kVacuum = true;
   static constexpr bool kDefer = false;
   __device__ __forceinline__ static double dv(double a, double b) { return a / b; }
   __device__ __forceinline__ static double sq(double x) { return sqrt(x); }
@@ -557,6 +558,9 @@ using PowF64 = PowLib;
 template <class P, int LANES = 256>
 struct Deferring : P {
   static constexpr bool kDefer = true;
+  // gas beside a vacuum in the walk; left to P in tube_run, which takes P on the
+  // spot (1024 cells at gamma 1.45: 19.6 us a step, 21.9 with it)
+  static constexpr bool kVacuum = LANES == 256;
   __device__ __forceinline__ static uint32_t& flag() {
     __shared__ uint32_t flags[LANES];
     return flags[threadIdx.x];
@@ -1113,10 +1117,40 @@ __device__ __forceinline__ bool star_sample(const Consts& k, double lr, const do
   return true;
 }
 
+// Gas u beside a vacuum, on its right (right = true) or left side
+// (rhyme_riemann_problem_solve.f90:37-60, with its own front speeds): the vacuum
+// or the undisturbed gas.  False for states out of plain_range, and inside the
+// rarefaction, which those speeds leave no room for unless gamma > 3.
+template <int ND, int A>
+__device__ __forceinline__ bool beside_vacuum(const Consts& k, const double* u, bool right,
+                                              double& rho, double* v, double& p) {
+  const double ir = recip(u[0]);
+  double ke2 = 0.0;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    v[d] = u[1 + d] * ir;
+    ke2 = d == 0 ? u[1] * v[0] : ke2 + u[1 + d] * v[d];
+  }
+  const double g = (u[ND + 1] - .5 * ke2) * k.gm1;
+  rho = u[0];
+  p = dmax(g, k.w_p);
+  const double c = sqrt_of(k.g * (g * ir)), sc = right ? c : -c;
+  const bool head = 0.0 > v[A] + sc, front = 0.0 > v[A] + k.c2g * sc;
+  if (right ? !head && !front : front) {
+    rho = k.w_rho;
+    p = k.w_p;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) v[d] = 0.0;
+    return plain_range(u[0]) && g > 0x1p-200 && g < 0x1p200;
+  }
+  return head == right && plain_range(u[0]) && g > 0x1p-200 && g < 0x1p200;
+}
+
 // The FP64 state sampled at x/t = 0: side states, exact contacts (these need
 // no sound speed: both sides carry the upwind side's rho and v with p* = p,
-// u* = u), then star_sample; vacuum, pressures at or under the floor and
-// whatever star_sample refuses through riemann_sample_ref or the fixup.
+// u* = u), then star_sample; a vacuum on one side by beside_vacuum, and what
+// either refuses (vacuum generated, no pressure, states out of range) through
+// riemann_sample_ref or the fixup.
 template <int ND, int A, class PW>
 __device__ __forceinline__ void riemann_sample(const Consts& k, const double* l, const double* r,
                                                double& srho, double* sv, double& sp) {
@@ -1125,7 +1159,32 @@ __device__ __forceinline__ void riemann_sample(const Consts& k, const double* l,
     return;
   } else {
     bool ok = plain_range(l[0]) && plain_range(r[0]) && l[0] >= k.e_rho && r[0] >= k.e_rho;
-    if (ok) {
+    // the rare faces first and out of the registers: held in them across the
+    // star state's solve they cost every face 5 to 15% of a step (256^3 971 ->
+    // 1123 us)
+    const bool gas = ok;
+    constexpr bool kHere = PW::kVacuum;
+    volatile double stash[ND + 2];
+    if (kHere && !wave_all(gas)) {
+      if (!gas) {
+        const bool vl = l[0] < k.e_rho, vr = r[0] < k.e_rho;
+        double rho = k.w_rho, v[ND], p = k.w_p;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) v[d] = 0.0;
+        ok = vl && vr;
+        if (vl != vr) {
+          double u[ND + 2];
+#pragma unroll
+          for (int c = 0; c < ND + 2; ++c) u[c] = vl ? r[c] : l[c];
+          ok = u[0] > k.e_rho && beside_vacuum<ND, A>(k, u, vl, rho, v, p);
+        }
+        stash[0] = rho;
+        stash[ND + 1] = p;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) stash[1 + d] = v[d];
+      }
+    }
+    if (gas) {
       const double il = recip(l[0]), ir = recip(r[0]);
       double lv[ND], rv[ND], lk = 0.0, rk = 0.0;
 #pragma unroll
@@ -1135,9 +1194,10 @@ __device__ __forceinline__ void riemann_sample(const Consts& k, const double* l,
         lk = d == 0 ? l[1] * lv[0] : lk + l[1 + d] * lv[d];
         rk = d == 0 ? r[1] * rv[0] : rk + r[1 + d] * rv[d];
       }
-      const double lp = (l[ND + 1] - .5 * lk) * k.gm1;
-      const double rp = (r[ND + 1] - .5 * rk) * k.gm1;
-      ok = lp > k.w_p && rp > k.w_p && plain_range(lp) && plain_range(rp);
+      // the floor is the pressure's, not the sound speed's (side_prims)
+      const double lg = (l[ND + 1] - .5 * lk) * k.gm1, rg = (r[ND + 1] - .5 * rk) * k.gm1;
+      const double lp = dmax(lg, k.w_p), rp = dmax(rg, k.w_p);
+      ok = lg > 0x1p-200 && rg > 0x1p-200 && lp < 0x1p200 && rp < 0x1p200;
 #if RHY_CONTACT_EXACT
       if (ok && lp == rp && lv[A] == rv[A]) {
         const bool right = 0.0 > lv[A];
@@ -1150,9 +1210,18 @@ __device__ __forceinline__ void riemann_sample(const Consts& k, const double* l,
 #endif
       // c^2 = gamma p / rho
       if (ok)
-        ok = star_sample<ND, A>(k, l[0], lv, lp, sqrt_of(k.g * (lp * il)), r[0], rv, rp,
-                                sqrt_of(k.g * (rp * ir)), srho, sv, sp);
-    } else if (l[0] < k.e_rho && r[0] < k.e_rho) {  // vacuum on both sides
+        ok = star_sample<ND, A>(k, l[0], lv, lp, sqrt_of(k.g * (lg * il)), r[0], rv, rp,
+                                sqrt_of(k.g * (rg * ir)), srho, sv, sp);
+    }
+    if (kHere && !wave_all(gas)) {
+      if (!gas) {
+        srho = stash[0];
+        sp = stash[ND + 1];
+#pragma unroll
+        for (int d = 0; d < ND; ++d) sv[d] = stash[1 + d];
+      }
+    }
+    if (!kHere && l[0] < k.e_rho && r[0] < k.e_rho) {  // vacuum on both sides
       srho = k.w_rho;
       sp = k.w_p;
 #pragma unroll
