@@ -519,7 +519,9 @@ int run_steps(rhy_box* b, const rhy_params_t* p, const double* dx, int32_t nstep
   int rc;
   if ((rc = ensure_dt_log(b, nsteps > 0 ? nsteps : 1))) return rc;
   const double cmdx = p->courant * min_dx(ND, dx);
-  const int tube = ND == 1 && b->prof_every == 0 ? tube_threads(b->geom.n[0]) : 0;
+  const int tube = ND == 1 && b->prof_every == 0
+                       ? tube_threads(b->geom.n[0], b->precision == RHY_MIXED)
+                       : 0;
   if (tube > 0) {
     if ((rc = launch_bc<ND>(b, p, -1))) return rc;
     launch_tube(b, k, bc, dx[0], cmdx, nsteps, tube);

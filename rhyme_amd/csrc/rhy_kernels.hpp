@@ -1165,8 +1165,8 @@ __global__ __launch_bounds__(256) void acc_fixup_kernel(
 // tube_run: nsteps steps of a small 1D box in one workgroup and one launch,
 // its state in LDS: a step through kernels of its own (the fluxes, their
 // fixup, the update, dt and a reset) is 20.5 us whatever its cells, most of
-// it launches and first loads; here it is 5.5 us at 64 cells, 8.7 at 766,
-// 12.4 at 1024 and 15.3 at 2040, the chain of dependent operations of one
+// it launches and first loads; here it is 5.2 us at 64 cells, 8.7 at 766,
+// 12.5 at 1024 and 15.1 at 1534, the chain of dependent operations of one
 // half step and one Riemann solve for each round of cells.  A thread takes every blockDim-th cell; the
 // right half states of a strip of cells lie in `rf` for the cells above, and
 // a face's flux takes the slot of the half state that only it reads.  A face
@@ -1174,7 +1174,7 @@ __global__ __launch_bounds__(256) void acc_fixup_kernel(
 // The arithmetic and its order are flux_xrows', update_kernel's and
 // dt_kernel's.
 constexpr int kTubeLanes = 768;  // 3 waves per SIMD: 168 VGPRs
-constexpr int kTubeCells = 2040;  // 4 rounds would be 19 us of the 20.5
+constexpr int kTubeCells = 2 * kTubeLanes - 2;  // two rounds (tube_threads)
 using PowF64Tube = typename WithLanes<PowF64Flux, kTubeLanes>::type;
 using MixedTube = typename WithLanes<MixedFlux, kTubeLanes>::type;
 
@@ -1282,10 +1282,15 @@ __global__ __launch_bounds__(kTubeLanes) RHY_FLUX_OCCUPANCY void tube_run_kernel
   if (tid < 4) defer_count[tid] = tid == 0 ? deferred : 0u;
 }
 
-// Threads of tube_run for n cells, 0 for more than it holds: the fewest rounds of at most kTubeLanes cells, evenly filled.
-inline int tube_threads(int n) {
-  if (n > kTubeCells) return 0;
+// Threads of tube_run for n cells, in the fewest rounds of at most kTubeLanes
+// half steps, evenly filled; 0 where the kernels of a step are the faster: from
+// the third round on, and in the mixed form, whose face solves are longer, from
+// the second.  us a step, tube_run against the kernels of a step (17 to 20 at any
+// size): FP64 766 cells 8.7, 1534 15.1, 2040 21.3; mixed 766 cells 14.2,
+// 1024 21.5, 2040 36.5.
+inline int tube_threads(int n, bool mixed) {
   const int rounds = (n + 2 + kTubeLanes - 1) / kTubeLanes;
+  if (rounds > (mixed ? 1 : 2)) return 0;
   const int per = (n + 2 + rounds - 1) / rounds;
   return (per + 63) / 64 * 64;
 }
