@@ -430,7 +430,7 @@ void launch_acc_step_lim(rhy_box* b, const Consts& k, const double* dx,
   timed_begin(b, 0, tl);
   hipLaunchKernelGGL((walk_xy_kernel<ND, LIM, R, PW, MODE>),
                      dim3(grid_for(xy_threads(G, b->xy_L))), dim3(kThreads), 0, b->stream, k, G,
-                     cur, xy, step_consts(b), b->xy_L, order, xy_waves(G), dlxy, b->partial);
+                     cur, xy, step_consts(b), b->xy_L, order, xy_waves(G, b->xy_L), dlxy, b->partial);
   tl.axes = 2;
   timed_end(b, tl);
   if constexpr (PW::kDefer)

@@ -665,10 +665,12 @@ __device__ __forceinline__ double lane_above(double x) {
   return __builtin_bit_cast(double, lo | (hi << 32));
 }
 
-// walk_xy: a wave takes 64 consecutive columns of the x rows at one y --
-// columns numbered row after row over z with all ghosts, n0 + 4 to a row, so
-// that they are consecutive in memory -- and walks L cells along y.  Each
-// lane's cells pass through its LDS ring (loaded from HBM once, the next one
+// walk_xy: a wave takes 64 consecutive columns of the x rows at one y (2D: at
+// the first y of one or several chunks) -- columns numbered row after row over z
+// (2D: over the chunks) with all ghosts, n0 + 4 to a row, so that a row's are
+// consecutive in memory -- and walks L cells along y.  (A wave for each 60 columns
+// of one 2D chunk left most of its lanes idle on a narrow box: 16 x 65536 mixed
+// 401 us a step.)  Each lane's cells pass through its LDS ring (loaded from HBM once, the next one
 // during the half steps).  At a row, the x half steps take their stencil from
 // the neighbouring lanes' ring slots, the low side of the face (l-1, l) and
 // the flux of the face (l, l+1) come from the neighbouring lanes by DPP, so
@@ -687,22 +689,23 @@ __device__ __forceinline__ double walk_xy(const Geom& G,
   constexpr int NV = ND + 2;
   defer_clear<PW>();
   double smax = 0.0;
+  // 2D: the rows' columns, chunk after chunk; 3D: a chunk's columns, z after z
   const int32_t rowlen = G.n[0] + 4;
-  const int32_t ncol = rowlen * G.n[2];
-  const int32_t chunk = wave / nwaves;
-  const int f0 = chunk * L;
-  if (f0 >= G.n[1]) return smax;  // the whole wave
-  const int nc = G.n[1] - f0 < L ? G.n[1] - f0 : L;  // cells f0+1 .. f0+nc
+  const int32_t ncol = rowlen * (ND == 2 ? (G.n[1] + L - 1) / L : G.n[2]);
+  const int32_t chunk = ND == 2 ? 0 : wave / nwaves;
+  if (ND == 2 ? wave >= nwaves : chunk * L >= G.n[1]) return smax;  // the whole wave
   const int lane = threadIdx.x & 63;
   int32_t q = (wave - chunk * nwaves) * kXyOwn + lane;
   const bool valid = q < ncol;
   q = valid ? q : ncol - 1;
   const int32_t row = q / rowlen;
   const int ci = q - row * rowlen - 1;  // x index, -1 .. n0+2
+  const int f0 = (ND == 2 ? row : chunk) * L;
+  const int nc = G.n[1] - f0 < L ? G.n[1] - f0 : L;  // cells f0+1 .. f0+nc
   const bool own = valid && lane >= 2 && lane <= 61 && ci >= 1 && ci <= G.n[0];
   const bool xhalf = valid && lane >= 1 && lane <= 62 && ci >= 0 && ci <= G.n[0] + 1;
   const bool xface = valid && lane >= 2 && lane <= 62 && ci >= 1 && ci <= G.n[0] + 1;
-  const int64_t o = goff(G, ci, f0, row + 1);
+  const int64_t o = goff(G, ci, f0, ND == 2 ? 1 : row + 1);
   const int64_t s = G.s[1];
   const R dtdx0 = (R)sc[1], dtdx1 = (R)sc[2];
   const R hdtdx0 = (R)sc[4], hdtdx1 = (R)sc[5];
@@ -799,13 +802,14 @@ __device__ __forceinline__ double walk_xy(const Geom& G,
   return smax;
 }
 
-// Waves across the columns of walk_xy.
-__host__ __device__ inline int32_t xy_waves(const Geom& G) {
-  return ((G.n[0] + 4) * G.n[2] - 4 + kXyOwn - 1) / kXyOwn;
+// Waves across the columns of walk_xy with chunks of L cells (2D: of all chunks).
+__host__ __device__ inline int32_t xy_waves(const Geom& G, int L) {
+  const int32_t rows = G.n[2] > 1 ? G.n[2] : (G.n[1] + L - 1) / L;
+  return ((G.n[0] + 4) * rows - 4 + kXyOwn - 1) / kXyOwn;
 }
 // Threads of walk_xy with chunks of L cells.
 __host__ __device__ inline int64_t xy_threads(const Geom& G, int L) {
-  return (int64_t)xy_waves(G) * ((G.n[1] + L - 1) / L) * 64;
+  return (int64_t)xy_waves(G, L) * (G.n[2] > 1 ? (G.n[1] + L - 1) / L : 1) * 64;
 }
 
 template <int ND, int LIM, typename R, class PW, int MODE>
