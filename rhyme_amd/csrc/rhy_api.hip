@@ -87,6 +87,7 @@ struct rhy_box {
   int32_t acc_blocks = 0;         // partials of the last accumulating walk
   int32_t nf[3] = {8, 8, 8};      // walk lengths for this shape (choose_walks): the
   int32_t xy_L = 16, acc_L = 16;  // flux walks', walk_xy's and the z walk's
+  bool planes = false;            // rhy_run steps through the flux planes (choose_walks)
   int32_t partial_cap = 0;
   double* host_max = nullptr;     // pinned: the wave speed of rhy_cfl_time_step (lazy)
   double* scalars = nullptr;      // [16..16+6*RHY_MAX_CMP) inflow states
@@ -199,7 +200,26 @@ int64_t axis_faces(const Geom& G, int a) {
 }
 
 
-// The walk lengths of a box's shape (walk_length).
+// Whether a 2D box's rhy_run steps through the flux planes instead of walk_xy.
+// The walk leaves the lanes of each row's four ghosts idle, n0 of n0 + 4 at work,
+// in the y faces too; the planes cost their traffic, little while they and the
+// state stay in the 256 MB last-level cache.  us a step, walk against planes:
+//   FP64   16 x 65536 139 / 116   32 x 32768 122 / 110   128 x 8192 104 / 105;
+//          beyond the cache 16 x 262144 472 / 472, still gas 245 / 394
+//   mixed  16 x 65536 188 / 143   64 x 16384 157 / 128   256 x 4096 139 / 123;
+//          beyond 32 x 262144 1040 / 873, still gas 285 / 357
+// Still gas, whose walk is short of bytes rather than of lanes, draws the line in
+// FP64: 64 x 16384 70 / 78 (mixed 86 / 71).  Boxes too small to fill the chip
+// are short of neither and keep one route at all widths.
+bool planes_faster(const rhy_box* b) {
+  const Geom& G = b->geom;
+  const int64_t cells = (int64_t)G.n[0] * G.n[1];
+  const int64_t bytes = 3 * 4 * cells * (int64_t)b->esz;  // a state, two flux planes of 4
+  return b->ndim == 2 && G.n[0] < (b->precision == RHY_MIXED ? 65 : 32) &&
+         cells >= 1 << 17 && bytes <= (int64_t)256 << 20;
+}
+
+// The walk lengths of a box's shape (walk_length), and its route.
 void choose_walks(rhy_box* b) {
   const Geom& G = b->geom;
   for (int a = 0; a < b->ndim; ++a)  // the axes' walks share a launch
@@ -208,6 +228,7 @@ void choose_walks(rhy_box* b) {
       for (int d = 0; d < b->ndim; ++d) w += flux_threads(G, d, L) / 64;
       return w;
     });
+  b->planes = planes_faster(b);
   if (b->ndim > 1)
     b->xy_L = even_length(
         G.n[1], walk_length(G.n[1], 1.0, [&](int L) { return xy_threads(G, L) / 64; }));
@@ -505,9 +526,10 @@ void launch_tube(rhy_box* b, const Consts& k, const BcTypes& bc, double dx, doub
 
 // The main loop's steps (src/main.f90:109-136) on the device.  Small 1D
 // boxes: all of them in one launch (tube_run_kernel; not while launches are
-// timed, which name the phases of a step).  Other 1D boxes: fluxes into planes, then the update with the fused epilogue (ghost
-// images and CFL partials of the new state).  2D/3D boxes: the
-// accumulating walks, whose last one writes the new state's interior and
+// timed, which name the phases of a step).  Other 1D boxes and narrow 2D
+// ones (planes_faster): fluxes into planes, then the update with the fused
+// epilogue (ghost images and CFL partials of the new state).  Other 2D/3D boxes:
+// the accumulating walks, whose last one writes the new state's interior and
 // CFL partials into the other state buffer (the buffers swap every step),
 // then the ghost fill of the new state.  Writing the ghost images from the
 // last walk instead costs that walk more than the separate fill takes.
@@ -536,21 +558,23 @@ int run_steps(rhy_box* b, const rhy_params_t* p, const double* dx, int32_t nstep
     if (b->prof_every > 1) b->profiling = s % b->prof_every == 0;
     // partials: the CFL pass's before the first step, the last walk's and
     // the fixup's slot after
-    const int32_t np = ND > 1 && s > 0 ? b->acc_blocks + 1 : b->partial_n;
+    const bool walks = ND > 2 || (ND == 2 && !b->planes);
+    const int32_t np = walks && s > 0 ? b->acc_blocks + 1 : b->partial_n;
     TimedLaunch tl;
     timed_begin(b, 4, tl);
     hipLaunchKernelGGL(dt_kernel, dim3(1), dim3(1024), 0, b->stream, b->partial, np, cmdx, b->dt,
                        b->dt_log + s, (double*)nullptr, dx[0], dx[1], dx[2], step_consts(b),
-                       b->defer_count,
-                       ND > 1 ? b->partial + b->acc_blocks : (double*)nullptr);
+                       b->defer_count, walks ? b->partial + b->acc_blocks : (double*)nullptr);
     timed_end(b, tl);
     if constexpr (ND > 1) {
-      if ((rc = launch_acc_step<ND>(b, k, dx, p->solver_type))) return rc;
-      if ((rc = launch_bc<ND>(b, p, -1))) return rc;  // the new state's ghosts
-    } else {
-      if ((rc = launch_flux<ND>(b, k, dx))) return rc;
-      if ((rc = launch_update<ND>(b, k, dx, p->solver_type, true, bc))) return rc;
+      if (walks) {
+        if ((rc = launch_acc_step<ND>(b, k, dx, p->solver_type))) return rc;
+        if ((rc = launch_bc<ND>(b, p, -1))) return rc;  // the new state's ghosts
+        continue;
+      }
     }
+    if ((rc = launch_flux<ND>(b, k, dx))) return rc;
+    if ((rc = launch_update<ND>(b, k, dx, p->solver_type, true, bc))) return rc;
   }
   b->profiling = b->prof_every == 1;
   b->last_nsteps = nsteps;
@@ -770,6 +794,7 @@ int rhy_box_resize(rhy_box_t* b, const int32_t dims[3]) {
   b->acc_blocks = t.acc_blocks;
   for (int a = 0; a < 3; ++a) b->nf[a] = t.nf[a];
   b->xy_L = t.xy_L;
+  b->planes = t.planes;
   b->acc_L = t.acc_L;
   b->partial_cap = t.partial_cap;
   b->defer_count = t.defer_count;
