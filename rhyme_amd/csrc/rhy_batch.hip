@@ -271,17 +271,26 @@ inline int64_t fill_threads(const Geom& G, int ndim) {
   return n;
 }
 
-// Ghost fill of every box.
+// The tiles of a ghost fill: those of nruns boxes, run i the tiles from first[i]
+// on; before[i]: the tiles of the runs before it.
+constexpr int kFillRuns = 16;
+struct FillPlan {
+  int32_t nruns;
+  int32_t first[kFillRuns], before[kFillRuns + 1];
+};
+
+// Ghost fill of the plan's boxes.
 template <int ND, typename R>
 __global__ __launch_bounds__(256) void batch_bc_kernel(const BBox* __restrict__ boxes,
                                                        const BSeg* __restrict__ segs,
                                                        const int32_t* __restrict__ tile_seg,
-                                                       int32_t first, int32_t ntiles,
-                                                       R* __restrict__ arena,
+                                                       FillPlan plan, R* __restrict__ arena,
                                                        const double* __restrict__ inflow,
                                                        int32_t ncmp) {
-  for (int32_t ti = first + blockIdx.x; ti < first + ntiles; ti += gridDim.x) {
-    const BTile T = tile_of(segs, tile_seg, ti);
+  for (int32_t i = blockIdx.x; i < plan.before[plan.nruns]; i += gridDim.x) {
+    int run = 0;
+    while (i >= plan.before[run + 1]) ++run;
+    const BTile T = tile_of(segs, tile_seg, plan.first[run] + i - plan.before[run]);
     if ((int32_t)threadIdx.x >= T.count) continue;
     const BBox& B = boxes[T.box];
     int64_t t = T.base + threadIdx.x;
@@ -948,18 +957,34 @@ void enqueue_step(rhy_batch* b, const Consts& k, int order, int lim, double fixe
 template <int ND, typename R>
 int prologue(rhy_batch* b, const Consts& k, bool need_partials) {
   R* a = static_cast<R*>(b->arena);
-  // (one launch for all boxes: the fill of one whose ghosts are current changes
-  // nothing, and a launch for each box is 2.7 us, 2.7 of the 38 ms of 40
-  // steps over 8 fine boxes, which are filled before every substep)
-  bool fill = !b->pool;
-  for (int i : b->active) {
-    fill = fill || b->slots[i].needs_bc;
-    b->slots[i].needs_bc = false;
+  // (One launch: one for each box is 2.7 us, 2.7 of the 38 ms of 40 steps over 8
+  // fine boxes, which are filled before every substep.  It names up to kFillRuns
+  // boxes; with more it fills all, which changes nothing where the ghosts are
+  // current but takes 62 us for 200 boxes of 24^3.)
+  FillPlan plan{};
+  int need = 0;
+  const size_t seg0 = b->hsegs.size() - b->active.size();  // the boxes' ghost segments
+  for (size_t i = 0; i < b->active.size(); ++i) {
+    Slot& S = b->slots[b->active[i]];
+    if (b->pool && !S.needs_bc) continue;
+    S.needs_bc = false;
+    if (need < kFillRuns) {
+      const BSeg& g = b->hsegs[seg0 + i];
+      plan.first[need] = g.start;
+      plan.before[need + 1] = plan.before[need] + (int32_t)cdiv(g.threads, b->block);
+    }
+    ++need;
   }
-  if (fill)
-    hipLaunchKernelGGL((batch_bc_kernel<ND, R>), dim3(persistent_grid(b, b->nbc_tiles)),
-                       dim3(b->block), 0, b->stream, b->dboxes, b->dsegs, b->dtile_seg,
-                       b->nflux_tiles + b->nupd_tiles, b->nbc_tiles, a, b->inflow, b->ncmp);
+  plan.nruns = need;
+  if (need > kFillRuns) {
+    plan.nruns = 1;
+    plan.first[0] = b->nflux_tiles + b->nupd_tiles;
+    plan.before[1] = b->nbc_tiles;
+  }
+  if (need > 0)
+    hipLaunchKernelGGL((batch_bc_kernel<ND, R>),
+                       dim3(persistent_grid(b, plan.before[plan.nruns])), dim3(b->block), 0,
+                       b->stream, b->dboxes, b->dsegs, b->dtile_seg, plan, a, b->inflow, b->ncmp);
   if (need_partials && (!b->pool || !b->partials_valid)) {
     const unsigned g = persistent_grid(b, b->nupd_tiles);
     hipLaunchKernelGGL((batch_cfl_kernel<ND, R>), dim3(g), dim3(b->block), 0, b->stream, k,
