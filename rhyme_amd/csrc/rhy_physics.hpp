@@ -329,9 +329,10 @@ __device__ __forceinline__ double slope_of(int type, double dL, double dR) {
   const int t = LIM ? LIM : type;
   const double a = fabs(dL), b = fabs(dR);
   if (!((dL > 0.0 && dR > 0.0) || (dL < 0.0 && dR < 0.0))) return 0.0;
-  if (b < kTiny) return 0.0;
-  if (t == 1) return a > b ? dR : dL;
-  if (a > b) return dR;
+  if (__builtin_amdgcn_class(dR, 0x294)) return 0.0;  // denormal, or r = dL / inf
+  const double hi = __builtin_fma(0.0, dL, dR);  // dR; for an infinite dL no number, as xi_R d
+  if (t == 1) return a > b ? hi : dL;
+  if (a > b) return hi;
   const double d = .5 * (dL + dR);
   switch (t) {
     case 2:
