@@ -20,6 +20,13 @@ namespace rhy {
 
 constexpr double kTiny = 2.2250738585072014e-308;  // tiny(0d0)
 
+// Build option RHY_FP64_POW_FAST=0: the FP64 walks evaluate the reference's
+// expressions operation for operation, with IEEE quotients and libm's pow, as the
+// unit-level kernels do: last-bit agreement with a host of the same libm.
+#ifndef RHY_FP64_POW_FAST
+#define RHY_FP64_POW_FAST 1
+#endif
+
 // Problem constants that the reference keeps in module-private globals
 // (rhyme_riemann_problem.f90:11-16, rhyme_irs.f90:9-14,
 // rhyme_thermo_base.f90:25-26) and derived-type defaults.
@@ -356,7 +363,7 @@ template <int ND, int A, int LIM = 0, typename R = double>
 __device__ __forceinline__ void half_step(const Consts& k, const R* um, const R* u, const R* up,
                                           R hdtdx, R* l, R* r, int type = 0) {
   constexpr int NV = ND + 2;
-  constexpr bool kF64 = sizeof(R) == sizeof(double);
+  constexpr bool kF64 = sizeof(R) == sizeof(double) && RHY_FP64_POW_FAST;
   R fl[NV], fr[NV];
   const R w = R(k.omega);
   if (kF64 && w == R(0)) {
@@ -532,11 +539,8 @@ struct MixedMath : PowFast {
   }
 };
 
-// Exponentials of the FP64 path: PowFast unless RHY_FP64_POW_FAST=0 selects
-// libm pow (last-bit agreement with a libm host, ~20% slower flux kernels).
-#ifndef RHY_FP64_POW_FAST
-#define RHY_FP64_POW_FAST 1
-#endif
+// Exponentials of the FP64 path: PowFast, or with RHY_FP64_POW_FAST=0
+// libm pow.
 #if RHY_FP64_POW_FAST
 using PowF64 = PowFast;
 #else
@@ -1267,7 +1271,12 @@ __device__ __forceinline__ void riemann_state(const Consts& k, const double* l, 
 // and the sampling, which round to those same FP32 states.
 template <int ND, int A, class PW, typename R>
 __device__ __forceinline__ void riemann_flux(const Consts& k, const R* l, const R* r, R* F) {
-  if constexpr (sizeof(R) == sizeof(double)) {
+  if constexpr (sizeof(R) == sizeof(double) && !RHY_FP64_POW_FAST) {
+    double rho, v[ND], p, u[ND + 2];
+    riemann_sample_ref<ND, A, PW, double>(k, l, r, 0.0, rho, v, p);
+    prim_to_cons<ND, double>(k, rho, v, p, u);
+    flux<ND, A, double>(k, u, F);
+  } else if constexpr (sizeof(R) == sizeof(double)) {
     double rho, v[ND], p;
     riemann_sample<ND, A, PW>(k, l, r, rho, v, p);
     if (fabs(rho) < kTiny) {
