@@ -90,7 +90,8 @@ struct rhy_box {
   bool planes = false;            // rhy_run steps through the flux planes (choose_walks)
   int32_t partial_cap = 0;
   double* host_max = nullptr;     // pinned: the wave speed of rhy_cfl_time_step (lazy)
-  double* scalars = nullptr;      // [16..16+6*RHY_MAX_CMP) inflow states
+  double* scalars = nullptr;      // [0] the wave speed without host_max, [8..14] step
+                                  // constants, [16..16+6*RHY_MAX_CMP) inflow states
   double inflow_copied[6 * RHY_MAX_CMP] = {};  // what the device inflow slots hold
   bool inflow_valid = false;
   double* dt = nullptr;           // current dt
@@ -1150,19 +1151,22 @@ int rhy_cfl_time_step(rhy_box_t* b, const rhy_params_t* p, const double dx[3], d
   else if (b->ndim == 2) rc = launch_cfl<2>(b, k);
   else rc = launch_cfl<3>(b, k);
   if (rc) return rc;
-  // the speed goes straight to host memory: a copy of 8 bytes is a launch of
-  // its own
+  // the speed goes straight to pinned memory, where there is any: a copy of 8
+  // bytes is a launch of its own
   if (!b->host_max &&
       hipHostMalloc(reinterpret_cast<void**>(&b->host_max), sizeof(double)) != hipSuccess) {
     (void)hipGetLastError();
     b->host_max = nullptr;
-    return fail(RHY_ERR_OOM, "host memory for the wave speed");
   }
   hipLaunchKernelGGL(dt_kernel, dim3(1), dim3(1024), 0, b->stream, b->partial, b->partial_n, 0.0,
-                     (double*)nullptr, (double*)nullptr, b->host_max);
+                     (double*)nullptr, (double*)nullptr, b->host_max ? b->host_max : b->scalars);
   HIP_TRY(hipGetLastError());
+  double maxu = 0.0;
+  if (!b->host_max)
+    HIP_TRY(hipMemcpyAsync(&maxu, b->scalars, sizeof(maxu), hipMemcpyDeviceToHost, b->stream));
   HIP_TRY(hipStreamSynchronize(b->stream));
-  *dt = p->courant * min_dx(b->ndim, dx) / *b->host_max;
+  if (b->host_max) maxu = *b->host_max;
+  *dt = p->courant * min_dx(b->ndim, dx) / maxu;
   return RHY_OK;
 }
 
