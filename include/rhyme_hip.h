@@ -199,10 +199,10 @@ int rhy_box_last_dts(rhy_box_t *box, int32_t n, double *dts);
  * rhy_run / rhy_run_async call with s % N == 0 (step 0, N, 2N, ...) and of
  * nothing else, so that the events (a few microseconds each) perturb only
  * the sampled steps; on = 0: off.  rhy_box_kernel_stats returns, for kernel
- * index kidx (0: the flux kernels, 1: update, 2: bc, 3: cfl, 4: dt, 5: the
- * deferred-face list reset and fixup), the number of launches timed (0: of
- * axis walks; a kernel that walks two axes counts as two) and their summed
- * milliseconds.  RHY_ERR_ARG for on < 0. */
+ * index kidx (0: the flux kernels, 1: update, 2: bc, 3: cfl, 4: dt and the
+ * reset of the deferred-face list, 5: the fixup of deferred faces), the number
+ * of launches timed (0: of axis walks; a kernel that walks two axes counts as
+ * two) and their summed milliseconds.  RHY_ERR_ARG for on < 0. */
 int rhy_box_set_profiling(rhy_box_t *box, int32_t on);
 int rhy_box_kernel_stats(rhy_box_t *box, int32_t kidx, int64_t *launches,
                          double *total_ms);

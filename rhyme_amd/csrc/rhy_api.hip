@@ -284,7 +284,7 @@ void launch_flux_r(rhy_box* b, const Consts& k, const double* dx) {
     timed_begin(b, 5, tf);
     hipLaunchKernelGGL((flux_fixup_kernel<ND, R, P>), dim3(kFixupBlocks), dim3(kThreads), 0,
                        b->stream, k, b->geom, static_cast<const R*>(b->cells),
-                       static_cast<R*>(b->flux), b->dt, dx[0], dx[1], dx[2], dl, -1);
+                       static_cast<R*>(b->flux), b->dt, dx[0], dx[1], dx[2], dl);
     timed_end(b, tf);
   }
 }

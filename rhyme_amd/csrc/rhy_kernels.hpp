@@ -18,7 +18,7 @@
 // 4 -> 128, 3 -> 168, 2 -> 256); 0 leaves the choice to the compiler, which
 // can exceed 256 registers with AGPRs and drop to one wave per SIMD.  With
 // the slow paths of the Riemann solve deferred to the fixup kernel the flux
-// kernels need 145-167 VGPRs, so 3 waves fit without spills.
+// kernels need 145-168 VGPRs, so 3 waves fit without spills where it is hot.
 #ifndef RHY_FLUX_WPE
 #define RHY_FLUX_WPE 3
 #endif
@@ -304,11 +304,12 @@ __device__ __forceinline__ double lane_below(double x) {
 
 // The Consts a kernel was launched with (its first parameter), read from the
 // kernel's arguments where they are used.  Held in scalar registers across a
-// walk, their 60 registers beside the masks of the Riemann solve were spilled
+// walk, their 42 registers beside the masks of the Riemann solve were spilled
 // to vector lanes: 420 v_readlane in walk_xy, one VALU instruction in ten of a
 // moving gas, and 4 to 13 vector registers to memory, whose reloads wait for
-// the walk's stores.  The scalar loads hit the scalar cache; the empty asm
-// keeps them from being moved out of the walk's loop.
+// the walk's stores (now some 16 v_readlane, and spills in the exp and log of
+// other gammas than 5/3, 7/5 and 4/3 only).  The scalar loads hit the scalar
+// cache; the empty asm keeps them from being moved out of the walk's loop.
 __device__ __forceinline__ const Consts& kernel_consts() {
   typedef const __attribute__((address_space(4))) Consts* Args;
   Args p = (Args)__builtin_amdgcn_kernarg_segment_ptr();
@@ -1056,7 +1057,7 @@ __global__ __launch_bounds__(256) void flux_fixup_kernel(Consts k, Geom G,
                                                          R* __restrict__ F,
                                                          const double* __restrict__ dtp,
                                                          double dx0, double dx1, double dx2,
-                                                         DeferList dl, int axis_only) {
+                                                         DeferList dl) {
   const uint32_t n = *dl.count;
   if (n == 0) return;
   const double dt = *dtp;
@@ -1072,7 +1073,6 @@ __global__ __launch_bounds__(256) void flux_fixup_kernel(Consts k, Geom G,
     return;
   }
   for (int a = 0; a < ND; ++a) {
-    if (axis_only >= 0 && a != axis_only) continue;
     const int64_t na = faces_of_axis(G, a);
     for (int64_t q = t0; q < na; q += stride)
       flux_face_fix<ND, R, PW>(k, G, cells, F, dt, dx, a, face_low_cell(G, a, q));

@@ -3,11 +3,13 @@
 // iterative Riemann solver, all evaluated per lane in registers.
 //
 // Arithmetic order is part of the contract: the file must be compiled with
-// -ffp-contract=off, and each expression keeps the parse of the reference
-// Fortran routine it restates (cited file:line, relative to the reference's
-// src/), so that FP64 results agree with the reference CPU path to rounding
-// of pow() only.  Division and sqrt of doubles are IEEE correctly rounded on
-// gfx950 under the default (non fast-math) lowering.
+// -ffp-contract=off.  The unit-level kernels, and with RHY_FP64_POW_FAST=0 the
+// walks, keep the parse of the reference Fortran routine each expression restates
+// (cited file:line, relative to the reference's src/), with IEEE division and
+// sqrt (gfx950's default, non fast-math, lowering), so that they agree with the
+// reference CPU path to rounding of pow() only.  The FP64 walks of the default
+// build evaluate the same formulas with shared reciprocals and roots, each good
+// to an ulp ("FP64 arithmetic of the walks" below).
 //
 // Template parameter ND is the box dimensionality (1, 2, 3); a state vector
 // holds NV = ND + 2 conserved values: rho, rho*v[0..ND), e_tot.
@@ -58,9 +60,9 @@ __device__ __forceinline__ double tiny_of<double>() { return kTiny; }
 template <>
 __device__ __forceinline__ float tiny_of<float>() { return 1.17549435e-38f; }
 
-// a / b and sqrt in the bulk type: IEEE for double (the FP64 path, whose
-// results match the oracle bit for bit), hardware reciprocal times a and
-// hardware square root for float (the mixed form; <= 1.5 ulp).
+// a / b and sqrt in the bulk type: IEEE for double (the unit-level FP64
+// kernels), hardware reciprocal times a and hardware square root for float (the
+// mixed form; <= 1.5 ulp).
 template <typename R>
 __device__ __forceinline__ R rdiv(R a, R b);
 template <>
@@ -982,9 +984,10 @@ __device__ __forceinline__ void riemann_sample_ref(const Consts& k, const RI* l,
 //   * the two-rarefaction guess needs one of its two equal terms
 //     p_K x_K^(1/z), and quotients over one divisor share its reciprocal.
 //
-// Returns false where the reference leaves this path (vacuum generated, a
-// Newton iterate below zero, a state out of range): the caller then takes
-// riemann_sample_ref, or defers the face to the fixup kernel, which does.
+// The sound speeds are the states' own; the pressures may be w_vacuum's, the
+// floor (side_prims).  Returns false where the reference leaves this path (vacuum
+// generated, a Newton iterate below zero, a state out of range): the caller then
+// takes riemann_sample_ref, or defers the face to the fixup kernel, which does.
 
 // b^5, b^7 or b^8
 __device__ __forceinline__ double pow_n(int n, double b) {
@@ -993,8 +996,9 @@ __device__ __forceinline__ double pow_n(int n, double b) {
 }
 
 // x^z, z = (gamma-1)/2gamma, x > 0.  n = 1/z: y0 = x^(1/n) in FP32 (relative
-// error 2^-22), then Halley's y = y0 + 2 y0 (x - y0^n) / ((n+1) y0^n + (n-1) x),
-// whose error is of order y0's cubed.
+// error 2^-22 near x = 1, 2^-19 towards 2^-100 and 2^100, where the logarithm's
+// own rounding is 2^-18), then Halley's y = y0 + 2 y0 (x - y0^n) / ((n+1) y0^n +
+// (n-1) x), whose relative error is (n^2-1)/12 times y0's cubed, 2^-54 at most.
 __device__ __forceinline__ double root_z(const Consts& k, double x) {
   if (k.nroot > 0 && x > 0x1p-100 && x < 0x1p100) {
     const float e = __builtin_amdgcn_logf((float)x) * (float)k.gm1_2g;
