@@ -144,9 +144,7 @@ __global__ __launch_bounds__(256) void batch_fixup_kernel(Consts k, const BBox* 
       const uint64_t it = dl.items[i];
       const int32_t bx = (int32_t)(it >> 42);
       const BBox& B = boxes[bx];
-      Consts kb = k;
-      kb.limiter = B.limiter;
-      flux_face_fix<ND, R, PW>(kb, B.G, arena + B.cell_off, arena + B.flux_off, dt[bx], B.dx,
+      flux_face_fix<ND, R, PW>(&kernel_consts(), B.limiter, B.G, arena + B.cell_off, arena + B.flux_off, dt[bx], B.dx,
                                (int)((it >> 40) & 3), (int64_t)(it & ((1ull << 40) - 1)));
     }
     return;
@@ -154,12 +152,10 @@ __global__ __launch_bounds__(256) void batch_fixup_kernel(Consts k, const BBox* 
   for (int32_t ai = 0; ai < nactive; ++ai) {
     const int32_t bx = active[ai];
     const BBox& B = boxes[bx];
-    Consts kb = k;
-    kb.limiter = B.limiter;
     for (int a = 0; a < ND; ++a) {
       const int64_t na = faces_of_axis(B.G, a);
       for (int64_t q = t0; q < na; q += stride)
-        flux_face_fix<ND, R, PW>(kb, B.G, arena + B.cell_off, arena + B.flux_off, dt[bx], B.dx,
+        flux_face_fix<ND, R, PW>(&kernel_consts(), B.limiter, B.G, arena + B.cell_off, arena + B.flux_off, dt[bx], B.dx,
                                  a, face_low_cell(B.G, a, q));
     }
   }
@@ -633,12 +629,13 @@ __global__ __launch_bounds__(256) void amr_register_kernel(const AmrItem* __rest
 // axis FROM_STATE after rhy_amr_coarse_step, formed from the pre-step
 // state `prev` with policy P, the step's constants k, dt and dx.
 template <int ND, typename R, int FROM_STATE = -1, class P = PowF64Fix>
-__global__ __launch_bounds__(256) void amr_reflux_kernel(const AmrItem* __restrict__ items,
+__global__ __launch_bounds__(256) void amr_reflux_kernel(Consts k,
+                                                         const AmrItem* __restrict__ items,
                                                          int nitems, int64_t total, int64_t base,
                                                          const double* __restrict__ reg,
                                                          Geom GC, R* __restrict__ coarse,
                                                          const R* __restrict__ cflux,
-                                                         double dtdx, Consts k = Consts{},
+                                                         double dtdx,
                                                          const R* __restrict__ prev = nullptr,
                                                          double dt = 0.0, double dx = 1.0) {
   const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -665,7 +662,8 @@ __global__ __launch_bounds__(256) void amr_reflux_kernel(const AmrItem* __restri
   if constexpr (FROM_STATE >= 0) {
     // the coarse face's flux formed again from the state the coarse step
     // started from, as the step's walk formed it
-    face_flux<ND, FROM_STATE, R, P>(k, GC, prev, dt, dx, ol, Fs);
+    face_flux<ND, FROM_STATE, R, P>(&kernel_consts(), kernel_consts().limiter, GC, prev, dt, dx, ol,
+                                    Fs);
   }
 #pragma unroll
   for (int c = 0; c < ND + 2; ++c) {
@@ -1997,13 +1995,14 @@ static int amr_reflux_v(const BoxView& vc, rhy_batch_t* f, const int32_t* lo, do
     const int a = pass / 2;
 #define RHY_REFLUX(ND, R)                                                                       \
   hipLaunchKernelGGL((amr_reflux_kernel<ND, R>), dim3(cdiv(f->reg_pt[pass], 256)), dim3(256), 0, \
-                     f->stream, items, ni, f->reg_pt[pass], base, f->amr_reg, vc.geom,         \
+                     f->stream, vc.k, items, ni, f->reg_pt[pass], base, f->amr_reg, vc.geom,         \
                      static_cast<R*>(vc.cells), static_cast<const R*>(vc.flux), dtdx)
 #define RHY_REFLUX_S(ND, A, R, P)                                                               \
   hipLaunchKernelGGL((amr_reflux_kernel<ND, R, A, P>), dim3(cdiv(f->reg_pt[pass], 256)),       \
-                     dim3(256), 0, f->stream, items, ni, f->reg_pt[pass], base, f->amr_reg,    \
-                     vc.geom, static_cast<R*>(vc.cells), static_cast<const R*>(vc.flux), dtdx, \
-                     vc.k, static_cast<const R*>(vc.prev), vc.step_dt, vc.step_dx[a])
+                     dim3(256), 0, f->stream, vc.k, items, ni, f->reg_pt[pass], base,          \
+                     f->amr_reg, vc.geom, static_cast<R*>(vc.cells),                           \
+                     static_cast<const R*>(vc.flux), dtdx, static_cast<const R*>(vc.prev),     \
+                     vc.step_dt, vc.step_dx[a])
     if (vc.prev) {  // coarse fluxes of an accumulating coarse step
       if (f->precision == RHY_MIXED) {
         if (nd == 2) {

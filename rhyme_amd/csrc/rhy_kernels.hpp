@@ -317,6 +317,15 @@ __device__ __forceinline__ const Consts& kernel_consts() {
   return *(const Consts*)p;
 }
 
+// The same from its address, the same on every lane, in a function of its own.
+__device__ __forceinline__ const Consts& uniform_consts(const Consts* args) {
+  typedef const __attribute__((address_space(4))) Consts* Args;
+  const uint64_t a = (uint64_t)args;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return *(const Consts*)(Args)((uint64_t)hi << 32 | lo);
+}
+
 // Intercell flux on every face normal to axis A that the interior update
 // reads: face f in [0, n_A] sits between cells f and f+1, the other indices
 // run over the interior (the faces-only range the update consumes,
@@ -987,31 +996,34 @@ inline int even_length(int n, int L) {
 // stencil of four cells along A) and the Riemann solve with policy PW, the
 // computation the flux walks make for it.  of: offset of the low cell.
 // (Out of line: its callers are the fixup and reflux kernels, which hold
-// several of these calls and run on few faces.)
+// several of these calls and run on few faces.  args: the kernel's constants,
+// read where they lie by scalar loads; a reference to a kernel's copy would have
+// it copied to private memory.  type: the limiter.)
 template <int ND, int A, typename R, class PW>
-__device__ __noinline__ void face_flux(const Consts& k, const Geom& G,
-                                          const R* __restrict__ cells, double dt, double dx,
-                                          int64_t of, R* Fr) {
+__device__ __noinline__ void face_flux(const Consts* args, int type, const Geom& G,
+                                       const R* __restrict__ cells, double dt, double dx,
+                                       int64_t of, R* Fr) {
   constexpr int NV = ND + 2;
+  const Consts& k = uniform_consts(args);
   const int64_t s = G.s[A];
   const R hdtdx = (R)(.5 * dt / dx);
   R um[NV], u0[NV], up[NV], l0[NV], r0[NV], l1[NV], r1[NV];
   load_state<ND, R>(cells, G.plane, of - s, um);
   load_state<ND, R>(cells, G.plane, of, u0);
   load_state<ND, R>(cells, G.plane, of + s, up);
-  half_step<ND, A, 0, R>(k, um, u0, up, hdtdx, l0, r0, k.limiter);
+  half_step<ND, A, 0, R>(k, um, u0, up, hdtdx, l0, r0, type);
   load_state<ND, R>(cells, G.plane, of + 2 * s, um);
-  half_step<ND, A, 0, R>(k, u0, up, um, hdtdx, l1, r1, k.limiter);
+  half_step<ND, A, 0, R>(k, u0, up, um, hdtdx, l1, r1, type);
   riemann_flux<ND, A, PW, R>(k, r0, l1, Fr);
 }
 
 template <int ND, int A, typename R, class PW>
-__device__ __forceinline__ void flux_one_face(const Consts& k, const Geom& G,
+__device__ __forceinline__ void flux_one_face(const Consts* k, int type, const Geom& G,
                                               const R* __restrict__ cells, R* __restrict__ FA,
                                               double dt, double dx, int64_t of) {
   constexpr int NV = ND + 2;
   R Fr[NV];
-  face_flux<ND, A, R, PW>(k, G, cells, dt, dx, of, Fr);
+  face_flux<ND, A, R, PW>(k, type, G, cells, dt, dx, of, Fr);
 #pragma unroll
   for (int c = 0; c < NV; ++c) FA[of + c * G.plane] = Fr[c];
 }
@@ -1019,15 +1031,15 @@ __device__ __forceinline__ void flux_one_face(const Consts& k, const Geom& G,
 // The same for a face given by axis at run time; F holds the NDIM flux
 // plane sets of the box one after the other.
 template <int ND, typename R, class PW>
-__device__ __noinline__ void flux_face_fix(const Consts& k, const Geom& G,
-                                           const R* __restrict__ cells, R* __restrict__ F,
-                                           double dt, const double* dx, int a, int64_t of) {
+__device__ __forceinline__ void flux_face_fix(const Consts* k, int type, const Geom& G,
+                                              const R* __restrict__ cells, R* __restrict__ F,
+                                              double dt, const double* dx, int a, int64_t of) {
   R* FA = F + (int64_t)a * (ND + 2) * G.plane;
-  if (a == 0) flux_one_face<ND, 0, R, PW>(k, G, cells, FA, dt, dx[0], of);
+  if (a == 0) flux_one_face<ND, 0, R, PW>(k, type, G, cells, FA, dt, dx[0], of);
   if constexpr (ND > 1)
-    if (a == 1) flux_one_face<ND, 1, R, PW>(k, G, cells, FA, dt, dx[1], of);
+    if (a == 1) flux_one_face<ND, 1, R, PW>(k, type, G, cells, FA, dt, dx[1], of);
   if constexpr (ND > 2)
-    if (a == 2) flux_one_face<ND, 2, R, PW>(k, G, cells, FA, dt, dx[2], of);
+    if (a == 2) flux_one_face<ND, 2, R, PW>(k, type, G, cells, FA, dt, dx[2], of);
 }
 
 // Number of faces of axis a that a step computes, and the low cell of the
@@ -1067,7 +1079,7 @@ __global__ __launch_bounds__(256) void flux_fixup_kernel(Consts k, Geom G,
   if (n <= dl.cap) {
     for (int64_t i = t0; i < (int64_t)n; i += stride) {
       const uint64_t it = dl.items[i];
-      flux_face_fix<ND, R, PW>(k, G, cells, F, dt, dx, (int)((it >> 40) & 3),
+      flux_face_fix<ND, R, PW>(&kernel_consts(), kernel_consts().limiter, G, cells, F, dt, dx, (int)((it >> 40) & 3),
                                (int64_t)(it & ((1ull << 40) - 1)));
     }
     return;
@@ -1075,7 +1087,7 @@ __global__ __launch_bounds__(256) void flux_fixup_kernel(Consts k, Geom G,
   for (int a = 0; a < ND; ++a) {
     const int64_t na = faces_of_axis(G, a);
     for (int64_t q = t0; q < na; q += stride)
-      flux_face_fix<ND, R, PW>(k, G, cells, F, dt, dx, a, face_low_cell(G, a, q));
+      flux_face_fix<ND, R, PW>(&kernel_consts(), kernel_consts().limiter, G, cells, F, dt, dx, a, face_low_cell(G, a, q));
   }
 }
 
@@ -1089,7 +1101,7 @@ __global__ __launch_bounds__(256) void flux_fixup_kernel(Consts k, Geom G,
 constexpr int kFixXy3 = 0, kFixXy2 = 1, kFixZ = 2;
 
 template <int WALK, typename R, class PW>
-__device__ __forceinline__ void acc_fix_cell(const Consts& k, const Geom& G,
+__device__ __forceinline__ void acc_fix_cell(const Consts* k, int type, const Geom& G,
                                              const R* __restrict__ cells,
                                              const R* __restrict__ acc, R* __restrict__ out,
                                              double dt, double dx0, double dx1, double dx2,
@@ -1107,21 +1119,21 @@ __device__ __forceinline__ void acc_fix_cell(const Consts& k, const Geom& G,
   R fl[NV], fu[NV], uc[NV], un[NV];
   load_state<ND, R>(cells, G.plane, oc, uc);
   if constexpr (WALK == kFixZ) {
-    face_flux<3, 2, R, PW>(k, G, cells, dt, dx2, oc - G.s[2], fl);
-    face_flux<3, 2, R, PW>(k, G, cells, dt, dx2, oc, fu);
+    face_flux<3, 2, R, PW>(k, type, G, cells, dt, dx2, oc - G.s[2], fl);
+    face_flux<3, 2, R, PW>(k, type, G, cells, dt, dx2, oc, fu);
     const R dtdx2 = (R)(dt / dx2);
 #pragma unroll
     for (int c = 0; c < NV; ++c)
       un[c] = acc_z<R>(uc[c], acc[oc + c * G.plane], dtdx2 * (fl[c] - fu[c]), order);
   } else {
     R a0[NV];
-    face_flux<ND, 0, R, PW>(k, G, cells, dt, dx0, oc - G.s[0], fl);
-    face_flux<ND, 0, R, PW>(k, G, cells, dt, dx0, oc, fu);
+    face_flux<ND, 0, R, PW>(k, type, G, cells, dt, dx0, oc - G.s[0], fl);
+    face_flux<ND, 0, R, PW>(k, type, G, cells, dt, dx0, oc, fu);
     const R dtdx0 = (R)(dt / dx0), dtdx1 = (R)(dt / dx1);
 #pragma unroll
     for (int c = 0; c < NV; ++c) a0[c] = dtdx0 * (fl[c] - fu[c]);
-    face_flux<ND, 1, R, PW>(k, G, cells, dt, dx1, oc - G.s[1], fl);
-    face_flux<ND, 1, R, PW>(k, G, cells, dt, dx1, oc, fu);
+    face_flux<ND, 1, R, PW>(k, type, G, cells, dt, dx1, oc - G.s[1], fl);
+    face_flux<ND, 1, R, PW>(k, type, G, cells, dt, dx1, oc, fu);
 #pragma unroll
     for (int c = 0; c < NV; ++c)
       un[c] = acc_xy<R, WALK == kFixXy3 ? kAccMid : kAccLast>(uc[c], a0[c],
@@ -1133,7 +1145,7 @@ __device__ __forceinline__ void acc_fix_cell(const Consts& k, const Geom& G,
     double ud[NV];
 #pragma unroll
     for (int c = 0; c < NV; ++c) ud[c] = (double)un[c];
-    const double sp = cfl_speed<ND>(k, ud);
+    const double sp = cfl_speed<ND>(*k, ud);
     if (sp > 0.0)
       atomicMax(reinterpret_cast<unsigned long long*>(slot),
                 (unsigned long long)__double_as_longlong(sp));
@@ -1162,7 +1174,8 @@ __global__ __launch_bounds__(256) void acc_fixup_kernel(
       const int64_t r = i / G.n[0];
       oc = goff(G, (int)(i % G.n[0]) + 1, (int)(r % G.n[1]) + 1, (int)(r / G.n[1]) + 1);
     }
-    acc_fix_cell<WALK, R, PW>(k, G, cells, acc, out, dt, dx0, dx1, dx2, order, oc, slot);
+    acc_fix_cell<WALK, R, PW>(&kernel_consts(), kernel_consts().limiter, G, cells, acc, out, dt, dx0,
+                              dx1, dx2, order, oc, slot);
   }
 }
 
