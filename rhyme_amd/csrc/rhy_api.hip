@@ -491,7 +491,7 @@ int launch_acc_step(rhy_box* b, const Consts& k, const double* dx,
   if (b->precision == RHY_MIXED)
     launch_acc_step_r<ND, float, MixedFlux, MixedMath>(b, k, dx, order);
   else
-    launch_acc_step_r<ND, double, PowF64Flux, PowF64Fix>(b, k, dx, order);
+    launch_acc_step_r<ND, double, PowF64Walk, PowF64Fix>(b, k, dx, order);
   HIP_TRY(hipGetLastError());
   return RHY_OK;
 }

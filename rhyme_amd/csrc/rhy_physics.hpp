@@ -430,7 +430,7 @@ struct PowLib {
 struct PowFast {
   static constexpr bool kFast = false;
   static constexpr bool kStar = true;
-  static constexpr bool kVacuum = true;
+  static constexpr int kVacuum = 1;  // kVacuumHere
   static constexpr bool kDefer = false;
   __device__ __forceinline__ static double dv(double a, double b) { return a / b; }
   __device__ __forceinline__ static double sq(double x) { return sqrt(x); }
@@ -562,12 +562,20 @@ using PowF64 = PowLib;
 // The flag is one LDS word per lane (a lane only touches its own word), so
 // policies need no state; kernels using it have at most LANES threads per
 // workgroup and clear the flag when they start.
-template <class P, int LANES = 256>
+//
+// VACUUM: where gas beside a vacuum is answered (beside_vacuum).
+//   kVacuumHere   in the flux-plane kernels, in the registers they have left;
+//   kVacuumAside  in the accumulating walks, whose fixup would solve four faces
+//                 for each: its answer waits in private memory meanwhile (in
+//                 registers 256^3 971 -> 1123 us, so 971 -> 970);
+//   kVacuumLater  by the fixup: in the batches' kernel, which either way would
+//                 spill 16 to 22 registers (40 boxes, 40 steps: 14.0 -> 14.4 ms),
+//                 and in tube_run, which takes P on the spot.
+enum { kVacuumLater = 0, kVacuumHere = 1, kVacuumAside = 2 };
+template <class P, int LANES = 256, int VACUUM = kVacuumHere>
 struct Deferring : P {
   static constexpr bool kDefer = true;
-  // gas beside a vacuum in the walk; left to P in tube_run, which takes P on the
-  // spot (1024 cells at gamma 1.45: 19.6 us a step, 21.9 with it)
-  static constexpr bool kVacuum = LANES == 256;
+  static constexpr int kVacuum = VACUUM;
   __device__ __forceinline__ static uint32_t& flag() {
     __shared__ uint32_t flags[LANES];
     return flags[threadIdx.x];
@@ -604,7 +612,8 @@ struct Deferring : P {
   }
 };
 
-// Policies of the flux kernels and of their fixup kernels.
+// Policies of the flux kernels, the accumulating walks, the batches' flux kernel
+// and the fixup kernels.
 // Build option RHY_FP64_FAST_RIEMANN=1: the FP64 flux kernels solve their
 // Riemann problems with the mixed form's FP64 policy (refined reciprocal
 // division and square root, the algebraic wave-function forms): about 4%
@@ -620,20 +629,28 @@ struct Deferring : P {
 #endif
 #if RHY_FP64_FAST_RIEMANN
 using PowF64Flux = Deferring<MixedMath>;
+using PowF64Walk = PowF64Flux;
+using PowF64Batch = PowF64Flux;
 using PowF64Fix = MixedMath;
 #elif RHY_FP64_POW_FAST
 using PowF64Flux = Deferring<PowFast>;
+using PowF64Walk = Deferring<PowFast, 256, kVacuumAside>;
+using PowF64Batch = Deferring<PowFast, 256, kVacuumLater>;
 using PowF64Fix = PowFast;
 #else
 using PowF64Flux = PowLib;
+using PowF64Walk = PowLib;
+using PowF64Batch = PowLib;
 using PowF64Fix = PowLib;
 #endif
 using MixedFlux = Deferring<MixedMath>;
-// the same with more lanes to a workgroup
+// tube_run's: the same with more lanes to a workgroup
 template <class PW, int LANES>
 struct WithLanes { using type = PW; };
-template <class P, int N, int LANES>
-struct WithLanes<Deferring<P, N>, LANES> { using type = Deferring<P, LANES>; };
+template <class P, int N, int V, int LANES>
+struct WithLanes<Deferring<P, N, V>, LANES> {
+  using type = Deferring<P, LANES, kVacuumLater>;
+};
 
 // rhyme_irs_nonlinear_wave_function.f90:13-23.  The terms that do not
 // depend on p (A_K, B_K of the shock branch, 2 c_K / (gamma-1) and
@@ -1126,6 +1143,12 @@ __device__ __forceinline__ bool star_sample(const Consts& k, double lr, const do
   return true;
 }
 
+// Values kept across the star state's solve: in registers, or (kVacuumAside) not.
+template <int V>
+struct Stash { using type = double; };
+template <>
+struct Stash<2> { using type = volatile double; };
+
 // Gas u beside a vacuum, on its right (right = true) or left side
 // (rhyme_riemann_problem_solve.f90:37-60, with its own front speeds): the vacuum
 // or the undisturbed gas.  False for states out of plain_range, and inside the
@@ -1168,12 +1191,10 @@ __device__ __forceinline__ void riemann_sample(const Consts& k, const double* l,
     return;
   } else {
     bool ok = plain_range(l[0]) && plain_range(r[0]) && l[0] >= k.e_rho && r[0] >= k.e_rho;
-    // the rare faces first and out of the registers: held in them across the
-    // star state's solve they cost every face 5 to 15% of a step (256^3 971 ->
-    // 1123 us)
+    // the rare faces first (see Deferring)
     const bool gas = ok;
-    constexpr bool kHere = PW::kVacuum;
-    volatile double stash[ND + 2];
+    constexpr bool kHere = PW::kVacuum != 0;  // kVacuumLater
+    typename Stash<PW::kVacuum>::type stash[ND + 2];
     if (kHere && !wave_all(gas)) {
       if (!gas) {
         const bool vl = l[0] < k.e_rho, vr = r[0] < k.e_rho;
