@@ -126,6 +126,11 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void batch_flux_kernel(Cons
   }
 }
 
+// Parts of a batch's list of deferred faces: on one counter their additions take
+// 3.6 ns each, 0.4 ms of a step of 4 half empty boxes of 96^3.
+constexpr int kDeferParts = 32;
+constexpr size_t kDeferBytes = sizeof(uint32_t) * kDeferParts * kDeferGap;
+
 // The faces the flux phase listed, recomputed with the full policy PW
 // (each with its box's limiter, dt and dx); if the list overflowed, every
 // face of every active box.
@@ -135,13 +140,19 @@ __global__ __launch_bounds__(256) void batch_fixup_kernel(Consts k, const BBox* 
                                                           int32_t nactive, R* __restrict__ arena,
                                                           const double* __restrict__ dt,
                                                           DeferList dl) {
-  const uint32_t n = *dl.count;
-  if (n == 0) return;
+  const int lane = (int)(threadIdx.x & 63);
+  const uint32_t n = lane < kDeferParts ? dl.count[lane * kDeferGap] : 0u;
+  if (wave_all(n == 0u)) return;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n <= dl.cap) {
-    for (int64_t i = t0; i < (int64_t)n; i += stride) {
-      const uint64_t it = dl.items[i];
+  if (wave_all(n <= dl.cap)) {
+    // a part's items by every kDeferParts-th workgroup
+    const int part = (int)(blockIdx.x % kDeferParts);
+    const uint32_t np = __builtin_amdgcn_readlane(n, part);
+    const uint64_t* items = dl.items + (size_t)part * dl.cap;
+    for (uint32_t i = blockIdx.x / kDeferParts * blockDim.x + threadIdx.x; i < np;
+         i += gridDim.x / kDeferParts * blockDim.x) {
+      const uint64_t it = items[i];
       const int32_t bx = (int32_t)(it >> 42);
       const BBox& B = boxes[bx];
       flux_face_fix<ND, R, PW>(&kernel_consts(), B.limiter, B.G, arena + B.cell_off, arena + B.flux_off, dt[bx], B.dx,
@@ -342,8 +353,9 @@ __global__ __launch_bounds__(256) void batch_dt_kernel(const BBox* __restrict__ 
     dt[b] = d;
     const int32_t s = *step;
     if (dtlog && s < log_steps) dtlog[(int64_t)s * log_stride + b] = d;
-    if (defer_count && blockIdx.x == 0) *defer_count = 0u;
   }
+  if (defer_count && blockIdx.x == 0 && threadIdx.x < kDeferParts)
+    defer_count[threadIdx.x * kDeferGap] = 0u;
 }
 
 __global__ void batch_set_counter_kernel(int32_t* step, int32_t v) {
@@ -360,8 +372,8 @@ __global__ __launch_bounds__(256) void batch_set_dt_kernel(const int32_t* __rest
                                                            int32_t log_steps, int32_t log_stride,
                                                            uint32_t* __restrict__ defer_count) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < kDeferParts) defer_count[i * kDeferGap] = 0u;
   if (i >= nactive) return;
-  if (i == 0) *defer_count = 0u;
   const int b = active[i];
   dt[b] = value;
   const int32_t s = *step;
@@ -683,6 +695,7 @@ unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
 constexpr int64_t kAlign = 64;  // arena blocks start on 64-element (>= 256 B) boundaries
 constexpr int kFixupBlocks = 256;  // workgroups of the fixup kernel (one per CU)
+static_assert(kFixupBlocks % kDeferParts == 0, "every part of the list has its workgroups");
 
 struct Slot {
   bool active = false;
@@ -726,7 +739,7 @@ struct rhy_batch {
   hipGraphExec_t graph = nullptr;
   uint64_t graph_key = 0;
   DiagPartial* diag = nullptr;  // workgroup partials of rhy_batch_diagnostics
-  uint32_t* defer_count = nullptr;  // faces the flux phase left to the fixup
+  uint32_t* defer_count = nullptr;  // faces the flux phase left to the fixup, by part
   uint64_t* defer_items = nullptr;
   uint32_t defer_cap = 0;
   float* snap = nullptr;  // staging of the FP32 snapshot payload (lazy, grows)
@@ -889,7 +902,9 @@ DeferList defer_list(rhy_batch* b) {
   dl.count = b->defer_count;
   dl.items = b->defer_items;
   const int64_t cap = defer_cap_setting();
-  dl.cap = cap >= 0 ? (uint32_t)std::min<int64_t>(cap, b->defer_cap) : b->defer_cap;
+  const int64_t room = cap >= 0 ? std::min<int64_t>(cap, b->defer_cap) : b->defer_cap;
+  dl.cap = (uint32_t)(room / kDeferParts);
+  dl.last_part = kDeferParts - 1;
   return dl;
 }
 
@@ -1141,9 +1156,9 @@ rhy_batch* new_batch(int32_t ndim, int32_t ncmp, int32_t precision, int64_t aren
   // deferred-face list: about one entry per 64 arena elements, within
   // [4096, 2^20] (the fixup recomputes every face past that)
   b->defer_cap = (uint32_t)std::min<int64_t>(std::max<int64_t>(arena_elems / 64, 4096), 1 << 20);
-  if (dev_alloc(&b->defer_count, sizeof(uint32_t)) != hipSuccess ||
+  if (dev_alloc(&b->defer_count, kDeferBytes) != hipSuccess ||
       dev_alloc(&b->defer_items, sizeof(uint64_t) * (size_t)b->defer_cap) != hipSuccess ||
-      hipMemsetAsync(b->defer_count, 0, sizeof(uint32_t), b->stream) != hipSuccess) {
+      hipMemsetAsync(b->defer_count, 0, kDeferBytes, b->stream) != hipSuccess) {
     rhy_batch_destroy(b);
     *rc = bfail(RHY_ERR_OOM, "deferred-face list allocation failed");
     return nullptr;
@@ -2061,10 +2076,11 @@ int rhy_batch_sync(rhy_batch_t* b) {
 
 int rhy_batch_last_deferred(rhy_batch_t* b, int64_t* n) {
   if (!b || !n) return bfail(RHY_ERR_ARG, "NULL argument");
-  uint32_t c = 0;
+  uint32_t c[kDeferParts * kDeferGap];
   BHIP_TRY(hipStreamSynchronize(b->stream));
-  BHIP_TRY(hipMemcpy(&c, b->defer_count, sizeof(c), hipMemcpyDeviceToHost));
-  *n = c;
+  BHIP_TRY(hipMemcpy(c, b->defer_count, kDeferBytes, hipMemcpyDeviceToHost));
+  *n = 0;
+  for (int i = 0; i < kDeferParts; ++i) *n += c[i * kDeferGap];
   return RHY_OK;
 }
 

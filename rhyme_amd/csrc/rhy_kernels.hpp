@@ -161,11 +161,15 @@ int box_view(rhy_box_t* b, BoxView* v);
 // Faces whose Riemann solve needs a slow path (Deferring<P>), listed by the
 // flux kernels for the fixup kernel: item = box << 42 | axis << 40 | the
 // offset of the face's low cell in its box's planes.  count may pass cap;
-// the fixup then recomputes every face.
+// the fixup then recomputes every face.  A list can be in 2^n parts, which the
+// workgroups take in turn: part i's count in count[i * kDeferGap], its room of cap
+// items from items[i * cap] on.
+constexpr int kDeferGap = 16;  // a cache line
 struct DeferList {
   uint32_t* count;
   uint64_t* items;
   uint32_t cap;
+  uint32_t last_part = 0;
 };
 
 __device__ __forceinline__ uint64_t defer_item(uint32_t box, int axis, int64_t of) {
@@ -183,8 +187,9 @@ __device__ __forceinline__ bool defer_take(const Consts& k, const DeferList& dl,
     if (k.defer_every > 0 && of % k.defer_every == 0) f = 1u;
     if (f) {
       f = 0u;
-      const uint32_t i = atomicAdd(dl.count, 1u);
-      if (i < dl.cap) dl.items[i] = defer_item(box, axis, of);
+      const uint32_t part = blockIdx.x & dl.last_part;
+      const uint32_t i = atomicAdd(dl.count + part * kDeferGap, 1u);
+      if (i < dl.cap) dl.items[(size_t)part * dl.cap + i] = defer_item(box, axis, of);
       return true;
     }
   }

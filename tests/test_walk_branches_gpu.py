@@ -16,7 +16,8 @@ import numpy as np
 import pytest
 
 import oracle
-from rhyme_amd import hydro
+from rhyme_amd import hydro, ics
+from rhyme_amd.batch import SamrBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -181,3 +182,31 @@ def test_vacuum_generated(ndim, axis):
     gamma = 5.0 / 3.0
     row = row_of(gamma, [((1.0, 1.0), (0.8, 0.9), 8.0)])
     step(ndim, axis, row, params(ndim, gamma))
+
+
+@pytest.mark.parametrize("kind", ["vacuum", "floor"])
+@pytest.mark.parametrize("ndim,dims", [(1, [[40], [700]]), (2, [[30, 21], [64, 9]]),
+                                       (3, [[20, 17, 9], [40, 33, 27]])])
+def test_batches_equal_boxes_alone(ndim, dims, kind):
+    """Half empty boxes, and gas under the floor, in a batch (whose kernel leaves
+    vacuum to the fixup, in a list of several parts) and alone."""
+    p = params(ndim, 5.0 / 3.0, w_p=1e-3 if kind == "floor" else 0.0)
+    cells = [ics.random_smooth(ndim, d, seed=8 + i) for i, d in enumerate(dims)]
+    for c, d in zip(cells, dims):
+        if kind == "floor":
+            c[1:ndim + 2] *= 1e-4
+        else:
+            c[..., 2 + d[0] // 2:] = 0.0
+    b = SamrBatch(ndim, dims, [[0.1] * ndim] * len(dims))
+    for i, c in enumerate(cells):
+        b.upload(i, c)
+    dts = b.run(p, 3)
+    assert kind == "floor" or b.last_deferred() > 0
+    for i, (c, d) in enumerate(zip(cells, dims)):
+        box = hydro.SamrBox(ndim, d, cells=c.copy())
+        box.upload()
+        assert np.array_equal(hydro.run(p, box, [0.1] * ndim, 3), dts[:, i])
+        inner = (slice(0, ndim + 2),) + (slice(2, -2),) * ndim
+        assert np.array_equal(box.download()[inner], b.download(i)[inner], equal_nan=True)
+        box.close()
+    b.close()
