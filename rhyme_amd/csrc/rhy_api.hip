@@ -54,6 +54,7 @@ constexpr int kThreads = 256;
 static_assert(kThreads <= kWalkLanes, "the walks' LDS ring has one slot column per thread");
 // workgroups of the fixup kernel (grid-stride over the deferred faces)
 constexpr int kFixupBlocks = 128;
+static_assert(kFixupBlocks % kDeferParts == 0, "every part of a list has its workgroups");
 constexpr int kNumKernelIds = 6;  // flux/step, update, bc, cfl, dt, deferred-face fixup
 
 struct TimedLaunch {
@@ -97,8 +98,9 @@ struct rhy_box {
   double* dt = nullptr;           // current dt
   double* dt_log = nullptr;       // per-step dt of the last run
   void* diag = nullptr;           // workgroup partials of rhy_box_diagnostics
-  uint32_t* defer_count = nullptr;  // faces the flux kernels left to the fixup:
-                                    // [0] or per axis [0..ndim)
+  uint32_t* defer_count = nullptr;  // faces the flux kernels left to the fixup, by
+                                    // part: of the planes or x and y; of z
+  uint32_t defer_parts = kDeferParts;
   uint64_t* defer_items = nullptr;
   uint32_t defer_cap = 0;           // the whole list (one list for every axis)
   uint32_t defer_cap_axis[3] = {0, 0, 0};  // per-axis lists carved from it
@@ -238,14 +240,18 @@ void choose_walks(rhy_box* b) {
         G.n[2], walk_length(G.n[2], 1.0, [&](int L) { return acc_threads(G, 2, L) / 64; }));
 }
 
-DeferList defer_list(rhy_box* b) {
+// List 0 or 1 of deferred faces, with room for that many items from `items` on.
+DeferList defer_list_of(rhy_box* b, int list, uint64_t* items, int64_t room) {
   DeferList dl;
-  dl.count = b->defer_count;
-  dl.items = b->defer_items;
+  dl.count = b->defer_count + list * b->defer_parts * kDeferGap;
+  dl.items = items;
   const int64_t cap = defer_cap_setting();
-  dl.cap = cap >= 0 ? (uint32_t)std::min<int64_t>(cap, b->defer_cap) : b->defer_cap;
+  dl.cap = (uint32_t)((cap >= 0 ? std::min(cap, room) : room) / b->defer_parts);
+  dl.last_part = b->defer_parts - 1;
   return dl;
 }
+
+DeferList defer_list(rhy_box* b) { return defer_list_of(b, 0, b->defer_items, b->defer_cap); }
 
 template <int ND, int LIM, typename R, class PW>
 void launch_flux_lim(rhy_box* b, const Consts& k, const double* dx, const DeferList& dl) {
@@ -409,14 +415,8 @@ double* step_consts(rhy_box* b) { return b->scalars + 8; }
 // The deferred-face lists of the accumulating step: of walk_xy (the x and y
 // axes' parts together) and of the z walk.
 DeferList defer_list_walk(rhy_box* b, bool z) {
-  DeferList dl;
-  const int a = z ? 2 : 0;
-  const uint32_t room = z ? b->defer_cap_axis[2] : b->defer_cap_axis[0] + b->defer_cap_axis[1];
-  dl.count = b->defer_count + a;
-  dl.items = b->defer_items + b->defer_off_axis[a];
-  const int64_t cap = defer_cap_setting();
-  dl.cap = cap >= 0 ? (uint32_t)std::min<int64_t>(cap, room) : room;
-  return dl;
+  if (z) return defer_list_of(b, 1, b->defer_items + b->defer_off_axis[2], b->defer_cap_axis[2]);
+  return defer_list_of(b, 0, b->defer_items, (int64_t)b->defer_cap_axis[0] + b->defer_cap_axis[1]);
 }
 
 // The fixup of an accumulating walk.
@@ -650,13 +650,13 @@ int alloc_box_memory(rhy_box* b) {
     total += cap;
   }
   b->defer_cap = (uint32_t)std::min<int64_t>(total, 0xffffffffll);
-  if (dev_alloc(&b->defer_count, sizeof(uint32_t) * 4) != hipSuccess ||
+  if (dev_alloc(&b->defer_count, 2 * kDeferBytes) != hipSuccess ||
       dev_alloc(&b->defer_items, sizeof(uint64_t) * (size_t)total) != hipSuccess) {
     free_box_memory(b);
     return fail(RHY_ERR_OOM, "deferred-face list allocation failed");
   }
   // ghosts start at 0 (rhyme_samr_bc_init.f90:61-87)
-  if (hipMemsetAsync(b->defer_count, 0, sizeof(uint32_t) * 4, b->stream) != hipSuccess ||
+  if (hipMemsetAsync(b->defer_count, 0, 2 * kDeferBytes, b->stream) != hipSuccess ||
       hipMemsetAsync(b->block, 0, b->esz * (size_t)P * planes, b->stream) != hipSuccess) {
     free_box_memory(b);
     return fail(RHY_ERR_HIP, "clearing the new box storage failed");
@@ -892,10 +892,11 @@ int rhy_box_last_deferred(rhy_box_t* b, int64_t* n) {
   int rc;
   if ((rc = check_box(b))) return rc;
   if (!n) return fail(RHY_ERR_ARG, "n is NULL");
-  uint32_t c[4] = {0, 0, 0, 0};
+  uint32_t c[2 * kDeferParts * kDeferGap];
   HIP_TRY(hipStreamSynchronize(b->stream));
   HIP_TRY(hipMemcpy(c, b->defer_count, sizeof(c), hipMemcpyDeviceToHost));
-  *n = (int64_t)c[0] + c[1] + c[2] + c[3];
+  *n = 0;
+  for (int i = 0; i < 2 * kDeferParts; ++i) *n += c[i * kDeferGap];
   return RHY_OK;
 }
 
@@ -1183,7 +1184,11 @@ int mh_solve_enqueue(rhy_box* b, const rhy_params_t* p, const double* dx, double
   if (p->solver_type != RHY_CPU_INTENSIVE && p->solver_type != RHY_MEMORY_INTENSIVE)
     return fail(RHY_ERR_SOLVER, "Unknown solver type");
   const Consts k = consts_of(p);
-  hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(64), 0, b->stream, b->dt, dt, b->defer_count);
+  // both lists, of which the planes take the first; a view of a caller's state has
+  // the first only
+  const uint32_t lists = b->defer_parts == kDeferParts ? 2 : 1;
+  hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(64), 0, b->stream, b->dt, dt, b->defer_count,
+                     lists * b->defer_parts);
   const BcTypes bc = make_bc(p);
   if (b->ndim == 1) {
     if ((rc = launch_flux<1>(b, k, dx))) return rc;
@@ -1306,6 +1311,7 @@ int rhy_mh_solve_noalloc(const rhy_params_t* p, int32_t ndim, const int32_t dims
   b.defer_items = reinterpret_cast<uint64_t*>(base + flux_bytes);
   const size_t list_bytes = align256(sizeof(uint64_t) * (size_t)b.defer_cap);
   b.defer_count = reinterpret_cast<uint32_t*>(base + flux_bytes + list_bytes);
+  b.defer_parts = 256 / (sizeof(uint32_t) * kDeferGap);  // of the one list it takes
   b.dt = reinterpret_cast<double*>(base + flux_bytes + list_bytes + 256);
   choose_walks(&b);
   b.profiling = false;

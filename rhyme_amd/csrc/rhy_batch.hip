@@ -126,11 +126,6 @@ __global__ __launch_bounds__(256) RHY_FLUX_OCCUPANCY void batch_flux_kernel(Cons
   }
 }
 
-// Parts of a batch's list of deferred faces: on one counter their additions take
-// 3.6 ns each, 0.4 ms of a step of 4 half empty boxes of 96^3.
-constexpr int kDeferParts = 32;
-constexpr size_t kDeferBytes = sizeof(uint32_t) * kDeferParts * kDeferGap;
-
 // The faces the flux phase listed, recomputed with the full policy PW
 // (each with its box's limiter, dt and dx); if the list overflowed, every
 // face of every active box.
@@ -140,19 +135,13 @@ __global__ __launch_bounds__(256) void batch_fixup_kernel(Consts k, const BBox* 
                                                           int32_t nactive, R* __restrict__ arena,
                                                           const double* __restrict__ dt,
                                                           DeferList dl) {
-  const int lane = (int)(threadIdx.x & 63);
-  const uint32_t n = lane < kDeferParts ? dl.count[lane * kDeferGap] : 0u;
-  if (wave_all(n == 0u)) return;
+  const DeferShare ds = defer_share(dl);
+  if (ds.none) return;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (wave_all(n <= dl.cap)) {
-    // a part's items by every kDeferParts-th workgroup
-    const int part = (int)(blockIdx.x % kDeferParts);
-    const uint32_t np = __builtin_amdgcn_readlane(n, part);
-    const uint64_t* items = dl.items + (size_t)part * dl.cap;
-    for (uint32_t i = blockIdx.x / kDeferParts * blockDim.x + threadIdx.x; i < np;
-         i += gridDim.x / kDeferParts * blockDim.x) {
-      const uint64_t it = items[i];
+  if (!ds.all) {
+    for (uint32_t i = ds.first; i < ds.n; i += ds.step) {
+      const uint64_t it = ds.items[i];
       const int32_t bx = (int32_t)(it >> 42);
       const BBox& B = boxes[bx];
       flux_face_fix<ND, R, PW>(&kernel_consts(), B.limiter, B.G, arena + B.cell_off, arena + B.flux_off, dt[bx], B.dx,

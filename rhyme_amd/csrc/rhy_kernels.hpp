@@ -160,17 +160,42 @@ int box_view(rhy_box_t* b, BoxView* v);
 
 // Faces whose Riemann solve needs a slow path (Deferring<P>), listed by the
 // flux kernels for the fixup kernel: item = box << 42 | axis << 40 | the
-// offset of the face's low cell in its box's planes.  count may pass cap;
-// the fixup then recomputes every face.  A list can be in 2^n parts, which the
-// workgroups take in turn: part i's count in count[i * kDeferGap], its room of cap
-// items from items[i * cap] on.
+// offset of the face's low cell in its box's planes.  A list is in last_part + 1
+// parts (2^n, 32 at most), which the workgroups take in turn, since the additions
+// to one counter take 3.6 ns each (4 half empty boxes of 96^3: 0.4 of 1.05 ms a
+// step): part i's count in count[i * kDeferGap], its room of cap items from
+// items[i * cap] on.  A count may pass cap; the fixup then recomputes every face.
 constexpr int kDeferGap = 16;  // a cache line
+constexpr int kDeferParts = 32;
+constexpr size_t kDeferBytes = sizeof(uint32_t) * kDeferParts * kDeferGap;  // a list's counts
 struct DeferList {
   uint32_t* count;
   uint64_t* items;
   uint32_t cap;
   uint32_t last_part = 0;
 };
+
+// What a workgroup of a fixup kernel takes of a list: nothing at all (none), or
+// everything, shared with the others (all: some part overflowed), or items
+// i = first, first + step, .. < n of its part.
+struct DeferShare {
+  bool none, all;
+  uint32_t n, first, step;
+  const uint64_t* items;
+};
+__device__ __forceinline__ DeferShare defer_share(const DeferList& dl) {
+  const uint32_t lane = threadIdx.x & 63, parts = dl.last_part + 1;
+  const uint32_t n = lane < parts ? dl.count[lane * kDeferGap] : 0u;
+  const uint32_t part = blockIdx.x & dl.last_part;
+  DeferShare s;
+  s.none = wave_all(n == 0u);
+  s.all = !wave_all(n <= dl.cap);
+  s.n = __builtin_amdgcn_readlane(n, part);
+  s.first = blockIdx.x / parts * blockDim.x + threadIdx.x;
+  s.step = gridDim.x / parts * blockDim.x;
+  s.items = dl.items + (size_t)part * dl.cap;
+  return s;
+}
 
 __device__ __forceinline__ uint64_t defer_item(uint32_t box, int axis, int64_t of) {
   return ((uint64_t)box << 42) | ((uint64_t)axis << 40) | (uint64_t)of;
@@ -1075,15 +1100,15 @@ __global__ __launch_bounds__(256) void flux_fixup_kernel(Consts k, Geom G,
                                                          const double* __restrict__ dtp,
                                                          double dx0, double dx1, double dx2,
                                                          DeferList dl) {
-  const uint32_t n = *dl.count;
-  if (n == 0) return;
+  const DeferShare ds = defer_share(dl);
+  if (ds.none) return;
   const double dt = *dtp;
   const double dx[3] = {dx0, dx1, dx2};
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n <= dl.cap) {
-    for (int64_t i = t0; i < (int64_t)n; i += stride) {
-      const uint64_t it = dl.items[i];
+  if (!ds.all) {
+    for (uint32_t i = ds.first; i < ds.n; i += ds.step) {
+      const uint64_t it = ds.items[i];
       flux_face_fix<ND, R, PW>(&kernel_consts(), kernel_consts().limiter, G, cells, F, dt, dx, (int)((it >> 40) & 3),
                                (int64_t)(it & ((1ull << 40) - 1)));
     }
@@ -1162,18 +1187,18 @@ __global__ __launch_bounds__(256) void acc_fixup_kernel(
     Consts k, Geom G, const R* __restrict__ cells, const R* __restrict__ acc, R* __restrict__ out,
     const double* __restrict__ dtp, double dx0, double dx1, double dx2, int order, DeferList dl,
     double* slot) {
-  const uint32_t n = *dl.count;
-  if (n == 0) return;
+  const DeferShare ds = defer_share(dl);
+  if (ds.none) return;
   const double dt = *dtp;
-  const int64_t total = (int64_t)G.n[0] * G.n[1] * G.n[2];
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const bool listed = n <= dl.cap;
+  const bool listed = !ds.all;
   // the list's faces name two cells each; past its capacity, every cell
-  const int64_t work = listed ? 2 * (int64_t)n : total;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < work; i += stride) {
+  const int64_t work = listed ? 2 * (int64_t)ds.n : (int64_t)G.n[0] * G.n[1] * G.n[2];
+  const int64_t stride = listed ? ds.step : (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = listed ? ds.first : (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < work;
+       i += stride) {
     int64_t oc;
     if (listed) {
-      const uint64_t it = dl.items[i >> 1];
+      const uint64_t it = ds.items[i >> 1];
       oc = (int64_t)(it & ((1ull << 40) - 1)) + ((i & 1) ? G.s[(it >> 40) & 3] : 0);
     } else {
       const int64_t r = i / G.n[0];
@@ -1301,7 +1326,7 @@ __global__ __launch_bounds__(kTubeLanes) RHY_FLUX_OCCUPANCY void tube_run_kernel
   for (int i = tid; i < P1; i += T)
 #pragma unroll
     for (int c = 0; c < NV; ++c) cells[c * G.plane + i] = u[c * P1 + i];
-  if (tid < 4) defer_count[tid] = tid == 0 ? deferred : 0u;
+  for (int i = tid; i < 2 * kDeferParts; i += T) defer_count[i * kDeferGap] = i ? 0u : deferred;
 }
 
 // Threads of tube_run for n cells, in the fewest rounds of at most kTubeLanes
@@ -1558,7 +1583,7 @@ __device__ __forceinline__ double strided_max(const double* __restrict__ p, int6
 // courant*minval(dx) is formed on the host.  Writes dt (and logs it) and the
 // raw max_u bits to maxu_out when given.
 // reset (with stepc): after the reduction has read every partial, also the
-// step's deferred-face counters (4) and, if given, the fixup's partial slot.
+// step's two lists of deferred faces and, if given, the fixup's partial slot.
 [[maybe_unused]] static __global__ __launch_bounds__(1024) void dt_kernel(
     const double* __restrict__ partial, int32_t n, double cmdx, double* dt_out, double* dt_log,
     double* maxu_out, double dx0 = 1.0, double dx1 = 1.0, double dx2 = 1.0,
@@ -1590,17 +1615,16 @@ __device__ __forceinline__ double strided_max(const double* __restrict__ p, int6
         }
       }
     }
-    if (reset_counts)
-      for (int i = 0; i < 4; ++i) reset_counts[i] = 0u;
     if (reset_slot) *reset_slot = 0.0;
   }
+  if (reset_counts && threadIdx.x < 2 * kDeferParts) reset_counts[threadIdx.x * kDeferGap] = 0u;
 }
 
-// A given dt, and empty deferred-face counters (4), before a solve.
-[[maybe_unused]] static __global__ void set_dt_kernel(double* dt_out, double dt,
-                                                      uint32_t* counts) {
+// A given dt, and an empty list of deferred faces (in n parts), before a solve.
+[[maybe_unused]] static __global__ void set_dt_kernel(double* dt_out, double dt, uint32_t* counts,
+                                                      uint32_t n) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *dt_out = dt;
-  if (threadIdx.x < 4 && blockIdx.x == 0) counts[threadIdx.x] = 0u;
+  if (threadIdx.x < n && blockIdx.x == 0) counts[threadIdx.x * kDeferGap] = 0u;
 }
 
 // A given dt and the step constants the walks read, as dt_kernel forms them.
@@ -1608,8 +1632,9 @@ __device__ __forceinline__ double strided_max(const double* __restrict__ p, int6
                                                         double dx0, double dx1, double dx2,
                                                         uint32_t* reset_counts,
                                                         double* reset_slot) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  for (int i = 0; i < 4; ++i) reset_counts[i] = 0u;  // as dt_kernel
+  if (blockIdx.x != 0) return;
+  if (threadIdx.x < 2 * kDeferParts) reset_counts[threadIdx.x * kDeferGap] = 0u;  // as dt_kernel
+  if (threadIdx.x != 0) return;
   *reset_slot = 0.0;
   const double dx[3] = {dx0, dx1, dx2};
   *dt_out = dt;
