@@ -211,15 +211,18 @@ int rhy_box_kernel_stats(rhy_box_t *box, int32_t kidx, int64_t *launches,
  * No counterpart in the reference (its Riemann solve runs the slow paths
  * inline: libm pow in rhyme_irs_nonlinear_wave_function.f90:20-22 and the
  * restarts from guesses 2-6 in rhyme_irs_exec.f90:24-42).  The flux kernels
- * leave faces that need those paths to a fixup kernel, which recomputes them
- * with the full solver in the same step; results are those of the full
- * solver bit for bit.
+ * leave faces that need those paths, gas without a pressure, a vacuum formed
+ * between two sides or (FP64 batches and pools) a vacuum on one side to a fixup
+ * kernel, which recomputes them with the full solver in the same step; results
+ * are those of the full solver bit for bit.  Where more than a few cells in a
+ * hundred lack a pressure, the fixup is most of the step's time.
  * rhy_box_last_deferred (rhy_batch_last_deferred for batches and pools):
- * faces listed by the last flux phase (waits for the stream).  rhy_debug_defer is a process-wide test hook
- * for callers that check the fixup path: every > 0 also lists every face
- * whose low-cell offset is a multiple of `every`, cap >= 0 caps the list (the
- * fixup then recomputes every face of the step); rhy_debug_defer(0, -1)
- * restores normal operation.  Not thread-safe with concurrent runs. */
+ * faces listed by the last flux phase (waits for the stream).
+ * rhy_debug_defer is a process-wide test hook for callers that check the fixup
+ * path: every > 0 also lists every face whose low-cell offset is a multiple of
+ * `every`, cap >= 0 caps the list (the fixup then recomputes every face of the
+ * step); rhy_debug_defer(0, -1) restores normal operation.  Not thread-safe
+ * with concurrent runs. */
 int rhy_box_last_deferred(rhy_box_t *box, int64_t *n);
 int rhy_debug_defer(int32_t every, int64_t cap);
 
@@ -482,9 +485,9 @@ int rhy_batch_last_deferred(rhy_batch_t *batch, int64_t *n);
  *   rhy_mh_solve, bit for bit) through the accumulating walks of rhy_run
  *   instead of the flux planes: the box keeps the state it stepped from in
  *   its second state buffer, from which rhy_amr_reflux forms the coarse
- *   fluxes it needs (as the walks formed them, bit for bit).  Any later call that changes the box
- *   (upload, step, paint, draw, resize, unpack) ends that; the box's ghost
- *   faces are not filled after the step.  1D boxes take rhy_mh_solve.
+ *   fluxes it needs (as the walks formed them, bit for bit).  Any later call
+ *   that changes the box (upload, step, paint, draw, resize, unpack) ends that;
+ *   the box's ghost faces are not filled after the step.  1D boxes take rhy_mh_solve.
  * The prolong, restrict, register and reflux calls wait for both sides'
  * streams; rhy_amr_coarse_step returns when its step is done. */
 int rhy_batch_cfl_dts(rhy_batch_t *batch, const rhy_params_t *p, double *dts);
